@@ -433,15 +433,15 @@ ela::StepArgs<T> base_args(ela_handle* h, T* o[9], T* c[9]) {
   return a;
 }
 
-// which: bit 0 = velocity kernel, bit 1 = stress kernel; FV / FS: the
-// ela::F_* work fused into the velocity / stress launch.
+// which: bit 0 = velocity blocks, bit 1 = stress blocks; FV / FS: the
+// ela::F_* work fused into them.
 template <typename T, int BX, int MODE, int FV, int FS>
 int launch_step_bx(ela_handle* h, ela::StepArgs<T> a, int which) {
   Tiles t = tiles_for(h, BX, a.ychunk);
   a.nbz = t.nbz; a.nbx = t.nbx; a.nby = t.nby;
   dim3 block(ela::TZ, BX);
-  if (which & 1) launch(h, ela::k_velocity<T, BX, MODE, FV>, dim3(t.nblocks), block, a);
-  if (which & 2) launch(h, ela::k_stress<T, BX, MODE, FS>, dim3(t.nblocks), block, a);
+  a.first = which & 1 ? 0 : t.nblocks;
+  launch(h, ela::k_step<T, BX, MODE, FV, FS>, dim3(which == 3 ? 2 * t.nblocks : t.nblocks), block, a);
   return ELA_OK;
 }
 

@@ -5,8 +5,8 @@
 //   staggered derivatives, cosine sponge. The reference runs, per fine step,
 //   one stepper launch (kernelsElaGpu_3D.cu:110-460), 7 injection launches, a
 //   damping launch over both time levels (:1182-1226) and 7 recording launches.
-//   Here one fine step is two stencil launches (velocity update, stress update;
-//   they read only level n so they are independent) plus one injection and one
+//   Here one fine step is one stencil launch (velocity and stress blocks, which
+//   read only level n and so are independent) plus one injection and one
 //   recording launch, with the sponge folded into the stencil:
 //       n = w * (w * o + M D(c) [+ secondary source])
 //   where every stored level has been damped exactly once. This equals the
@@ -90,6 +90,7 @@ struct StepArgs {
   int64_t ys;           // nx * nzi
   int ychunk;
   int nbz, nbx, nby;    // tile counts along z, x, y-chunks
+  int first;            // first tile of the launch: 0, or the tile count (stress blocks alone)
   int remap;            // tile order (see tile_coord)
   int xgroup;           // x columns per group of the y-major order
   const int* chunks;    // stacked windows: per y chunk {y0, y1, window y0, window ny, window nx}, or null
@@ -343,11 +344,10 @@ struct TileCoord {
 // xgroup > 1, x) neighbours share an L2 while the grid is swept in the
 // hardware order.
 template <int BX>
-__device__ __forceinline__ TileCoord tile_coord(int nbz, int nbx, int nby, int ychunk, int nz, int nzi, int zoff,
-                                                int nx, int ny, int order, int xgroup, const int* chunks) {
+__device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int nby, int ychunk, int nz, int nzi,
+                                                int zoff, int nx, int ny, int order, int xgroup, const int* chunks) {
   const int nb = nbz * nbx * nby;
-  const int lb = order == 3 ? xcd_group(blockIdx.x, nb, nbz * xgroup)
-                 : order ? xcd_remap(blockIdx.x, nb) : (int)blockIdx.x;
+  const int lb = order == 3 ? xcd_group(bid, nb, nbz * xgroup) : order ? xcd_remap(bid, nb) : bid;
   int bz, bx, by;
   if (order == 2) {
     const int per_z = nbx * nby;
@@ -476,7 +476,7 @@ __device__ __forceinline__ void normal_moduli(T tdt, double tdt64, T lam, T mu, 
 }
 
 template <typename T, int BX, int MODE, int F>
-__global__ void __launch_bounds__(TZ * BX) k_velocity(StepArgs<T> a) {
+__device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, VelLds<T, BX, (F & F_MED3) != 0>& L) {
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
@@ -484,12 +484,9 @@ __global__ void __launch_bounds__(TZ * BX) k_velocity(StepArgs<T> a) {
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
   static_assert(!MED3 || MODE == MODE_FWD || MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_PM,
                 "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
-  // one LDS object: the compiler's wait analysis then tells the rows the
-  // direct loads fill (buffer b ^ 1) from the rows the stencil reads (buffer b)
-  __shared__ VelLds<T, BX, MED3> L;
   auto& l_xx = L.xx; auto& l_zz = L.zz; auto& l_xy = L.xy; auto& l_xz = L.xz; auto& l_yz = L.yz;
   auto& l_rho = L.rho;
-  const TileCoord t = tile_coord<BX>(a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   const StressVal<T, MODE> S{a}, SXl{a}, SXh{a}, SZ{a};
@@ -681,7 +678,7 @@ struct StressStage {
 };
 
 template <typename T, int BX, int MODE, int F>
-__global__ void __launch_bounds__(TZ * BX) k_stress(StepArgs<T> a) {
+__device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, StressLds<T, BX, (F & F_MED3) != 0>& L) {
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
@@ -689,13 +686,12 @@ __global__ void __launch_bounds__(TZ * BX) k_stress(StepArgs<T> a) {
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
   static_assert(!MED3 || MODE == MODE_FWD || MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_PM,
                 "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
-  __shared__ StressLds<T, BX, MED3> L;  // one LDS object (see k_velocity)
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz; auto& l_mu = L.mu;
-  const TileCoord t = tile_coord<BX>(a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   const VelVal<T, MODE> V{a}, Vlo{a}, Vhi{a}, Vzh{a};
-  // FP32 rows that are plain array values go straight from HBM to LDS (see k_velocity)
+  // FP32 rows that are plain array values go straight from HBM to LDS (see velocity_block)
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
   auto src = [&](int f) -> const T* { return MODE == MODE_BORN_ADJ_PM ? a.q[f] : a.c[f]; };
   const int r = t.ty + FAT, q = t.tz + FAT;
@@ -791,10 +787,10 @@ __global__ void __launch_bounds__(TZ * BX) k_stress(StepArgs<T> a) {
       fetch(nx_, iy + 1, b ^ 1);
       if (MED3) fetch_mu(nx_, iy + 1, b ^ 1);
     }
-    if (QS ? t.xin : t.active) {  // F_Q16 stores: see k_velocity
+    if (QS ? t.xin : t.active) {  // F_Q16 stores: see velocity_block
       const uint32_t i = (uint32_t)iy * ys + (QS ? t.colu : t.col);
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
-      // FP32: every per-cell operand is loaded before the first store (see k_velocity)
+      // FP32: every per-cell operand is loaded before the first store (see velocity_block)
       T o6[6], ss6[6], al6[6], ar6[6], g5[5], d6[6];
       auto load_ss = [&](int f) { return *at(a.ssl[f], i) * a.ssfl + *at(a.ssr[f], i) * a.ssfr; };
       auto load_grad = [&]() {
@@ -922,6 +918,37 @@ __global__ void __launch_bounds__(TZ * BX) k_stress(StepArgs<T> a) {
     __syncthreads();
     b ^= 1;
   }
+}
+
+// ---------------------------------------------------------------------------
+// One fine step: the velocity blocks, then the stress blocks, in one launch
+// (both read level n only). Small grids are bound by the latency of a march
+// (about 1.2 us a plane) and by the launch itself, which the two halves now
+// share: 40x36x44 tile 8x4 20.5 -> 13.8 us a step with inject and record,
+// 110x93x121 49.8 -> 43.4 us, 152x152x148 105.8 -> 96.9 us (FP32, tile 8x8,
+// order 3/2). Large grids gain only the first half's tail (232x328x324 638.7
+// -> 637.2 us, 328x472x468 1721.8 -> 1718.6 us): they are bound by HBM.
+// ---------------------------------------------------------------------------
+// Waves per SIMD asked of the compiler: the FP32 steps without per-cell extra
+// operands need 115-129 VGPRs and run at 4 (at most 128); the others hold more
+// and take what they get (1: no request).
+template <typename T, int FV, int FS>
+constexpr int step_waves() {
+  return sizeof(T) == 4 && ((FV | FS) & (F_SS | F_ACC | F_GRAD)) == 0 ? 4 : 1;
+}
+
+template <typename T, int BX, int MODE, int FV, int FS>
+__global__ void __launch_bounds__(TZ * BX, (step_waves<T, FV, FS>())) k_step(StepArgs<T> a) {
+  // one LDS object: the compiler's wait analysis then tells the rows the
+  // direct loads fill (buffer b ^ 1) from the rows the stencil reads (buffer b)
+  union Lds {
+    VelLds<T, BX, (FV & F_MED3) != 0> v;
+    StressLds<T, BX, (FS & F_MED3) != 0> s;
+  };
+  __shared__ Lds L;
+  const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
+  if (bid < nb) velocity_block<T, BX, MODE, FV>(a, bid, L.v);
+  else stress_block<T, BX, MODE, FS>(a, bid - nb, L.s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1127,7 +1154,7 @@ struct ImagingArgs {
 };
 
 // The imaging kernels' LDS: double-buffered planes of the coarse vx, vy, vz
-// slice V[its] (one LDS object, see k_velocity).
+// slice V[its] (one LDS object, see k_step).
 template <typename T, int BX>
 struct ImagingLds {
   Plane<T, BX> vx[2], vy[2], vz[2];
@@ -1148,7 +1175,7 @@ template <typename T, int BX, bool ADJ>
 __global__ void __launch_bounds__(TZ * BX) k_imaging(ImagingArgs<T> a) {
   __shared__ ImagingLds<T, BX> L;
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz;
-  const TileCoord t = tile_coord<BX>(a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<BX>(blockIdx.x, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4;
