@@ -195,11 +195,11 @@ struct ela_handle {
   bool have_medium = false;
   std::vector<double> filt; // 2*(sub+1)
   int64_t last_steps = 0;
-  int by_x = 16;            // x extent of a tile
+  int by_x = 4;             // x extent of a tile (initial launch shape: initial_shape)
   int by_x_t = 0;           // x extent of the premultiplied transposed steps' tiles (0: by_x)
   int ychunk = 8;           // y planes per block
-  int remap = 0;            // tile order (ela_set_tile_order)
-  int xgroup = 1;           // x columns per group of the y-major order
+  int remap = 3;            // tile order (ela_set_tile_order)
+  int xgroup = 4;           // x columns per group of orders 2 and 3
   int64_t born_segment = 0; // Born adjoint storage: 0 auto, -1 all samples, K > 0 checkpoints every K
   int64_t born_budget = 0;  // device-memory budget of the automatic plan [bytes], 0: free memory
   int64_t born_last_segment = 0;  // plan of the last Born adjoint (-1 full storage)
@@ -404,6 +404,32 @@ Tiles tiles_for(const ela_handle* h, int bx, int ychunk) {
   t.nby = h->win_y0.empty() ? (int)((iy + ychunk - 1) / ychunk) : h->nchunks;
   t.nblocks = t.nbz * t.nbx * t.nby;
   return t;
+}
+
+// Launch shape of a new handle (until ela_set_tiling / ela_set_tile_order).
+// 256-thread blocks of 4 x rows, whole z columns in groups of 4 x columns per
+// XCD: the fastest or within 1 % of it on every grid and step kind measured
+// but the recomputation with derivative store (2 % behind 8 rows) and the
+// FP64 forward of large grids (3 % behind 8x16); against the former 16x8 in
+// hardware order, us per FP32 step with (rho, lambda, mu): 152x152x148 100.8
+// -> 96, 201x187x143 173 -> 155, 232x328x324 661 -> 631, 328x472x468 1736 ->
+// 1712; its transposed step with imaging 1572 -> 1186 (232x328x324), where 16
+// rows spill. Planes per block: 8, the prologue's 7 planes of queue values
+// being paid once per block, unless the blocks of the two halves then leave
+// CUs idle; a shorter march has less latency to pay as long as the blocks are
+// resident together (256 CUs x 4 waves per SIMD of FP32 blocks, 2 of FP64
+// ones): 72x72x72 18.6 us a step with 8 planes, 15.5 with 2; 40x36x44 15.8
+// -> 10.8. 7/8 of the residency counts as full: 88x97x90 (1012 blocks of 1024)
+// 28.8 us with 8 planes, 29.4 with 4; a march of 1 gains nothing over 2.
+void initial_shape(ela_handle* h) {
+  const int64_t iz = h->cfg.nz - 2 * ela::FAT, ix = h->cfg.nx - 2 * ela::FAT, iy = h->cfg.ny - 2 * ela::FAT;
+  const int64_t cols = ((iz + ela::TZ - 1) / ela::TZ) * ((ix + h->by_x - 1) / h->by_x);
+  const int64_t resident = 256 * (h->esize == 4 ? 4 : 2);
+  const int planes[] = {8, 6, 4, 3, 2};
+  for (int yc : planes) {
+    h->ychunk = yc;
+    if (2 * cols * ((iy + yc - 1) / yc) >= resident * 7 / 8) break;
+  }
 }
 
 template <typename T>
@@ -2049,7 +2075,7 @@ int ela_create(const ela_config* cfg, ela_handle** out) {
     }
     rc = h->counter.alloc(256);
     if (rc) return bail(rc);
-    h->by_x = cfg->precision == ELA_FP64 ? 8 : 16;
+    initial_shape(h);
     // the device address of the allocation-free entry point's scratch on this device
     rc = scratch_address(cfg->device, &h->scratch_dev);
     if (rc) return bail(rc);

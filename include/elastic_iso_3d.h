@@ -379,17 +379,19 @@ int ela_set_windows(ela_handle* h, int n, const int64_t* y0, const int64_t* ny, 
 int ela_set_graph(ela_handle* h, int on);
 
 /* Tile shape of the stencil kernels: x extent of a 64-wide z tile (4, 8 or
- * 16 rows) and the number of y planes one block marches through. Any
- * setting gives the same result; it only changes speed. */
+ * 16 rows) and the number of y planes one block marches through (a new
+ * handle: 4 rows and 2 to 8 planes, by the grid's size). Any setting gives
+ * the same result; it only changes speed. */
 int ela_set_tiling(ela_handle* h, int tile_x, int y_chunk);
 int ela_get_tiling(const ela_handle* h, int* tile_x, int* y_chunk);
-/* Block-to-tile order of the stencil launches (speed only): 0 (default)
- * the hardware's round-robin dealing of blocks to the 8 XCDs over tiles
- * enumerated z, x, y; 1 each XCD a contiguous range of that enumeration; 2
- * each XCD a contiguous range of a y-major enumeration in groups of x_group
- * x columns, so that concurrently running neighbours share halo planes in
- * the XCD's L2; 3 the order-0 sweep with whole z columns (x_group adjacent
- * columns) dealt to one XCD, so that z and x neighbours share its L2. */
+/* Block-to-tile order of the stencil launches (speed only): 0 the hardware's
+ * round-robin dealing of blocks to the 8 XCDs over tiles enumerated z, x, y;
+ * 1 each XCD a contiguous range of that enumeration; 2 each XCD a contiguous
+ * range of a y-major enumeration in groups of x_group x columns, so that
+ * concurrently running neighbours share halo planes in the XCD's L2; 3 (the
+ * default, with groups of 4) the order-0 sweep with whole z columns (x_group
+ * adjacent columns) dealt to one XCD, so that z and x neighbours share its
+ * L2. */
 int ela_set_tile_order(ela_handle* h, int order, int x_group);
 
 /* Diagnostic timing: launch the velocity and the stress stencil kernels of a
