@@ -436,10 +436,12 @@ template <typename T>
 ela::StepArgs<T> base_args(ela_handle* h, T* o[9], T* c[9]) {
   ela::StepArgs<T> a;
   std::memset(&a, 0, sizeof(a));
-  for (int k = 0; k < 9; ++k) { a.o[k] = o[k]; a.c[k] = c[k]; }
-  for (int k = 0; k < 8; ++k) a.m[k] = arr<T>(h->med, h->stride, k);
+  a.o = o[0];
+  a.c = c[0];
+  a.m = arr<T>(h->med, h->stride, 0);
+  a.np = h->stride;
   if (h->have_elastic) {
-    for (int k = 0; k < 3; ++k) a.ep[k] = arr<T>(h->elastic, h->stride, k);
+    a.ep = arr<T>(h->elastic, h->stride, 0);
     a.tdt = (T)h->tdt;
     a.tdt64 = h->tdt;
   }
@@ -462,24 +464,33 @@ ela::StepArgs<T> base_args(ela_handle* h, T* o[9], T* c[9]) {
 // which: bit 0 = velocity blocks, bit 1 = stress blocks; FV / FS: the
 // ela::F_* work fused into them.
 template <typename T, int BX, int MODE, int FV, int FS>
-int launch_step_bx(ela_handle* h, ela::StepArgs<T> a, int which) {
+int launch_step_bx(ela_handle* h, ela::StepArgs<T> a, int which, const ela::PointArgs<T>& inj,
+                   const ela::PointArgs<T>& rec) {
   Tiles t = tiles_for(h, BX, a.ychunk);
   a.nbz = t.nbz; a.nbx = t.nbx; a.nby = t.nby;
   dim3 block(ela::TZ, BX);
   a.first = which & 1 ? 0 : t.nblocks;
-  launch(h, ela::k_step<T, BX, MODE, FV, FS>, dim3(which == 3 ? 2 * t.nblocks : t.nblocks), block, a);
+  // recording blocks follow the stress blocks (a recorded step runs both halves)
+  const unsigned nrec = (unsigned)((rec.off[9] + ela::TZ * BX - 1) / (ela::TZ * BX));
+  const unsigned nb = (unsigned)(which == 3 ? 2 * t.nblocks : t.nblocks);
+  launch(h, ela::k_step<T, BX, MODE, FV, FS>, dim3(nb + nrec), block, a, inj, rec);
   return ELA_OK;
 }
 
 template <typename T, int MODE, int FV, int FS>
-int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which = 3) {
+int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::PointArgs<T>& inj,
+                const ela::PointArgs<T>& rec) {
   // the premultiplied transposed steps (Born adjoint, gradient) may take a tile of their own
   const int bx = MODE == ela::MODE_BORN_ADJ_PM && h->by_x_t ? h->by_x_t : h->by_x;
-  switch (bx) {
-    case 4: return launch_step_bx<T, 4, MODE, FV, FS>(h, a, which);
-    case 8: return launch_step_bx<T, 8, MODE, FV, FS>(h, a, which);
-    default: return launch_step_bx<T, 16, MODE, FV, FS>(h, a, which);
+  // 16 rows (1024 threads, at most 128 registers) only where the step fits:
+  // FP64 and the steps with per-cell extra operands spill there (Born adjoint
+  // of 232x328x324 69-97 ms with 16 rows, 60 with 4) and run 4 rows instead
+  constexpr bool wide = sizeof(T) == 4 && ((FV | FS) & (ela::F_SS | ela::F_ACC | ela::F_GRAD)) == 0;
+  if (bx == 8) return launch_step_bx<T, 8, MODE, FV, FS>(h, a, which, inj, rec);
+  if constexpr (wide) {
+    if (bx == 16) return launch_step_bx<T, 16, MODE, FV, FS>(h, a, which, inj, rec);
   }
+  return launch_step_bx<T, 4, MODE, FV, FS>(h, a, which, inj, rec);
 }
 
 // Forward, nonlinear-adjoint and premultiplied transposed steps form the
@@ -488,11 +499,12 @@ int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which = 3) {
 // the 8 scaled arrays, which k_scale_medium derives with the steppers'
 // operations, so both routes give bit-identical results.
 template <typename T, int MODE, int FV, int FS>
-int launch_step_m(ela_handle* h, const ela::StepArgs<T>& a, int which = 3) {
+int launch_step_m(ela_handle* h, const ela::StepArgs<T>& a, int which = 3,
+                  const ela::PointArgs<T>& inj = ela::PointArgs<T>{}, const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
   if constexpr (MODE == ela::MODE_FWD || MODE == ela::MODE_ADJ || MODE == ela::MODE_BORN_ADJ_PM) {
-    if (h->have_elastic) return launch_step<T, MODE, FV | ela::F_MED3, FS | ela::F_MED3>(h, a, which);
+    if (h->have_elastic) return launch_step<T, MODE, FV | ela::F_MED3, FS | ela::F_MED3>(h, a, which, inj, rec);
   }
-  return launch_step<T, MODE, FV, FS>(h, a, which);
+  return launch_step<T, MODE, FV, FS>(h, a, which, inj, rec);
 }
 
 template <typename T>
@@ -538,7 +550,30 @@ int copy_out_3d(ela_handle* h, void* dst, const void* src, int n_arrays, int mem
 struct DevPoints {
   const int32_t* pos[7];
   int64_t n[7];
+  const int* box = nullptr;  // device box of the points (ela::inject_tile), or null
+  bool fuse = false;         // an injection at these points is fused into the steps
 };
+
+// Longest list (over the 9 components) whose injection may be fused: two
+// points a thread of the smallest block.
+constexpr int64_t kFusePoints = 512;
+
+int64_t total_points(const DevPoints& p) {
+  int64_t n = 0;
+  for (int c = 0; c < 9; ++c) n += p.n[kCompGrid[c]];
+  return n;
+}
+
+// Whether an injection goes into the step's own blocks: the list is short and
+// the tiles that meet its box (box[6] as k_convert_pos leaves it) are at most
+// one resident round of blocks. A block that meets the box pays about 1 us
+// (barrier, positions) at its end; the separate launch costs 4.7 us a step.
+bool fuse_injection(const ela_handle* h, const DevPoints& p, const int* box) {
+  const int64_t n = total_points(p);
+  if (n == 0 || n > kFusePoints) return false;
+  const auto tiles = [](int lo_top, int hi, int64_t tile) { return (int64_t)(hi - (ela::POS_TOP - lo_top)) / tile + 2; };
+  return tiles(box[0], box[1], ela::TZ) * tiles(box[2], box[3], h->by_x) * tiles(box[4], box[5], h->ychunk) <= 1024;
+}
 
 // Copies (host) or reads (device) the caller's int64 positions, converts them
 // to internal int32 offsets on the GPU and checks that every point lies in the
@@ -565,14 +600,16 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   int64_t* s64 = (int64_t*)base;
   int32_t* s32 = (int32_t*)(base + b64);
   int* flag = (int*)(base + b64 + b32);
-  launch(h, ela::k_fill<int>, dim3(1), dim3(64), flag, (int64_t)1, 0);
+  launch(h, ela::k_fill<int>, dim3(1), dim3(64), flag, (int64_t)64, 0);  // flag[0]; boxes at 8 and 16
   int64_t off = 0;
   for (int side = 0; side < 2; ++side) {
     const ela_points* p = side ? rp : sp;
     DevPoints& d = side ? dr : ds;
+    for (int g = 0; g < 7; ++g) d.n[g] = p->n[g];
+    int* box = total_points(d) <= kFusePoints ? flag + 8 + 8 * side : nullptr;
+    d.box = box;
     for (int g = 0; g < 7; ++g) {
       const int64_t n = p->n[g];
-      d.n[g] = n;
       d.pos[g] = s32 + off;
       if (n) {
         const int64_t* src = p->pos[g];
@@ -582,15 +619,17 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
         }
         launch(h, ela::k_convert_pos, dim3((unsigned)((n + 255) / 256)), dim3(256), src,
                            s32 + off, n, (int)h->cfg.nz, (int)h->cfg.nx, (int)h->cfg.ny, (int)h->nzi, (int)h->zoff,
-                           h->win_y0.empty() ? nullptr : (const int*)h->ytab.p, flag);
+                           h->win_y0.empty() ? nullptr : (const int*)h->ytab.p, flag, box);
       }
       off += n;
     }
   }
-  int bad = 0;
-  HIPCHK(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  int host[24];
+  HIPCHK(hipMemcpyAsync(host, flag, sizeof(host), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  if (bad) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
+  ds.fuse = ds.box && fuse_injection(h, ds, host + 8);
+  dr.fuse = dr.box && fuse_injection(h, dr, host + 16);
+  if (host[0]) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
   return ELA_OK;
 }
 
@@ -617,6 +656,7 @@ ela::PointArgs<T> make_points(ela_handle* h, const DevPoints& pts, T* const fiel
   a.nz = (int)h->cfg.nz; a.nx = (int)h->cfg.nx; a.ny = (int)h->cfg.ny;
   a.nzi = (int)h->nzi; a.zoff = (int)h->zoff;
   a.ytab = h->win_y0.empty() ? nullptr : (const int*)h->ytab.p;
+  a.box = pts.box;
   return a;
 }
 
@@ -651,12 +691,20 @@ struct DevStep {
   int advance = 0;
 };
 
-template <typename T, bool ACC, bool GRAD = false, bool PM = false>
-void launch_inject(ela_handle* h, ela::PointArgs<T> a, int its, double fa, double fb) {
-  if (a.off[9] == 0) return;
-  set_time(a, its, fa, fb);
-  const unsigned nb = (unsigned)((a.off[9] + 255) / 256);
-  launch(h, ela::k_inject<T, ACC, GRAD, PM>, dim3(nb), dim3(256), a);
+// One fine step: the stencil, the injection (in the stencil's blocks where
+// the points allow it, else a launch behind it) and the recording `rec` of
+// the level the step reads (an empty list: none). Level n is recorded by the
+// step that computes n + 1, whose blocks leave it untouched: no launch of its
+// own, and its scattered reads overlap the stencil's.
+template <typename T, int MODE, int FV, int FS>
+int step_with_points(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& ip, const ela::PointArgs<T>& inj,
+                     const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
+  CHK((launch_step_m<T, MODE, FV, FS>(h, a, 3, ip.fuse ? inj : ela::PointArgs<T>{}, rec)));
+  if (ip.fuse || inj.off[9] == 0) return ELA_OK;
+  const unsigned nb = (unsigned)((inj.off[9] + 255) / 256);
+  launch(h, ela::k_inject<T, ((FV | FS) & ela::F_ACC) != 0, ((FV | FS) & ela::F_GRAD) != 0,
+                          MODE == ela::MODE_BORN_ADJ_PM>, dim3(nb), dim3(256), inj);
+  return ELA_OK;
 }
 
 template <typename T>
@@ -753,7 +801,8 @@ Wave<T> wave_ptrs(DevBuf& b, int64_t stride, bool premultiplied = false) {
 // Premultiplied Born-adjoint step arguments: read M c from q1, write M n to q0.
 template <typename T>
 void set_pm(ela_handle* h, ela::StepArgs<T>& a, const Wave<T>& w) {
-  for (int k = 0; k < 9; ++k) { a.q[k] = w.q1[k]; a.qn[k] = w.q0[k]; }
+  a.q = w.q1[0];
+  a.qn = w.q0[0];
   (void)h;
 }
 
@@ -781,12 +830,6 @@ int64_t interior_cells(const ela_handle* h) {
   int64_t n = 0;
   for (size_t w = 0; w < h->win_y0.size(); ++w)
     n += (h->cfg.nz - 2 * ela::FAT) * (h->win_nx[w] - 2 * ela::FAT) * (h->win_ny[w] - 2 * ela::FAT);
-  return n;
-}
-
-int64_t total_points(const DevPoints& p) {
-  int64_t n = 0;
-  for (int c = 0; c < 9; ++c) n += p.n[kCompGrid[c]];
   return n;
 }
 
@@ -849,29 +892,27 @@ int nl_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, cons
   const double* f = h->filt.data();
   // One coarse step: sub fine steps (stepper, injection, recording). With
   // its_dev the coarse index is read from device memory (graph replays).
+  // The level a step reads is recorded by it: the one the fine step before it
+  // left (of the coarse step before for the first), none before the first.
   auto coarse_step = [&](int64_t its, const int* its_dev) -> int {
-    if (!adjoint) {
-      for (int64_t it2 = 1; it2 <= sub; ++it2) {
-        ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
-        CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a)));
-        ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
-        ela::PointArgs<T> R = make_points<T>(h, rp, w.p0, tmv, true, nrec_tot);
-        S.its_dev = R.its_dev = its_dev;
-        launch_inject<T, false>(h, S, (int)its, f[it2 - 1], f[hh + it2 - 1]);
-        launch_record<T>(h, R, (int)its, f[it2], f[hh + it2]);
-        w.swap();
-      }
-    } else {
-      for (int64_t it2 = sub - 1; it2 >= 0; --it2) {
-        ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
-        CHK((launch_step_m<T, ela::MODE_ADJ, 0, 0>(h, a)));
-        ela::PointArgs<T> R = make_points<T>(h, rp, w.p0, tmv, true, nrec_tot);
-        ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
-        S.its_dev = R.its_dev = its_dev;
-        launch_inject<T, false>(h, R, (int)its, f[it2 + 1], f[hh + it2 + 1]);
-        launch_record<T>(h, S, (int)its, f[it2], f[hh + it2]);
-        w.swap();
-      }
+    for (int64_t j = 0; j < sub; ++j) {
+      ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
+      const int dir = adjoint ? -1 : 1;
+      const int64_t its_r = j ? its : its - dir;   // coarse step the recorded level belongs to
+      ela::PointArgs<T> I = adjoint ? make_points<T>(h, rp, w.p0, tmv, true, nrec_tot)
+                                    : make_points<T>(h, sp, w.p0, src_tr, false, 0);
+      ela::PointArgs<T> R = adjoint ? make_points<T>(h, sp, w.p1, src_tr, false, 0)
+                                    : make_points<T>(h, rp, w.p1, tmv, true, nrec_tot);
+      I.its_dev = R.its_dev = its_dev;
+      R.its_off = (int)(its_r - its);
+      R.nmax = (int)(nts - 1);
+      const int64_t fi = adjoint ? sub - j : j, fr = adjoint ? (j ? sub - j : 0) : (j ? j : sub);
+      set_time(I, (int)its, f[fi], f[hh + fi]);
+      set_time(R, (int)its_r, f[fr], f[hh + fr]);
+      if (!its_dev && (its_r < 0 || its_r > nts - 2)) R.off[9] = 0;
+      if (adjoint) CHK((step_with_points<T, ela::MODE_ADJ, 0, 0>(h, a, rp, I, R)));
+      else CHK((step_with_points<T, ela::MODE_FWD, 0, 0>(h, a, sp, I, R)));
+      w.swap();
     }
     return ELA_OK;
   };
@@ -900,6 +941,9 @@ int nl_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, cons
   } else {
     for (int64_t its = nts - 2; its >= 0; --its) CHK(coarse_step(its, nullptr));
   }
+  // the last level
+  if (!adjoint) launch_record<T>(h, make_points<T>(h, rp, w.p1, tmv, true, nrec_tot), (int)(nts - 2), f[sub], f[hh + sub]);
+  else launch_record<T>(h, make_points<T>(h, sp, w.p1, src_tr, false, 0), 0, f[0], f[hh]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   HIPCHK(hipGetLastError());
   h->last_steps = (nts - 1) * sub;
@@ -948,13 +992,14 @@ int bg_coarse_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_
   const double* f = h->filt.data();
   for (int64_t it2 = 1; it2 <= sub; ++it2) {
     ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
-    for (int c = 0; c < 3; ++c) { a.accl[c] = VL + c * np; a.accr[c] = VR + c * np; }
+    a.accl = VL;
+    a.accr = VR;
     a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
-    CHK((launch_step_m<T, ela::MODE_FWD, ela::F_ACC, 0>(h, a)));
     ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
-    for (int c = 0; c < 3; ++c) { S.accl[c] = a.accl[c]; S.accr[c] = a.accr[c]; }
+    for (int c = 0; c < 3; ++c) { S.accl[c] = VL + c * np; S.accr[c] = VR + c * np; }
     S.accfl = a.accfl; S.accfr = a.accfr;
-    launch_inject<T, true>(h, S, (int)k, f[it2 - 1], f[hh + it2 - 1]);
+    set_time(S, (int)k, f[it2 - 1], f[hh + it2 - 1]);
+    CHK((step_with_points<T, ela::MODE_FWD, ela::F_ACC, 0>(h, a, sp, S)));
     w.swap();
   }
   return ELA_OK;
@@ -1090,11 +1135,15 @@ int born_forward_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
     launch_imaging<T, false>(h, imaging_args<T>(h, V(its), V(its + 1), V(its + 2), its + 1, dm, nullptr, ssR));
     for (int64_t it2 = 1; it2 <= sub; ++it2) {
       ela::StepArgs<T> a = base_args<T>(h, sc.p0, sc.p1);
-      for (int k = 0; k < 9; ++k) { a.ssl[k] = ssL[k]; a.ssr[k] = ssR[k]; }
+      a.ssl = ssL[0];
+      a.ssr = ssR[0];
       a.ssfl = T(f[it2 - 1]); a.ssfr = T(f[hh + it2 - 1]);
-      CHK((launch_step_m<T, ela::MODE_FWD, ela::F_SS, ela::F_SS>(h, a)));
-      launch_record<T>(h, make_points<T>(h, rp, sc.p0, TmViews<T>(tm).v, true, nrec_tot), (int)its, f[it2],
-                       f[hh + it2]);
+      // records the level before (of the coarse step before for the first, none before level 1)
+      ela::PointArgs<T> R = make_points<T>(h, rp, sc.p1, TmViews<T>(tm).v, true, nrec_tot);
+      const int64_t ir = it2 > 1 ? it2 - 1 : sub, its_r = it2 > 1 ? its : its - 1;
+      set_time(R, (int)its_r, f[ir], f[hh + ir]);
+      if (its_r < 0) R.off[9] = 0;
+      CHK((launch_step_m<T, ela::MODE_FWD, ela::F_SS, ela::F_SS>(h, a, 3, ela::PointArgs<T>{}, R)));
       sc.swap();
     }
     for (int k = 0; k < 9; ++k) std::swap(ssL[k], ssR[k]);
@@ -1108,6 +1157,8 @@ int born_forward_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
     // V[0..k] are final (all of V once k == nts-2)
     while (next <= nts - 2 && (next + 2 <= k || k == nts - 2)) CHK(scattered_step(next++));
   }
+  launch_record<T>(h, make_points<T>(h, rp, sc.p1, TmViews<T>(tm).v, true, nrec_tot), (int)(nts - 2), f[sub],
+                   f[hh + sub]);
   h->last_steps = 2 * (nts - 1) * sub;
   return ELA_OK;
 }
@@ -1193,14 +1244,15 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
     for (int64_t it2 = sub - 1; it2 >= 0; --it2) {
       ela::StepArgs<T> a = base_args<T>(h, ad.p0, ad.p1);
       set_pm<T>(h, a, ad);
-      for (int k = 0; k < 9; ++k) { a.accl[k] = ssL[k]; a.accr[k] = ssR[k]; }
+      a.accl = ssL[0];
+      a.accr = ssR[0];
       a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
-      CHK((launch_step_m<T, ela::MODE_BORN_ADJ_PM, ela::F_ACC, ela::F_ACC>(h, a)));
       ela::PointArgs<T> R = make_points<T>(h, rp, ad.p0, TmViews<T>(tm).v, true, nrec_tot);
       set_pm<T>(h, R, ad);
       for (int k = 0; k < 9; ++k) { R.accl[k] = ssL[k]; R.accr[k] = ssR[k]; }
       R.accfl = a.accfl; R.accfr = a.accfr;
-      launch_inject<T, true, false, true>(h, R, (int)its, f[it2 + 1], f[hh + it2 + 1]);
+      set_time(R, (int)its, f[it2 + 1], f[hh + it2 + 1]);
+      CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_ACC, ela::F_ACC>(h, a, rp, R)));
       ad.swap();
     }
     launch_imaging<T, true>(h, imaging_args<T>(h, V(its), V(its + 1), V(its + 2), its + 1, nullptr, dm, ssR));
@@ -1357,16 +1409,13 @@ struct DrvSlot {
 
 template <typename T>
 void set_drv(const ela_handle* h, ela::StepArgs<T>& a, DrvSlot d, bool store) {
-  const int64_t np = h->stride;
-  for (int c = 0; c < 9; ++c) {
-    if (d.fmt == ELA_CK_S16) {
-      a.dq16[c] = reinterpret_cast<int16_t*>(d.p) + c * np;
-      a.dqs[c] = reinterpret_cast<float*>(d.p + (size_t)9 * np * 2) + c * (np / ela::DQ_BLOCK);
-    } else if (store) {
-      a.dst[c] = reinterpret_cast<T*>(d.p) + c * np;
-    } else {
-      a.drv[c] = reinterpret_cast<const T*>(d.p) + c * np;
-    }
+  if (d.fmt == ELA_CK_S16) {
+    a.dq16 = reinterpret_cast<int16_t*>(d.p);
+    a.dqs = reinterpret_cast<float*>(d.p + (size_t)9 * h->stride * 2);
+  } else if (store) {
+    a.dst = reinterpret_cast<T*>(d.p);
+  } else {
+    a.drv = reinterpret_cast<const T*>(d.p);
   }
 }
 
@@ -1523,17 +1572,17 @@ int grad_fwd_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_t
   const double* f = h->filt.data();
   const int its = (int)(k / sub), i2 = (int)(k % sub);  // forward it2 = i2 + 1
   ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
+  ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
+  if (ds.k) set_step(h, S, ds.k, ds.off, 0);
+  set_time(S, its, f[i2], f[hh + i2]);
   if (STORE) {
     set_drv<T>(h, a, dst, true);
     constexpr int FQ = sizeof(T) == 4 ? ela::F_STORE | ela::F_Q16 : ela::F_STORE;
-    if (dst.fmt == ELA_CK_S16) CHK((launch_step_m<T, ela::MODE_FWD, FQ, FQ>(h, a)));
-    else CHK((launch_step_m<T, ela::MODE_FWD, ela::F_STORE, ela::F_STORE>(h, a)));
+    if (dst.fmt == ELA_CK_S16) CHK((step_with_points<T, ela::MODE_FWD, FQ, FQ>(h, a, sp, S)));
+    else CHK((step_with_points<T, ela::MODE_FWD, ela::F_STORE, ela::F_STORE>(h, a, sp, S)));
   } else {
-    CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a)));
+    CHK((step_with_points<T, ela::MODE_FWD, 0, 0>(h, a, sp, S)));
   }
-  ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
-  if (ds.k) set_step(h, S, ds.k, ds.off, 0);
-  launch_inject<T, false>(h, S, its, f[i2], f[hh + i2]);
   if (ds.advance) launch(h, ela::k_count, dim3(1), dim3(64), ds.k, ds.advance);
   w.swap();
   return ELA_OK;
@@ -1636,12 +1685,16 @@ int grad_forward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in
   auto step = [&](Wave<T>& wv, int64_t k, DevStep ds) -> int {
     const int its = (int)(k / sub), i2 = (int)(k % sub);
     ela::StepArgs<T> a = base_args<T>(h, wv.p0, wv.p1);
-    CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a)));
     ela::PointArgs<T> S = make_points<T>(h, sp, wv.p0, src_tr, false, 0);
-    ela::PointArgs<T> R = make_points<T>(h, rp, wv.p0, TmViews<T>(tm).v, true, nrec_tot);
-    if (ds.k) { set_step(h, S, ds.k, ds.off, 0); set_step(h, R, ds.k, ds.off, 1); }
-    launch_inject<T, false>(h, S, its, f[i2], f[hh + i2]);
-    launch_record<T>(h, R, its, f[i2 + 1], f[hh + i2 + 1]);
+    // the level step k reads, which step k - 1 left (none before the first)
+    ela::PointArgs<T> R = make_points<T>(h, rp, wv.p1, TmViews<T>(tm).v, true, nrec_tot);
+    if (ds.k) { set_step(h, S, ds.k, ds.off, 0); set_step(h, R, ds.k, ds.off - 1, 1); }
+    R.nmax = (int)N;
+    set_time(S, its, f[i2], f[hh + i2]);
+    const int64_t kr = std::max<int64_t>(k - 1, 0), ir = kr % sub;
+    set_time(R, (int)(kr / sub), f[ir + 1], f[hh + ir + 1]);
+    if (!ds.k && k == 0) R.off[9] = 0;
+    CHK((step_with_points<T, ela::MODE_FWD, 0, 0>(h, a, sp, S, R)));
     if (ds.advance) launch(h, ela::k_count, dim3(1), dim3(64), ds.k, ds.advance);
     wv.swap();
     return ELA_OK;
@@ -1677,6 +1730,8 @@ int grad_forward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in
     }
   }
   if (ex) HIPCHK(hipEventRecord(h->graphs[G_FWD_REC].done, h->stream));
+  launch_record<T>(h, make_points<T>(h, rp, w.p1, TmViews<T>(tm).v, true, nrec_tot), (int)(nts - 2), f[sub],
+                   f[hh + sub]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   h->last_steps = N;
   int64_t off = 0;
@@ -1773,18 +1828,25 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
     ela::StepArgs<T> a = base_args<T>(h, av.p0, av.p1);
     set_pm<T>(h, a, av);
     set_drv<T>(h, a, d, false);
-    for (int m = 0; m < 8; ++m) a.grad[m] = g32 + m * np;
+    a.grad = g32;
     constexpr int FQ = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
-    if (d.fmt == ELA_CK_S16) CHK((launch_step_m<T, ela::MODE_BORN_ADJ_PM, FQ, FQ>(h, a)));
-    else CHK((launch_step_m<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, a)));
     ela::PointArgs<T> R = make_points<T>(h, rp, av.p0, TmViews<T>(tm_adj).v, true, nrec_tot);
     set_pm<T>(h, R, av);
-    for (int c = 0; c < 9; ++c) { R.drv[c] = a.drv[c]; R.dq16[c] = a.dq16[c]; R.dqs[c] = a.dqs[c]; }
-    for (int m = 0; m < 8; ++m) R.grad[m] = a.grad[m];
-    ela::PointArgs<T> S = make_points<T>(h, sp, av.p0, TmViews<T>(tm_src).v, true, nsrc_tot);
-    if (ds.k) { set_step(h, R, ds.k, ds.off, 1); set_step(h, S, ds.k, ds.off, 0); }
-    launch_inject<T, false, true, true>(h, R, its, f[i2 + 1], f[hh + i2 + 1]);
-    launch_record<T>(h, S, its, f[i2], f[hh + i2]);
+    for (int c = 0; c < 9; ++c) {
+      if (a.drv) R.drv[c] = a.drv + c * np;
+      if (a.dq16) { R.dq16[c] = a.dq16 + c * np; R.dqs[c] = a.dqs + c * (np / ela::DQ_BLOCK); }
+    }
+    for (int m = 0; m < 8; ++m) R.grad[m] = g32 + m * np;
+    // the level step k reads, which step k + 1 left (none before the first)
+    ela::PointArgs<T> S = make_points<T>(h, sp, av.p1, TmViews<T>(tm_src).v, true, nsrc_tot);
+    if (ds.k) { set_step(h, R, ds.k, ds.off, 1); set_step(h, S, ds.k, ds.off + 1, 0); }
+    S.nmax = (int)N;
+    set_time(R, its, f[i2 + 1], f[hh + i2 + 1]);
+    const int64_t kr = std::min(k + 1, N - 1), ir = kr % sub;
+    set_time(S, (int)(kr / sub), f[ir], f[hh + ir]);
+    if (!ds.k && k == N - 1) S.off[9] = 0;
+    if (d.fmt == ELA_CK_S16) CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, FQ, FQ>(h, a, rp, R, S)));
+    else CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, a, rp, R, S)));
     if (ds.advance) launch(h, ela::k_count, dim3(1), dim3(64), ds.k, ds.advance);
     av.swap();
     return ELA_OK;
@@ -1840,6 +1902,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
       CHK(fold_gradient<T>(h, g32, g64));
     }
   }
+  launch_record<T>(h, make_points<T>(h, sp, ad.p1, TmViews<T>(tm_src).v, true, nsrc_tot), 0, f[0], f[hh]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   h->last_steps = steps;
   CHK(copy_out_3d(h, grad8, g64, 8, mem, sizeof(double)));
@@ -1907,7 +1970,7 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   ela::StepArgs<T> g = base_args<T>(h, ad.p0, ad.p1);
   set_pm<T>(h, g, ad);
   set_drv<T>(h, g, slot, false);
-  for (int m = 0; m < 8; ++m) g.grad[m] = (T*)h->g32.p + m * np;
+  g.grad = (T*)h->g32.p;
   constexpr int FQS = sizeof(T) == 4 ? ela::F_STORE | ela::F_Q16 : ela::F_STORE;
   constexpr int FQG = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
   auto step = [&](int which) -> int {

@@ -61,23 +61,30 @@ enum { F_SS = 1,     // add the secondary sources ssl/ssr (Born forward)
 // value restored is q s, within s / 2 (2^-16 of the block's largest value).
 constexpr int DQ_BLOCK = 32;
 
+// Every family of arrays is one buffer with the handle's array stride np, so
+// an argument is its first array; array k of a family is fam(base, k, np).
+// Inside the march np comes from an asm the compiler cannot see through: it
+// forms each address where it is used (two scalar instructions) instead of
+// keeping up to 60 pointers in scalar registers, whose spills took vector
+// registers and, read back every plane, vector instructions.
 template <typename T>
 struct StepArgs {
-  T* o[9];              // level n-1 in, level n+1 out (in place)
-  const T* c[9];        // level n
-  const T* m[8];        // scaled medium
-  const T* ssl[9];      // secondary sources (left / right coarse slices)
-  const T* ssr[9];
-  T* accl[9];           // coarse-time accumulation targets
-  T* accr[9];
-  T* dst[9];            // F_STORE: sx sy sz exx eyy ezz gxz gxy gyz of this step
-  const T* drv[9];      // F_GRAD: the same combinations stored by the matching forward step
-  T* grad[8];           // F_GRAD: gradient accumulators, one per medium array
-  const T* q[9];        // MODE_BORN_ADJ_PM: M c of the current level
-  T* qn[9];             // MODE_BORN_ADJ_PM: M n of the new level (written)
-  const T* ep[3];       // F_MED3: rho, lambda, mu
-  int16_t* dq16[9];     // F_Q16: int16 derivative combinations (written by F_STORE, read by F_GRAD)
-  float* dqs[9];        // F_Q16: their scales, one per DQ_BLOCK elements
+  T* o;                 // level n-1 in, level n+1 out (in place)
+  const T* c;           // level n
+  const T* m;           // scaled medium
+  const T* ssl;         // secondary sources (left / right coarse slices)
+  const T* ssr;
+  T* accl;              // coarse-time accumulation targets
+  T* accr;
+  T* dst;               // F_STORE: sx sy sz exx eyy ezz gxz gxy gyz of this step
+  const T* drv;         // F_GRAD: the same combinations stored by the matching forward step
+  T* grad;              // F_GRAD: gradient accumulators, one per medium array
+  const T* q;           // MODE_BORN_ADJ_PM: M c of the current level
+  T* qn;                // MODE_BORN_ADJ_PM: M n of the new level (written)
+  const T* ep;          // F_MED3: rho, lambda, mu
+  int16_t* dq16;        // F_Q16: int16 derivative combinations (written by F_STORE, read by F_GRAD)
+  float* dqs;           // F_Q16: their scales, one per DQ_BLOCK elements
+  int64_t np;           // elements between the arrays of a family
   T tdt;                // F_MED3: 2 dtw
   double tdt64;         // F_MED3: 2 dtw in FP64 (FP32 steppers form buoyancies and normal moduli in FP64)
   T ssfl, ssfr;         // filter weights for the secondary source
@@ -95,6 +102,14 @@ struct StepArgs {
   int xgroup;           // x columns per group of the y-major order
   const int* chunks;    // stacked windows: per y chunk {y0, y1, window y0, window ny, window nx}, or null
 };
+
+template <typename P>
+__device__ __forceinline__ P* fam(P* base, int k, int64_t np) { return base + k * np; }
+
+__device__ __forceinline__ int64_t opaque(int64_t v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
 
 __device__ __forceinline__ int xcd_remap(int bid, int nb) {
   const int per = nb / NXCD, rem = nb % NXCD;
@@ -272,45 +287,35 @@ __device__ __forceinline__ float load_dq16(const int16_t* q, const float* sc, ui
 template <typename T, int MODE>
 struct StressVal {
   const StepArgs<T>& a;
-  __device__ __forceinline__ T pm(int f, uint32_t i) const { return *at(a.q[f], i); }
-  __device__ __forceinline__ T sxx(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SXX, i);
-    if (MODE == MODE_BORN_ADJ)
-      return *at(a.c[SXX], i) * *at(a.m[L2M], i) + (*at(a.c[SYY], i) + *at(a.c[SZZ], i)) * *at(a.m[LAM], i);
-    return *at(a.c[SXX], i);
+  int64_t np;
+  __device__ __forceinline__ T c(int f, uint32_t i) const {
+    return *at(fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np), i);
   }
-  __device__ __forceinline__ T syy(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SYY, i);
-    if (MODE == MODE_BORN_ADJ)
-      return *at(a.c[SYY], i) * *at(a.m[L2M], i) + (*at(a.c[SXX], i) + *at(a.c[SZZ], i)) * *at(a.m[LAM], i);
-    return *at(a.c[SYY], i);
+  __device__ __forceinline__ T m(int k, uint32_t i) const { return *at(fam(a.m, k, np), i); }
+  // f: the normal stress, g and h the two others
+  __device__ __forceinline__ T normal(int f, int g, int h, uint32_t i) const {
+    if (MODE == MODE_BORN_ADJ) return c(f, i) * m(L2M, i) + (c(g, i) + c(h, i)) * m(LAM, i);
+    return c(f, i);
   }
-  __device__ __forceinline__ T szz(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SZZ, i);
-    if (MODE == MODE_BORN_ADJ)
-      return *at(a.c[SZZ], i) * *at(a.m[L2M], i) + (*at(a.c[SXX], i) + *at(a.c[SYY], i)) * *at(a.m[LAM], i);
-    return *at(a.c[SZZ], i);
+  __device__ __forceinline__ T shear(int f, int k, uint32_t i) const {
+    return MODE == MODE_BORN_ADJ ? c(f, i) * m(k, i) : c(f, i);
   }
-  __device__ __forceinline__ T sxz(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SXZ, i);
-    return MODE == MODE_BORN_ADJ ? *at(a.c[SXZ], i) * *at(a.m[MXZ], i) : *at(a.c[SXZ], i);
-  }
-  __device__ __forceinline__ T sxy(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SXY, i);
-    return MODE == MODE_BORN_ADJ ? *at(a.c[SXY], i) * *at(a.m[MXY], i) : *at(a.c[SXY], i);
-  }
-  __device__ __forceinline__ T syz(uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return pm(SYZ, i);
-    return MODE == MODE_BORN_ADJ ? *at(a.c[SYZ], i) * *at(a.m[MYZ], i) : *at(a.c[SYZ], i);
-  }
+  __device__ __forceinline__ T sxx(uint32_t i) const { return normal(SXX, SYY, SZZ, i); }
+  __device__ __forceinline__ T syy(uint32_t i) const { return normal(SYY, SXX, SZZ, i); }
+  __device__ __forceinline__ T szz(uint32_t i) const { return normal(SZZ, SXX, SYY, i); }
+  __device__ __forceinline__ T sxz(uint32_t i) const { return shear(SXZ, MXZ, i); }
+  __device__ __forceinline__ T sxy(uint32_t i) const { return shear(SXY, MXY, i); }
+  __device__ __forceinline__ T syz(uint32_t i) const { return shear(SYZ, MYZ, i); }
 };
 
 template <typename T, int MODE>
 struct VelVal {
   const StepArgs<T>& a;
+  int64_t np;
   __device__ __forceinline__ T v(int f, uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return *at(a.q[f], i);
-    return MODE == MODE_BORN_ADJ ? *at(a.c[f], i) * *at(a.m[f], i) : *at(a.c[f], i);  // BX_/BY_/BZ_ == VX/VY/VZ
+    if (MODE == MODE_BORN_ADJ_PM) return *at(fam(a.q, f, np), i);
+    const T c = *at(fam(a.c, f, np), i);
+    return MODE == MODE_BORN_ADJ ? c * *at(fam(a.m, f, np), i) : c;  // BX_/BY_/BZ_ == VX/VY/VZ
   }
 };
 
@@ -407,6 +412,221 @@ __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int n
 }
 
 // ---------------------------------------------------------------------------
+// Sparse points: injection and recording of all 9 components.
+// ---------------------------------------------------------------------------
+template <typename T>
+struct PointArgs {
+  const int32_t* pos[9];   // internal-layout positions of the component's grid (-1: skip)
+  int64_t n[9];
+  int64_t off[10];         // prefix offsets over components
+  T* field[9];             // wavefield component arrays
+  T* tr[9];                // traces
+  int64_t tr_stride_pt;    // element stride between points in tr (nts for [n][nts], 1 for [nts][n])
+  int64_t tr_stride_t;     // element stride between time samples (1 for [n][nts], n for [nts][n])
+  int its;
+  T fa, fb;                // filter weights for its and its+1
+  // optional coarse accumulation of the injected value (Born passes)
+  T* accl[9];
+  T* accr[9];
+  T accfl, accfr;
+  // optional gradient imaging of the injected value (adjoint-state gradient);
+  // with dq16 set the derivative combinations are the F_Q16 int16 arrays
+  const T* drv[9];
+  const int16_t* dq16[9];
+  const float* dqs[9];
+  T* grad[8];
+  // optional premultiplied level to keep consistent (MODE_BORN_ADJ_PM)
+  T* q[9];
+  const T* m[8];
+  // damping (injection only)
+  const T* taper;
+  int min_pad, nz, nx, ny, nzi, zoff;
+  const int* ytab;         // stacked windows: per plane {window y0, window ny, window nx, 0}, or null
+  const int* its_dev;      // coarse sample index read from device memory (graph replays), or null
+  int its_off;             // added to the index read from its_dev
+  // fine step k = *step_dev + step_off read from device memory (graph replays
+  // of gradient steps), or null: the coarse sample is k / sub and the weights
+  // are filt[i + fo] and filt[sub + 1 + i + fo] with i = k % sub (the host's
+  // fa / fb of that step)
+  const int* step_dev;
+  const T* filt;
+  int sub, fo, step_off;
+  int nmax;                // > 0: a launch whose coarse sample (its_dev) or fine step (step_dev) is outside
+                           // [0, nmax) does nothing (the recording of a level before the first or after the last)
+  const int* box;          // box of the points (see inject_tile), for an injection fused into a step
+};
+
+// Coarse sample and time-filter weights of a point launch; false: outside the record.
+// (PA: PointArgs<T>, or the same in the kernel argument segment, see inject_tile.)
+template <typename T, typename PA>
+__device__ __forceinline__ bool point_time(const PA& a, int& its, T& fa, T& fb) {
+  if (a.step_dev) {
+    const int k = *a.step_dev + a.step_off;
+    if (a.nmax && (k < 0 || k >= a.nmax)) return false;
+    its = k / a.sub;
+    const int i = k - its * a.sub + a.fo;
+    fa = a.filt[i];
+    fb = a.filt[a.sub + 1 + i];
+  } else {
+    its = a.its_dev ? *a.its_dev + a.its_off : a.its;
+    if (a.its_dev && a.nmax && (its < 0 || its >= a.nmax)) return false;
+    fa = a.fa;
+    fb = a.fb;
+  }
+  return true;
+}
+
+template <typename T>
+__device__ __forceinline__ int comp_of(const PointArgs<T>& a, int64_t g) {
+  int c = 0;
+#pragma unroll
+  for (int k = 1; k < 9; ++k) c += (g >= a.off[k]) ? 1 : 0;
+  return c;
+}
+
+template <typename T, typename PA>
+__device__ __forceinline__ T point_taper(const PA& a, int32_t p) {
+  const int ys = a.nzi * a.nx;
+  const int iy = p / ys;
+  const int rem = p - iy * ys;
+  const int ix = rem / a.nzi;
+  const int iz = rem - ix * a.nzi - a.zoff;
+  int wy0 = 0, wny = a.ny, wnx = a.nx;
+  if (a.ytab) { wy0 = a.ytab[4 * iy]; wny = a.ytab[4 * iy + 1]; wnx = a.ytab[4 * iy + 2]; }
+  int d = min(min(iz - FAT, ix - FAT), min(a.nz - iz - 1 - FAT, wnx - ix - 1 - FAT));
+  d = min(d, min(iy - wy0 - FAT, wy0 + wny - iy - 1 - FAT));
+  return d < a.min_pad ? a.taper[d] : T(1);
+}
+
+// field[pos] += w(pos) * (tr[its] fa + tr[its+1] fb)
+// (ker_inject_source_* / ker_inject_data_*, kernelsElaGpu_3D.cu:11-52, with the
+// sponge factor that the reference applies right after injection).
+// Roundings are fixed (no contraction but the written fma), so that the
+// fused and the separate injection give the same bits.
+template <typename T, bool ACC, bool GRAD, bool PM, typename PA>
+__device__ __forceinline__ void inject_point(const PA& a, int c, int64_t k) {
+#pragma clang fp contract(off)
+  const int32_t p = a.pos[c][k];
+  int its;
+  T fa, fb;
+  (void)point_time<T>(a, its, fa, fb);
+  const T taper = point_taper<T>(a, p);
+  // the injected value of component cc at this point (the three normal
+  // stresses share their point list, so index k is the same point for them)
+  auto injected = [&](int cc) {
+    const T* tr = a.tr[cc] + k * a.tr_stride_pt;
+    return taper * fma(tr[(int64_t)its * a.tr_stride_t], fa, tr[(int64_t)(its + 1) * a.tr_stride_t] * fb);
+  };
+  const T v = injected(c);
+  a.field[c][p] += v;
+  if (ACC && a.accl[c]) {
+    a.accl[c][p] += v * a.accfl;
+    a.accr[c][p] += v * a.accfr;
+  }
+  // Points are unique within a component's list, so every update below has
+  // one writer; the normal stresses, coupled through lamb2MuDtw / lambDtw,
+  // are updated together by the sxx thread, with the stepper's formulas.
+  T vn[3] = {T(0), T(0), T(0)};
+  if ((PM || GRAD) && c == SXX) { vn[0] = v; vn[1] = injected(SYY); vn[2] = injected(SZZ); }
+  if (PM) {
+    // keep q = M n
+    if (c < 3) {
+      a.q[c][p] += v * a.m[c][p];
+    } else if (c == SXX) {
+      const T l2 = a.m[L2M][p], la = a.m[LAM][p];
+      a.q[SXX][p] += vn[0] * l2 + (vn[1] + vn[2]) * la;
+      a.q[SYY][p] += vn[1] * l2 + (vn[0] + vn[2]) * la;
+      a.q[SZZ][p] += vn[2] * l2 + (vn[0] + vn[1]) * la;
+    } else if (c >= SXZ) {
+      a.q[c][p] += v * a.m[MXZ + (c - SXZ)][p];
+    }
+  }
+  if (GRAD) {
+    // the stepper imaged the level before this injection; add the injected part
+    auto drv = [&](int cc) -> T {
+      return a.dq16[cc] ? T(load_dq16(a.dq16[cc], a.dqs[cc], (uint32_t)p)) : a.drv[cc][p];
+    };
+    if (c < 3) {
+      a.grad[c][p] += v * drv(c);
+    } else if (c == SXX) {
+      const T dxx = drv(SXX), dyy = drv(SYY), dzz = drv(SZZ);
+      const T l2 = vn[0] * dxx + vn[1] * dyy + vn[2] * dzz;
+      a.grad[L2M][p] += l2;
+      a.grad[LAM][p] += (vn[0] + vn[1] + vn[2]) * (dxx + dyy + dzz) - l2;
+    } else if (c >= SXZ) {
+      a.grad[MXZ + (c - SXZ)][p] += v * drv(c);
+    }
+  }
+}
+
+// tr[its] += field[pos] fa ; tr[its+1] += field[pos] fb
+// (ker_record_interp_data_* / ker_record_source_*, kernelsElaGpu_3D.cu:61-104).
+template <typename T>
+__device__ __forceinline__ void record_point(const PointArgs<T>& a, int64_t g) {
+  if (g >= a.off[9]) return;
+  const int c = comp_of(a, g);
+  const int64_t k = g - a.off[c];
+  const int32_t p = a.pos[c][k];
+  if (p < 0) return;
+  const T v = a.field[c][p];
+  int its;
+  T fa, fb;
+  if (!point_time<T>(a, its, fa, fb)) return;
+  T* tr = a.tr[c] + k * a.tr_stride_pt;
+  T& t0 = tr[(int64_t)its * a.tr_stride_t];
+  T& t1 = tr[(int64_t)(its + 1) * a.tr_stride_t];
+  t0 = fma(v, fa, t0);
+  t1 = fma(v, fb, t1);
+}
+
+// Injection by a step's own blocks: after its march a block whose tile meets
+// the points' box adds the listed points inside its tile (components c0 ..
+// c1 - 1, those the block has written) with inject_point, so that a step with
+// few sources is one launch. With the recording moved into the step after
+// (step_with_points) that took 40x36x44, 100 steps through host arrays, from
+// 1.68 to 1.17 ms, 152x152x148 (200 steps) from 20.1 to 18.6 ms and
+// 328x472x468 with 2.9 M recorded points (80 steps) from 143.0 to 138.9 ms. The barrier orders the block's stores of the new
+// level before the read-modify-writes; no other block touches these cells.
+// box: the largest of (POS_TOP - z, z, POS_TOP - x, x, POS_TOP - y, y) over
+// the points, in internal z, so that a zeroed box holds nothing.
+constexpr int POS_TOP = 1 << 30;
+
+//
+// Everything is read again from the kernel's argument segment (k_step's
+// second argument is the injection) through an address the compiler cannot
+// trace back, and the tile worked out again from the block index: kept live
+// across the march they cost scalar registers, whose spills take vector
+// registers (130 instead of 128, i.e. 3 waves per SIMD, in some steps).
+template <typename T, int BX, bool ACC, bool GRAD, bool PM>
+__device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
+#define ELA_KERNARG __attribute__((address_space(4)))
+  uint64_t seg = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(seg));
+  const auto& s = *(const ELA_KERNARG StepArgs<T>*)seg;
+  const auto& a = *(const ELA_KERNARG PointArgs<T>*)(seg + sizeof(StepArgs<T>));
+#undef ELA_KERNARG
+  if (a.off[9] == 0) return;  // kernel-uniform
+  const int bid = (int)blockIdx.x + s.first - half * s.nbz * s.nbx * s.nby;
+  const TileCoord t = tile_coord<BX>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
+  const int* b = a.box;
+  const bool hit = POS_TOP - b[0] < t.z0 + TZ && b[1] >= t.z0 && POS_TOP - b[2] < t.x0 + BX && b[3] >= t.x0 &&
+                   POS_TOP - b[4] < t.y1 && b[5] >= t.y0;
+  if (!hit) return;  // block-uniform
+  __syncthreads();
+  for (int g = (int)a.off[c0] + t.ty * TZ + t.tz; g < (int)a.off[c1]; g += TZ * BX) {
+    int c = c0;
+#pragma nounroll   // one offset at a time in a scalar register
+    for (int k = c0 + 1; k < c1; ++k) c += g >= (int)a.off[k] ? 1 : 0;
+    const int64_t k = g - a.off[c];
+    const int32_t p = a.pos[c][k];
+    if (p < 0) continue;
+    const int row = p / a.nzi, z = p - row * a.nzi, y = row / a.nx, x = row - y * a.nx;
+    if (z >= t.z0 && z < t.z0 + TZ && x >= t.x0 && x < t.x0 + BX && y >= t.y0 && y < t.y1)
+      inject_point<T, ACC, GRAD, PM>(a, c, k);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Velocity update: vx, vy, vz from the six stresses.
 //
 // Software pipeline per y plane: the global loads of plane iy+1 (new queue
@@ -489,11 +709,12 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
   const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
-  const StressVal<T, MODE> S{a}, SXl{a}, SXh{a}, SZ{a};
+  int64_t np = a.np;
+  auto S_ = [&]() { return StressVal<T, MODE>{a, np}; };
   // FP32 rows that are plain array values go straight from HBM to LDS
   // (MODE_BORN_ADJ multiplies them by the medium first, in registers)
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
-  auto src = [&](int f) -> const T* { return MODE == MODE_BORN_ADJ_PM ? a.q[f] : a.c[f]; };
+  auto src = [&](int f) -> const T* { return fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np); };
   const int r = t.ty + FAT, q = t.tz + FAT;
   // a wave is one row of the tile (blockDim.x == TZ == wavefront size): its row index is wave-uniform
   const int wy = __builtin_amdgcn_readfirstlane(t.ty), wr = wy + FAT;
@@ -506,37 +727,37 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
       row_to_lds(src(SZZ), pl + t.col, &l_zz[nb][wr][FAT]);
       row_to_lds(src(SXZ), pl + t.col, &l_xz[nb][wr][FAT]);
     } else {
-      v.xx = S.sxx(pl + t.col);
-      v.zz = S.szz(pl + t.col);
-      v.xz = S.sxz(pl + t.col);
+      v.xx = S_().sxx(pl + t.col);
+      v.zz = S_().szz(pl + t.col);
+      v.xz = S_().sxz(pl + t.col);
     }
-    v.nxy = S.sxy(pl + 4 * ys + t.col);
-    v.nyy = S.syy(pl + 3 * ys + t.col);
-    v.nyz = S.syz(pl + 4 * ys + t.col);
+    v.nxy = S_().sxy(pl + 4 * ys + t.col);
+    v.nyy = S_().syy(pl + 3 * ys + t.col);
+    v.nyz = S_().syz(pl + 4 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
         row_to_lds(src(SXX), pl + t.cxl, &l_xx[nb][wy][FAT]); row_to_lds(src(SXX), pl + t.cxh, &l_xx[nb][wr + BX][FAT]);
         row_to_lds(src(SXY), pl + t.cxl, &l_xy[nb][wy][FAT]); row_to_lds(src(SXY), pl + t.cxh, &l_xy[nb][wr + BX][FAT]);
         row_to_lds(src(SXZ), pl + t.cxl, &l_xz[nb][wy][FAT]); row_to_lds(src(SXZ), pl + t.cxh, &l_xz[nb][wr + BX][FAT]);
       } else {
-        v.hxx0 = SXl.sxx(pl + t.cxl); v.hxx1 = SXh.sxx(pl + t.cxh);
-        v.hxy0 = SXl.sxy(pl + t.cxl); v.hxy1 = SXh.sxy(pl + t.cxh);
-        v.hxz0 = SXl.sxz(pl + t.cxl); v.hxz1 = SXh.sxz(pl + t.cxh);
+        v.hxx0 = S_().sxx(pl + t.cxl); v.hxx1 = S_().sxx(pl + t.cxh);
+        v.hxy0 = S_().sxy(pl + t.cxl); v.hxy1 = S_().sxy(pl + t.cxh);
+        v.hxz0 = S_().sxz(pl + t.cxl); v.hxz1 = S_().sxz(pl + t.cxh);
       }
     }
     if (t.zh) {
-      v.hzz = SZ.szz(pl + t.czh); v.hxz = SZ.sxz(pl + t.czh); v.hyz = SZ.syz(pl + t.czh);
+      v.hzz = S_().szz(pl + t.czh); v.hxz = S_().sxz(pl + t.czh); v.hyz = S_().syz(pl + t.czh);
     }
     if (MED3) {
       // the column's own cell and its x - 1 / z - 1 neighbours
       if constexpr (DMA) {
-        row_to_lds(a.ep[0], pl + t.col, &l_rho[nb][wy + 1][1]);
-        if (wy == 0) row_to_lds(a.ep[0], pl + t.col - (uint32_t)a.nzi, &l_rho[nb][0][1]);
+        row_to_lds(fam(a.ep, 0, np), pl + t.col, &l_rho[nb][wy + 1][1]);
+        if (wy == 0) row_to_lds(fam(a.ep, 0, np), pl + t.col - (uint32_t)a.nzi, &l_rho[nb][0][1]);
       } else {
-        v.rho = *at(a.ep[0], pl + t.col);
-        if (t.ty == 0) v.rho_hx = *at(a.ep[0], pl + t.col - (uint32_t)a.nzi);
+        v.rho = *at(fam(a.ep, 0, np), pl + t.col);
+        if (t.ty == 0) v.rho_hx = *at(fam(a.ep, 0, np), pl + t.col - (uint32_t)a.nzi);
       }
-      if (t.tz == 0) v.rho_hz = *at(a.ep[0], pl + t.col - 1u);
+      if (t.tz == 0) v.rho_hz = *at(fam(a.ep, 0, np), pl + t.col - 1u);
     }
   };
   // the values fetch kept in registers, and the queue centres
@@ -558,15 +779,15 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     }
   };
   // F_MED3: density of the column on the previous plane (y - 1)
-  T rho_prev = MED3 ? *at(a.ep[0], (uint32_t)(t.y0 - 1) * ys + t.col) : T(0);
+  T rho_prev = MED3 ? *at(fam(a.ep, 0, np), (uint32_t)(t.y0 - 1) * ys + t.col) : T(0);
 
   // queues: sxy (D+y, q[j] = f[iy-3+j]), syy (D-y, f[iy-4+j]), syz (D+y)
   T qxy[8], qyy[8], qyz[8];
 #pragma unroll
   for (int j = 0; j < 7; ++j) {
-    qxy[j] = S.sxy((uint32_t)(t.y0 - 3 + j) * ys + t.col);
-    qyy[j] = S.syy((uint32_t)(t.y0 - 4 + j) * ys + t.col);
-    qyz[j] = S.syz((uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qxy[j] = S_().sxy((uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qyy[j] = S_().syy((uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qyz[j] = S_().syz((uint32_t)(t.y0 - 3 + j) * ys + t.col);
   }
   {
     VelStage<T> v0;
@@ -578,6 +799,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
   int b = 0;
   for (int iy = t.y0; iy < t.y1; ++iy) {
     const bool more = iy + 1 < t.y1;
+    np = opaque(a.np);
     VelStage<T> nx_;
     if (more) fetch(nx_, iy + 1, b ^ 1);  // buffer b ^ 1 is free: every wave passed the last barrier
     // F_STORE with F_Q16: the whole wave of an interior row takes the branch
@@ -590,18 +812,18 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
       // issued after a store waits for it); FP64 loads them where they are
       // used, which holds fewer registers (2 waves per SIMD)
       T o3[3], m3[3], ss3[3], al3[3], ar3[3], g3[3], d3[3];
-      auto load_ss = [&](int f) { return *at(a.ssl[f], i) * a.ssfl + *at(a.ssr[f], i) * a.ssfr; };
+      auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
-        o3[f] = ld_nt(a.o[f], i);
-        if (!MED3 && MODE != MODE_BORN_ADJ) m3[f] = ld_nt(a.m[f], i);
+        o3[f] = ld_nt(fam(a.o, f, np), i);
+        if (!MED3 && MODE != MODE_BORN_ADJ) m3[f] = ld_nt(fam(a.m, f, np), i);
         if constexpr (HOIST) {
           if (SS) ss3[f] = load_ss(f);
-          if (ACC) { al3[f] = *at(a.accl[f], i); ar3[f] = *at(a.accr[f], i); }
+          if (ACC) { al3[f] = *at(fam(a.accl, f, np), i); ar3[f] = *at(fam(a.accr, f, np), i); }
           if (F & F_GRAD) {  // BX_/BY_/BZ_ == VX/VY/VZ
-            g3[f] = *at(a.grad[f], i);
-            if constexpr (Q16) d3[f] = load_dq16(a.dq16[f], a.dqs[f], i);
-            else d3[f] = ld_nt(a.drv[f], i);
+            g3[f] = *at(fam(a.grad, f, np), i);
+            if constexpr (Q16) d3[f] = load_dq16(fam(a.dq16, f, np), fam(a.dqs, f, np / DQ_BLOCK), i);
+            else d3[f] = ld_nt(fam(a.drv, f, np), i);
           }
         }
       }
@@ -620,8 +842,8 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
       if (F & F_STORE) {
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
-          if constexpr (QS) store_dq16(a.dq16[f], a.dqs[f], i, t.active ? s3[f] : T(0));
-          else st_nt(a.dst[f], i, s3[f]);
+          if constexpr (QS) store_dq16(fam(a.dq16, f, np), fam(a.dqs, f, np / DQ_BLOCK), i, t.active ? s3[f] : T(0));
+          else st_nt(fam(a.dst, f, np), i, s3[f]);
         }
       }
 #pragma unroll
@@ -632,19 +854,19 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
         else u = w * o3[f] - s3[f];
         if constexpr (!HOIST) {
           if (SS) ss3[f] = load_ss(f);
-          if (ACC) { al3[f] = *at(a.accl[f], i); ar3[f] = *at(a.accr[f], i); }
-          if (F & F_GRAD) { g3[f] = *at(a.grad[f], i); d3[f] = ld_nt(a.drv[f], i); }
+          if (ACC) { al3[f] = *at(fam(a.accl, f, np), i); ar3[f] = *at(fam(a.accr, f, np), i); }
+          if (F & F_GRAD) { g3[f] = *at(fam(a.grad, f, np), i); d3[f] = ld_nt(fam(a.drv, f, np), i); }
         }
         if (SS) u += ss3[f];
         u *= w;
         if (QS && !t.active) continue;
-        st_nt(a.o[f], i, u);
-        if (MODE == MODE_BORN_ADJ_PM) st_nt(a.qn[f], i, u * m3[f]);
+        st_nt(fam(a.o, f, np), i, u);
+        if (MODE == MODE_BORN_ADJ_PM) st_nt(fam(a.qn, f, np), i, u * m3[f]);
         if (ACC) {
-          *at(a.accl[f], i) = al3[f] + u * a.accfl;
-          *at(a.accr[f], i) = ar3[f] + u * a.accfr;
+          *at(fam(a.accl, f, np), i) = al3[f] + u * a.accfl;
+          *at(fam(a.accr, f, np), i) = ar3[f] + u * a.accfr;
         }
-        if (F & F_GRAD) *at(a.grad[f], i) = g3[f] + u * d3[f];
+        if (F & F_GRAD) *at(fam(a.grad, f, np), i) = g3[f] + u * d3[f];
       }
     }
     if (MED3) rho_prev = l_rho[b][t.ty + 1][t.tz + 1];
@@ -657,6 +879,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     __syncthreads();
     b ^= 1;
   }
+  inject_tile<T, BX, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
 }
 
 // ---------------------------------------------------------------------------
@@ -690,19 +913,20 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
-  const VelVal<T, MODE> V{a}, Vlo{a}, Vhi{a}, Vzh{a};
+  int64_t np = a.np;
+  auto V_ = [&]() { return VelVal<T, MODE>{a, np}; };
   // FP32 rows that are plain array values go straight from HBM to LDS (see velocity_block)
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
-  auto src = [&](int f) -> const T* { return MODE == MODE_BORN_ADJ_PM ? a.q[f] : a.c[f]; };
+  auto src = [&](int f) -> const T* { return fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np); };
   const int r = t.ty + FAT, q = t.tz + FAT;
   const int wy = __builtin_amdgcn_readfirstlane(t.ty), wr = wy + FAT;  // wave-uniform row
 
   // plane p's values: LDS rows of buffer nb directly (DMA), the rest into v
   auto fetch = [&](StressStage<T>& v, int p, int nb) {
     const uint32_t pl = (uint32_t)p * ys;
-    v.nx = V.v(VX, pl + 3 * ys + t.col);
-    v.ny = V.v(VY, pl + 4 * ys + t.col);
-    v.nz = V.v(VZ, pl + 3 * ys + t.col);
+    v.nx = V_().v(VX, pl + 3 * ys + t.col);
+    v.ny = V_().v(VY, pl + 4 * ys + t.col);
+    v.nz = V_().v(VZ, pl + 3 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
         row_to_lds(src(VX), pl + t.cxl, &l_vx[nb][wy][FAT]); row_to_lds(src(VX), pl + t.cxh, &l_vx[nb][wr + BX][FAT]);
@@ -710,26 +934,26 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         row_to_lds(src(VZ), pl + t.cxl, &l_vz[nb][wy][FAT]); row_to_lds(src(VZ), pl + t.cxh, &l_vz[nb][wr + BX][FAT]);
       } else {
 #pragma unroll
-        for (int f = 0; f < 3; ++f) { v.hlo[f] = Vlo.v(f, pl + t.cxl); v.hhi[f] = Vhi.v(f, pl + t.cxh); }
+        for (int f = 0; f < 3; ++f) { v.hlo[f] = V_().v(f, pl + t.cxl); v.hhi[f] = V_().v(f, pl + t.cxh); }
       }
     }
     if (t.zh) {
 #pragma unroll
-      for (int f = 0; f < 3; ++f) v.hz[f] = Vzh.v(f, pl + t.czh);
+      for (int f = 0; f < 3; ++f) v.hz[f] = V_().v(f, pl + t.czh);
     }
   };
   // F_MED3: shear modulus of plane p around the column
   auto fetch_mu = [&](StressStage<T>& v, int p, int nb) {
     const uint32_t pl = (uint32_t)p * ys, nzi = (uint32_t)a.nzi;
     if constexpr (DMA) {
-      row_to_lds(a.ep[2], pl + t.col, &l_mu[nb][wy + 1][1]);
-      if (wy == 0) row_to_lds(a.ep[2], pl + t.col - nzi, &l_mu[nb][0][1]);
+      row_to_lds(fam(a.ep, 2, np), pl + t.col, &l_mu[nb][wy + 1][1]);
+      if (wy == 0) row_to_lds(fam(a.ep, 2, np), pl + t.col - nzi, &l_mu[nb][0][1]);
     } else {
-      v.mu = *at(a.ep[2], pl + t.col);
-      if (t.ty == 0) v.mu_hx = *at(a.ep[2], pl + t.col - nzi);
+      v.mu = *at(fam(a.ep, 2, np), pl + t.col);
+      if (t.ty == 0) v.mu_hx = *at(fam(a.ep, 2, np), pl + t.col - nzi);
     }
-    if (t.tz == 0) v.mu_hz = *at(a.ep[2], pl + t.col - 1u);
-    if (t.ty == 0 && t.tz == 0) v.mu_hc = *at(a.ep[2], pl + t.col - nzi - 1u);
+    if (t.tz == 0) v.mu_hz = *at(fam(a.ep, 2, np), pl + t.col - 1u);
+    if (t.ty == 0 && t.tz == 0) v.mu_hc = *at(fam(a.ep, 2, np), pl + t.col - nzi - 1u);
   };
   auto stage_mu = [&](int m, const StressStage<T>& v) {
     if constexpr (!DMA) {
@@ -754,9 +978,9 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   T qx[8], qy[8], qz[8];
 #pragma unroll
   for (int j = 0; j < 7; ++j) {
-    qx[j] = V.v(VX, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
-    qy[j] = V.v(VY, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
-    qz[j] = V.v(VZ, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qx[j] = V_().v(VX, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qy[j] = V_().v(VY, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qz[j] = V_().v(VZ, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
   }
   // F_MED3: the previous plane's terms carried in registers -- Sx(mu) of the
   // column, mu of the column and of its z - 1 neighbour -- which are the
@@ -764,9 +988,9 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   T sx_prev = T(0), mu_prev = T(0), muz_prev = T(0);
   if (MED3) {
     const uint32_t pl = (uint32_t)(t.y0 - 1) * ys;
-    mu_prev = *at(a.ep[2], pl + t.col);
-    muz_prev = *at(a.ep[2], pl + t.col - 1u);
-    sx_prev = T(0.5) * (mu_prev + *at(a.ep[2], pl + t.col - (uint32_t)a.nzi));
+    mu_prev = *at(fam(a.ep, 2, np), pl + t.col);
+    muz_prev = *at(fam(a.ep, 2, np), pl + t.col - 1u);
+    sx_prev = T(0.5) * (mu_prev + *at(fam(a.ep, 2, np), pl + t.col - (uint32_t)a.nzi));
   }
   {
     StressStage<T> v0;
@@ -782,6 +1006,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   int b = 0;
   for (int iy = t.y0; iy < t.y1; ++iy) {
     const bool more = iy + 1 < t.y1;
+    np = opaque(a.np);
     StressStage<T> nx_;
     if (more) {  // buffer b ^ 1 is free: every wave passed the last barrier
       fetch(nx_, iy + 1, b ^ 1);
@@ -792,22 +1017,22 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
       // FP32: every per-cell operand is loaded before the first store (see velocity_block)
       T o6[6], ss6[6], al6[6], ar6[6], g5[5], d6[6];
-      auto load_ss = [&](int f) { return *at(a.ssl[f], i) * a.ssfl + *at(a.ssr[f], i) * a.ssfr; };
+      auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
       auto load_grad = [&]() {
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-          if constexpr (Q16) d6[k] = load_dq16(a.dq16[SXX + k], a.dqs[SXX + k], i);
-          else d6[k] = ld_nt(a.drv[SXX + k], i);
+          if constexpr (Q16) d6[k] = load_dq16(fam(a.dq16, SXX + k, np), fam(a.dqs, SXX + k, np / DQ_BLOCK), i);
+          else d6[k] = ld_nt(fam(a.drv, SXX + k, np), i);
         }
 #pragma unroll
-        for (int m = 0; m < 5; ++m) g5[m] = *at(a.grad[L2M + m], i);
+        for (int m = 0; m < 5; ++m) g5[m] = *at(fam(a.grad, L2M + m, np), i);
       };
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
-        o6[k] = ld_nt(a.o[SXX + k], i);
+        o6[k] = ld_nt(fam(a.o, SXX + k, np), i);
         if constexpr (HOIST) {
           if (SS) ss6[k] = load_ss(SXX + k);
-          if (ACC) { al6[k] = *at(a.accl[SXX + k], i); ar6[k] = *at(a.accr[SXX + k], i); }
+          if (ACC) { al6[k] = *at(fam(a.accl, SXX + k, np), i); ar6[k] = *at(fam(a.accr, SXX + k, np), i); }
         }
       }
       if constexpr (HOIST && (F & F_GRAD) != 0) load_grad();
@@ -816,7 +1041,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         const int rr = t.ty + 1, qq = t.tz + 1;
         const T mu_c = l_mu[b][rr][qq], mu_xm = l_mu[b][rr - 1][qq], mu_zm = l_mu[b][rr][qq - 1];
         const T mu_xzm = l_mu[b][rr - 1][qq - 1];
-        const T lr = ld_nt(a.ep[1], i);
+        const T lr = ld_nt(fam(a.ep, 1, np), i);
         normal_moduli(a.tdt, a.tdt64, lr, mu_c, l2m, lam);
         const T sx_c = T(0.5) * (mu_c + mu_xm), sx_zm = T(0.5) * (mu_zm + mu_xzm);
         const T sy_c = T(0.5) * (mu_c + mu_prev), sy_zm = T(0.5) * (mu_zm + muz_prev);
@@ -824,8 +1049,8 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         mxy = (T(0.5) * (sx_c + sx_prev)) * a.tdt;
         myz = (T(0.5) * (sy_c + sy_zm)) * a.tdt;
       } else if (MODE != MODE_BORN_ADJ) {
-        l2m = ld_nt(a.m[L2M], i); lam = ld_nt(a.m[LAM], i);
-        mxz = ld_nt(a.m[MXZ], i); mxy = ld_nt(a.m[MXY], i); myz = ld_nt(a.m[MYZ], i);
+        l2m = ld_nt(fam(a.m, L2M, np), i); lam = ld_nt(fam(a.m, LAM, np), i);
+        mxz = ld_nt(fam(a.m, MXZ, np), i); mxy = ld_nt(fam(a.m, MXY, np), i); myz = ld_nt(fam(a.m, MYZ, np), i);
       }
       const T exx = dpx<T, BX>(l_vx[b], r, q, cx);
       const T eyy = dq(qy, cy);
@@ -839,10 +1064,10 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         if constexpr (QS) {
           const T e6[6] = {exx, eyy, ezz, gxz, gxy, gyz};
 #pragma unroll
-          for (int k = 0; k < 6; ++k) store_dq16(a.dq16[SXX + k], a.dqs[SXX + k], i, t.active ? e6[k] : T(0));
+          for (int k = 0; k < 6; ++k) store_dq16(fam(a.dq16, SXX + k, np), fam(a.dqs, SXX + k, np / DQ_BLOCK), i, t.active ? e6[k] : T(0));
         } else {
-          st_nt(a.dst[SXX], i, exx); st_nt(a.dst[SYY], i, eyy); st_nt(a.dst[SZZ], i, ezz);
-          st_nt(a.dst[SXZ], i, gxz); st_nt(a.dst[SXY], i, gxy); st_nt(a.dst[SYZ], i, gyz);
+          st_nt(fam(a.dst, SXX, np), i, exx); st_nt(fam(a.dst, SYY, np), i, eyy); st_nt(fam(a.dst, SZZ, np), i, ezz);
+          st_nt(fam(a.dst, SXZ, np), i, gxz); st_nt(fam(a.dst, SXY, np), i, gxy); st_nt(fam(a.dst, SYZ, np), i, gyz);
         }
       }
       T u[6];
@@ -867,26 +1092,26 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         const int f = SXX + k;
         if constexpr (!HOIST) {
           if (SS) ss6[k] = load_ss(f);
-          if (ACC) { al6[k] = *at(a.accl[f], i); ar6[k] = *at(a.accr[f], i); }
+          if (ACC) { al6[k] = *at(fam(a.accl, f, np), i); ar6[k] = *at(fam(a.accr, f, np), i); }
         }
         T v = u[k];
         if (SS) v += ss6[k];
         v *= w;
         u[k] = v;
         if (QS && !t.active) continue;
-        st_nt(a.o[f], i, v);
+        st_nt(fam(a.o, f, np), i, v);
         if (ACC) {
-          *at(a.accl[f], i) = al6[k] + v * a.accfl;
-          *at(a.accr[f], i) = ar6[k] + v * a.accfr;
+          *at(fam(a.accl, f, np), i) = al6[k] + v * a.accfl;
+          *at(fam(a.accr, f, np), i) = ar6[k] + v * a.accfr;
         }
       }
       if (MODE == MODE_BORN_ADJ_PM) {
-        st_nt(a.qn[SXX], i, u[0] * l2m + (u[1] + u[2]) * lam);
-        st_nt(a.qn[SYY], i, u[1] * l2m + (u[0] + u[2]) * lam);
-        st_nt(a.qn[SZZ], i, u[2] * l2m + (u[0] + u[1]) * lam);
-        st_nt(a.qn[SXZ], i, u[3] * mxz);
-        st_nt(a.qn[SXY], i, u[4] * mxy);
-        st_nt(a.qn[SYZ], i, u[5] * myz);
+        st_nt(fam(a.qn, SXX, np), i, u[0] * l2m + (u[1] + u[2]) * lam);
+        st_nt(fam(a.qn, SYY, np), i, u[1] * l2m + (u[0] + u[2]) * lam);
+        st_nt(fam(a.qn, SZZ, np), i, u[2] * l2m + (u[0] + u[1]) * lam);
+        st_nt(fam(a.qn, SXZ, np), i, u[3] * mxz);
+        st_nt(fam(a.qn, SXY, np), i, u[4] * mxy);
+        st_nt(fam(a.qn, SYZ, np), i, u[5] * myz);
       }
       if (F & F_GRAD) {
         // lamb2MuDtw multiplies exx, eyy, ezz in sxx, syy, szz; lambDtw the
@@ -894,11 +1119,11 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         if constexpr (!HOIST) load_grad();
         const T dxx = d6[0], dyy = d6[1], dzz = d6[2];
         const T l2 = u[0] * dxx + u[1] * dyy + u[2] * dzz;
-        *at(a.grad[L2M], i) = g5[0] + l2;
-        *at(a.grad[LAM], i) = g5[1] + ((u[0] + u[1] + u[2]) * (dxx + dyy + dzz) - l2);
-        *at(a.grad[MXZ], i) = g5[2] + u[3] * d6[3];
-        *at(a.grad[MXY], i) = g5[3] + u[4] * d6[4];
-        *at(a.grad[MYZ], i) = g5[4] + u[5] * d6[5];
+        *at(fam(a.grad, L2M, np), i) = g5[0] + l2;
+        *at(fam(a.grad, LAM, np), i) = g5[1] + ((u[0] + u[1] + u[2]) * (dxx + dyy + dzz) - l2);
+        *at(fam(a.grad, MXZ, np), i) = g5[2] + u[3] * d6[3];
+        *at(fam(a.grad, MXY, np), i) = g5[3] + u[4] * d6[4];
+        *at(fam(a.grad, MYZ, np), i) = g5[4] + u[5] * d6[5];
       }
     }
 #pragma unroll
@@ -918,6 +1143,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
     __syncthreads();
     b ^= 1;
   }
+  inject_tile<T, BX, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -938,7 +1164,7 @@ constexpr int step_waves() {
 }
 
 template <typename T, int BX, int MODE, int FV, int FS>
-__global__ void __launch_bounds__(TZ * BX, (step_waves<T, FV, FS>())) k_step(StepArgs<T> a) {
+__global__ void __launch_bounds__(TZ * BX, (step_waves<T, FV, FS>())) k_step(StepArgs<T> a, PointArgs<T> inj, PointArgs<T> rec) {
   // one LDS object: the compiler's wait analysis then tells the rows the
   // direct loads fill (buffer b ^ 1) from the rows the stencil reads (buffer b)
   union Lds {
@@ -946,170 +1172,27 @@ __global__ void __launch_bounds__(TZ * BX, (step_waves<T, FV, FS>())) k_step(Ste
     StressLds<T, BX, (FS & F_MED3) != 0> s;
   };
   __shared__ Lds L;
+  (void)inj;  // read by inject_tile
+  static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
   if (bid < nb) velocity_block<T, BX, MODE, FV>(a, bid, L.v);
-  else stress_block<T, BX, MODE, FS>(a, bid - nb, L.s);
+  else if (bid < 2 * nb) stress_block<T, BX, MODE, FS>(a, bid - nb, L.s);
+  else record_point(rec, (int64_t)(bid - 2 * nb) * (TZ * BX) + threadIdx.y * TZ + threadIdx.x);
 }
 
-// ---------------------------------------------------------------------------
-// Sparse point kernels. One launch covers all 9 components.
-// ---------------------------------------------------------------------------
-template <typename T>
-struct PointArgs {
-  const int32_t* pos[9];   // internal-layout positions of the component's grid (-1: skip)
-  int64_t n[9];
-  int64_t off[10];         // prefix offsets over components
-  T* field[9];             // wavefield component arrays
-  T* tr[9];                // traces
-  int64_t tr_stride_pt;    // element stride between points in tr (nts for [n][nts], 1 for [nts][n])
-  int64_t tr_stride_t;     // element stride between time samples (1 for [n][nts], n for [nts][n])
-  int its;
-  T fa, fb;                // filter weights for its and its+1
-  // optional coarse accumulation of the injected value (Born passes)
-  T* accl[9];
-  T* accr[9];
-  T accfl, accfr;
-  // optional gradient imaging of the injected value (adjoint-state gradient);
-  // with dq16 set the derivative combinations are the F_Q16 int16 arrays
-  const T* drv[9];
-  const int16_t* dq16[9];
-  const float* dqs[9];
-  T* grad[8];
-  // optional premultiplied level to keep consistent (MODE_BORN_ADJ_PM)
-  T* q[9];
-  const T* m[8];
-  // damping (injection only)
-  const T* taper;
-  int min_pad, nz, nx, ny, nzi, zoff;
-  const int* ytab;         // stacked windows: per plane {window y0, window ny, window nx, 0}, or null
-  const int* its_dev;      // coarse sample index read from device memory (graph replays), or null
-  // fine step k = *step_dev + step_off read from device memory (graph replays
-  // of gradient steps), or null: the coarse sample is k / sub and the weights
-  // are filt[i + fo] and filt[sub + 1 + i + fo] with i = k % sub (the host's
-  // fa / fb of that step)
-  const int* step_dev;
-  const T* filt;
-  int sub, fo, step_off;
-};
-
-// Coarse sample and time-filter weights of a point launch.
-template <typename T>
-__device__ __forceinline__ void point_time(const PointArgs<T>& a, int& its, T& fa, T& fb) {
-  if (a.step_dev) {
-    const int k = *a.step_dev + a.step_off;
-    its = k / a.sub;
-    const int i = k - its * a.sub + a.fo;
-    fa = a.filt[i];
-    fb = a.filt[a.sub + 1 + i];
-  } else {
-    its = a.its_dev ? *a.its_dev : a.its;
-    fa = a.fa;
-    fb = a.fb;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ int comp_of(const PointArgs<T>& a, int64_t g) {
-  int c = 0;
-#pragma unroll
-  for (int k = 1; k < 9; ++k) c += (g >= a.off[k]) ? 1 : 0;
-  return c;
-}
-
-template <typename T>
-__device__ __forceinline__ T point_taper(const PointArgs<T>& a, int32_t p) {
-  const int ys = a.nzi * a.nx;
-  const int iy = p / ys;
-  const int rem = p - iy * ys;
-  const int ix = rem / a.nzi;
-  const int iz = rem - ix * a.nzi - a.zoff;
-  int wy0 = 0, wny = a.ny, wnx = a.nx;
-  if (a.ytab) { wy0 = a.ytab[4 * iy]; wny = a.ytab[4 * iy + 1]; wnx = a.ytab[4 * iy + 2]; }
-  int d = min(min(iz - FAT, ix - FAT), min(a.nz - iz - 1 - FAT, wnx - ix - 1 - FAT));
-  d = min(d, min(iy - wy0 - FAT, wy0 + wny - iy - 1 - FAT));
-  return d < a.min_pad ? a.taper[d] : T(1);
-}
-
-// field[pos] += w(pos) * (tr[its] fa + tr[its+1] fb)
-// (ker_inject_source_* / ker_inject_data_*, kernelsElaGpu_3D.cu:11-52, with the
-// sponge factor that the reference applies right after injection).
+// The injection by itself: lists too long or too spread for a step's blocks.
 template <typename T, bool ACC, bool GRAD = false, bool PM = false>
 __global__ void __launch_bounds__(256) k_inject(PointArgs<T> a) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= a.off[9]) return;
   const int c = comp_of(a, g);
   const int64_t k = g - a.off[c];
-  const int32_t p = a.pos[c][k];
-  if (p < 0) return;
-  int its;
-  T fa, fb;
-  point_time(a, its, fa, fb);
-  const T taper = point_taper(a, p);
-  // the injected value of component cc at this point (the three normal
-  // stresses share their point list, so index k is the same point for them)
-  auto injected = [&](int cc) {
-    const T* tr = a.tr[cc] + k * a.tr_stride_pt;
-    return taper * (tr[(int64_t)its * a.tr_stride_t] * fa + tr[(int64_t)(its + 1) * a.tr_stride_t] * fb);
-  };
-  const T v = injected(c);
-  a.field[c][p] += v;
-  if (ACC && a.accl[c]) {
-    a.accl[c][p] += v * a.accfl;
-    a.accr[c][p] += v * a.accfr;
-  }
-  // Points are unique within a component's list, so every update below has
-  // one writer; the normal stresses, coupled through lamb2MuDtw / lambDtw,
-  // are updated together by the sxx thread, with the stepper's formulas.
-  T vn[3] = {T(0), T(0), T(0)};
-  if ((PM || GRAD) && c == SXX) { vn[0] = v; vn[1] = injected(SYY); vn[2] = injected(SZZ); }
-  if (PM) {
-    // keep q = M n
-    if (c < 3) {
-      a.q[c][p] += v * a.m[c][p];
-    } else if (c == SXX) {
-      const T l2 = a.m[L2M][p], la = a.m[LAM][p];
-      a.q[SXX][p] += vn[0] * l2 + (vn[1] + vn[2]) * la;
-      a.q[SYY][p] += vn[1] * l2 + (vn[0] + vn[2]) * la;
-      a.q[SZZ][p] += vn[2] * l2 + (vn[0] + vn[1]) * la;
-    } else if (c >= SXZ) {
-      a.q[c][p] += v * a.m[MXZ + (c - SXZ)][p];
-    }
-  }
-  if (GRAD) {
-    // the stepper imaged the level before this injection; add the injected part
-    auto drv = [&](int cc) -> T {
-      return a.dq16[cc] ? T(load_dq16(a.dq16[cc], a.dqs[cc], (uint32_t)p)) : a.drv[cc][p];
-    };
-    if (c < 3) {
-      a.grad[c][p] += v * drv(c);
-    } else if (c == SXX) {
-      const T dxx = drv(SXX), dyy = drv(SYY), dzz = drv(SZZ);
-      const T l2 = vn[0] * dxx + vn[1] * dyy + vn[2] * dzz;
-      a.grad[L2M][p] += l2;
-      a.grad[LAM][p] += (vn[0] + vn[1] + vn[2]) * (dxx + dyy + dzz) - l2;
-    } else if (c >= SXZ) {
-      a.grad[MXZ + (c - SXZ)][p] += v * drv(c);
-    }
-  }
+  if (a.pos[c][k] >= 0) inject_point<T, ACC, GRAD, PM>(a, c, k);
 }
 
-// tr[its] += field[pos] fa ; tr[its+1] += field[pos] fb
-// (ker_record_interp_data_* / ker_record_source_*, kernelsElaGpu_3D.cu:61-104).
 template <typename T>
 __global__ void __launch_bounds__(256) k_record(PointArgs<T> a) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= a.off[9]) return;
-  const int c = comp_of(a, g);
-  const int64_t k = g - a.off[c];
-  const int32_t p = a.pos[c][k];
-  if (p < 0) return;
-  const T v = a.field[c][p];
-  int its;
-  T fa, fb;
-  point_time(a, its, fa, fb);
-  T* tr = a.tr[c] + k * a.tr_stride_pt;
-  tr[(int64_t)its * a.tr_stride_t] += v * fa;
-  tr[(int64_t)(its + 1) * a.tr_stride_t] += v * fb;
+  record_point(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // Out-of-place transpose of a [rows][cols] block (row stride ld_in) into
@@ -1304,10 +1387,11 @@ __global__ void __launch_bounds__(TZ * BX) k_imaging(ImagingArgs<T> a) {
 
 // Reference-layout flat indices -> internal-layout offsets. Positions outside
 // the FD interior are replaced by -1 (skipped by the point kernels) and
-// reported through *bad.
+// reported through *bad; box (or null) becomes the box of the others (see
+// inject_tile).
 __global__ void __launch_bounds__(256) k_convert_pos(const int64_t* __restrict__ in, int32_t* __restrict__ out,
                                                      int64_t n, int nz, int nx, int ny, int nzi, int zoff,
-                                                     const int* ytab, int* bad) {
+                                                     const int* ytab, int* bad, int* box) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t p = in[i];
@@ -1322,6 +1406,10 @@ __global__ void __launch_bounds__(256) k_convert_pos(const int64_t* __restrict__
   }
   out[i] = ok ? (int32_t)(iy * nx * nzi + ix * nzi + iz + zoff) : -1;
   if (!ok) atomicOr(bad, 1);
+  else if (box) {
+    const int c[3] = {(int)iz + zoff, (int)ix, (int)iy};
+    for (int k = 0; k < 3; ++k) { atomicMax(box + 2 * k, POS_TOP - c[k]); atomicMax(box + 2 * k + 1, c[k]); }
+  }
 }
 
 // Device-side coarse-step counter of a replayed graph: *c += delta.

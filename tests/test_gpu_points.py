@@ -1,0 +1,85 @@
+"""Injection inside a step's own blocks and recording by the step after
+(few points) against the separate injection launch (many points) and the FP64
+oracle, at tile edges and the smallest records."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.problems import random_problem, rel
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"f64": 1e-11, "f32": 5e-6}      # the parity suite's bars
+# interior 70 x 9 x 11: two z tiles (64 + 6 cells), three x tiles of 4 rows, several y chunks
+NZ, NX, NY = 78, 17, 19
+
+
+def grid(nts, sub):
+    return O.Grid(nz=NZ, nx=NX, ny=NY, nts=nts, sub=sub, dz=10.0, dx=10.0, dy=10.0, dts=0.0005 * sub, minPad=3,
+                  alphaCos=0.95)
+
+
+def edge_points():
+    """Both sides of every tile edge and the interior's corners."""
+    zs, xs, ys = (4, 67, 68, NZ - 5), (4, 7, 8, NX - 5), (4, 5, 6, 11, 12, NY - 5)
+    return np.array([(y * NX + x) * NZ + z for y in ys for x in xs for z in zs], np.int64)
+
+
+def make_prop(g, precision):
+    from elasticisolib_3d_amd.propagator import Propagator
+    return Propagator(g.nz, g.nx, g.ny, g.nts, g.sub, g.dz, g.dx, g.dy, g.dts, g.minPad, g.alphaCos, precision)
+
+
+# points per list: 9 (few, one box), 56 (504 over the 9 components: still in the blocks), 57 (513: separate launch)
+@pytest.mark.parametrize("n", [9, 56, 57])
+@pytest.mark.parametrize("precision,nts,sub,graph", [("f64", 2, 1, False), ("f64", 3, 3, False), ("f64", 4, 2, True),
+                                                     ("f32", 3, 4, True), ("f32", 3, 2, False)])
+def test_points_in_the_steps_blocks(n, precision, nts, sub, graph):
+    g = grid(nts, sub)
+    P = random_problem(g, seed=5 + n)
+    pts = edge_points()
+    P["spos"] = [np.roll(pts, 7 * k)[:n] for k in range(7)]
+    P["rpos"] = [np.roll(pts, 11 * k + 3)[:n] for k in range(7)]
+    rng = np.random.default_rng(n)
+    P["src"] = [rng.standard_normal((n, nts)) * 1e3 for _ in range(9)]
+    P["rec"] = [rng.standard_normal((n, nts)) for _ in range(9)]
+    prop = make_prop(g, precision)
+    prop.set_graph(graph)
+    prop.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+    med = P["med"]
+    fwd, adj = (O.lib_nl_forward(g, med, P["src"], P["spos"], P["rpos"]),
+                O.lib_nl_adjoint(g, med, P["rec"], P["spos"], P["rpos"]))
+    for _ in range(2):   # a repeated call replays the kept graph
+        assert rel(prop.nl_forward(P["spos"], P["src"], P["rpos"]), fwd) < TOL[precision]
+        assert rel(prop.nl_adjoint(P["spos"], P["rec"], P["rpos"]), adj) < TOL[precision]
+    prop.set_gradient_checkpoints(2, 0, "native")
+    g8_ref, gs_ref = O.lib_gradient(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+    rec = prop.gradient_forward(P["spos"], P["src"], P["rpos"])
+    assert rel(rec, fwd) < TOL[precision]
+    g8, gs = prop.gradient_backward(P["spos"], P["src"], P["rpos"], P["rec"])
+    assert rel(g8, g8_ref) < 2 * TOL[precision] and rel(gs, gs_ref) < 2 * TOL[precision]
+    if nts >= 3:
+        born = O.lib_born_forward(g, med, P["src"], P["spos"], P["dm"], P["rpos"])
+        assert rel(prop.born_forward(P["spos"], P["src"], P["dm"], P["rpos"]), born) < TOL[precision]
+        img = O.lib_born_adjoint(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+        assert rel(prop.born_adjoint(P["spos"], P["src"], P["rec"], P["rpos"]), img) < TOL[precision]
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_fused_and_separate_injection_give_the_same_bits(precision):
+    """The tile shape decides whether a list's box is small enough for the
+    blocks (8 rows and 24 planes: at most 1024 tiles meet it; 4 rows and
+    single planes: more do), and the results do not depend on it."""
+    nz, nx, ny, nts, sub = 140, 90, 60, 3, 2
+    g = O.Grid(nz=nz, nx=nx, ny=ny, nts=nts, sub=sub, dz=10.0, dx=10.0, dy=10.0, dts=0.001, minPad=4, alphaCos=0.95)
+    P = random_problem(g, seed=3)
+    corner = np.array([(y * nx + x) * nz + z for y in (4, ny - 5) for x in (4, nx - 5) for z in (4, nz - 5)], np.int64)
+    pos = [corner] * 7
+    src = [np.random.default_rng(1).standard_normal((8, nts)) * 1e3 for _ in range(9)]
+    prop = make_prop(g, precision)
+    prop.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+    out = []
+    for tx, yc in ((8, 24), (4, 1)):
+        prop.set_tiling(tx, yc)
+        out.append(prop.nl_forward(pos, src, pos) + [prop.born_adjoint(pos, src, src, pos)])
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
