@@ -985,21 +985,40 @@ int nl_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, cons
 // kernels and their order are the same in all cases, so the results are
 // bit-identical.
 
-// One coarse step k of pass 1 (sub fine steps): VL = V[k], VR = V[k+1].
+// Steps j = 1 .. n whose levels are all accumulated (or imaged) in every
+// other step: step j takes its own level (1), its own and the one of step
+// j - 2, which it replaces (2), or none, step j + 2 taking it (0).
+int pair_role(int64_t j, int64_t n) {
+  const int64_t r = (j - 1) % 4;
+  return r >= 2 ? 2 : (j + 2 <= n ? 0 : 1);
+}
+
+// One coarse step k of pass 1 (sub fine steps): VL = V[k], VR = V[k+1], whose
+// interior is overwritten (the cells around it must hold zeros).
 template <typename T>
 int bg_coarse_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_tr[9], int64_t k, T* VL, T* VR) {
   const int64_t sub = h->cfg.sub, hh = sub + 1, np = h->stride;
   const double* f = h->filt.data();
+  bool first = true;   // V[k + 1] holds nothing yet
   for (int64_t it2 = 1; it2 <= sub; ++it2) {
     ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
-    a.accl = VL;
-    a.accr = VR;
-    a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
     ela::PointArgs<T> S = make_points<T>(h, sp, w.p0, src_tr, false, 0);
-    for (int c = 0; c < 3; ++c) { S.accl[c] = VL + c * np; S.accr[c] = VR + c * np; }
-    S.accfl = a.accfl; S.accfr = a.accfr;
     set_time(S, (int)k, f[it2 - 1], f[hh + it2 - 1]);
-    CHK((step_with_points<T, ela::MODE_FWD, ela::F_ACC, 0>(h, a, sp, S)));
+    const int role = pair_role(it2, sub);
+    if (role == 0) {
+      CHK((step_with_points<T, ela::MODE_FWD, 0, 0>(h, a, sp, S)));
+    } else {
+      a.accl = VL;
+      a.accr = VR;
+      a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
+      a.pair = role == 2;
+      if (a.pair) { a.acc2l = T(f[it2 - 2]); a.acc2r = T(f[hh + it2 - 2]); }
+      if (first) a.accfirst = 2;
+      first = false;
+      for (int c = 0; c < 3; ++c) { S.accl[c] = VL + c * np; S.accr[c] = VR + c * np; }
+      S.accfl = a.accfl; S.accfr = a.accfr;
+      CHK((step_with_points<T, ela::MODE_FWD, ela::F_ACC, 0>(h, a, sp, S)));
+    }
     w.swap();
   }
   return ELA_OK;
@@ -1152,7 +1171,6 @@ int born_forward_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
 
   int64_t next = 0;  // next scattered coarse step
   for (int64_t k = 0; k <= nts - 2; ++k) {
-    if (k >= 3) CHK(fill<T>(h, V(k + 1), 3 * np));  // reuse the slice of V[k-3]
     CHK(bg_coarse_step<T>(h, bg, sp, src_tr, k, V(k), V(k + 1)));
     // V[0..k] are final (all of V once k == nts-2)
     while (next <= nts - 2 && (next + 2 <= k || k == nts - 2)) CHK(scattered_step(next++));
@@ -1225,7 +1243,6 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
       HIPCHK(hipMemcpyAsync(c + 18 * np, rot[k0 % 2], 3 * np * sizeof(T), hipMemcpyDeviceToDevice, h->stream));
       for (int64_t k = k0; k < k1; ++k) {
         CHK(bg_coarse_step<T>(h, bg, sp, src_tr, k, rot[k % 2], rot[(k + 1) % 2]));
-        CHK(fill<T>(h, rot[k % 2], 3 * np));
       }
     }
     // the partial V[kl] (in rot[kl % 2]) to slot 0, the slots of V[kl + 1 .. nts - 1] cleared
@@ -1241,23 +1258,32 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
   CHK(fill<T>(h, h->wave2.p, 36 * np));
   CHK(fill<T>(h, h->ss.p, 18 * np));
   auto adjoint_step = [&](int64_t its) -> int {
+    bool first = true;   // ssL holds nothing of this coarse sample yet
     for (int64_t it2 = sub - 1; it2 >= 0; --it2) {
       ela::StepArgs<T> a = base_args<T>(h, ad.p0, ad.p1);
       set_pm<T>(h, a, ad);
-      a.accl = ssL[0];
-      a.accr = ssR[0];
-      a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
       ela::PointArgs<T> R = make_points<T>(h, rp, ad.p0, TmViews<T>(tm).v, true, nrec_tot);
       set_pm<T>(h, R, ad);
-      for (int k = 0; k < 9; ++k) { R.accl[k] = ssL[k]; R.accr[k] = ssR[k]; }
-      R.accfl = a.accfl; R.accfr = a.accfr;
       set_time(R, (int)its, f[it2 + 1], f[hh + it2 + 1]);
-      CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_ACC, ela::F_ACC>(h, a, rp, R)));
+      const int role = pair_role(sub - it2, sub);
+      if (role == 0) {
+        CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, a, rp, R)));
+      } else {
+        a.accl = ssL[0];
+        a.accr = ssR[0];
+        a.accfl = T(f[it2]); a.accfr = T(f[hh + it2]);
+        a.pair = role == 2;
+        if (a.pair) { a.acc2l = T(f[it2 + 2]); a.acc2r = T(f[hh + it2 + 2]); }
+        if (first) a.accfirst = 1;
+        first = false;
+        for (int k = 0; k < 9; ++k) { R.accl[k] = ssL[k]; R.accr[k] = ssR[k]; }
+        R.accfl = a.accfl; R.accfr = a.accfr;
+        CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_ACC, ela::F_ACC>(h, a, rp, R)));
+      }
       ad.swap();
     }
     launch_imaging<T, true>(h, imaging_args<T>(h, V(its), V(its + 1), V(its + 2), its + 1, nullptr, dm, ssR));
     for (int k = 0; k < 9; ++k) std::swap(ssL[k], ssR[k]);
-    for (int k = 0; k < 9; ++k) CHK(fill<T>(h, ssL[k], np));
     steps += sub;
     return ELA_OK;
   };
@@ -1416,6 +1442,18 @@ void set_drv(const ela_handle* h, ela::StepArgs<T>& a, DrvSlot d, bool store) {
     a.dst = reinterpret_cast<T*>(d.p);
   } else {
     a.drv = reinterpret_cast<const T*>(d.p);
+  }
+}
+
+// The derivative combinations of the level a paired imaging step replaces.
+template <typename T>
+void set_drv_pair(const ela_handle* h, ela::StepArgs<T>& a, DrvSlot d) {
+  a.pair = 1;
+  if (d.fmt == ELA_CK_S16) {
+    a.dq16b = reinterpret_cast<const int16_t*>(d.p);
+    a.dqsb = reinterpret_cast<const float*>(d.p + (size_t)9 * h->stride * 2);
+  } else {
+    a.drv2 = reinterpret_cast<const T*>(d.p);
   }
 }
 
@@ -1823,20 +1861,14 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   int64_t steps = 0;
 
   // adjoint step k (host index), or the step the device counter names (graph replays)
-  auto adj_step = [&](Wave<T>& av, int64_t k, DrvSlot d, DevStep ds) -> int {
+  // role: which levels the step images (pair_role), d2 the derivative
+  // combinations of the one it replaces
+  auto adj_step = [&](Wave<T>& av, int64_t k, DrvSlot d, DrvSlot d2, int role, DevStep ds) -> int {
     const int its = (int)(k / sub), i2 = (int)(k % sub);
     ela::StepArgs<T> a = base_args<T>(h, av.p0, av.p1);
     set_pm<T>(h, a, av);
-    set_drv<T>(h, a, d, false);
-    a.grad = g32;
-    constexpr int FQ = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
     ela::PointArgs<T> R = make_points<T>(h, rp, av.p0, TmViews<T>(tm_adj).v, true, nrec_tot);
     set_pm<T>(h, R, av);
-    for (int c = 0; c < 9; ++c) {
-      if (a.drv) R.drv[c] = a.drv + c * np;
-      if (a.dq16) { R.dq16[c] = a.dq16 + c * np; R.dqs[c] = a.dqs + c * (np / ela::DQ_BLOCK); }
-    }
-    for (int m = 0; m < 8; ++m) R.grad[m] = g32 + m * np;
     // the level step k reads, which step k + 1 left (none before the first)
     ela::PointArgs<T> S = make_points<T>(h, sp, av.p1, TmViews<T>(tm_src).v, true, nsrc_tot);
     if (ds.k) { set_step(h, R, ds.k, ds.off, 1); set_step(h, S, ds.k, ds.off + 1, 0); }
@@ -1845,8 +1877,21 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
     const int64_t kr = std::min(k + 1, N - 1), ir = kr % sub;
     set_time(S, (int)(kr / sub), f[ir], f[hh + ir]);
     if (!ds.k && k == N - 1) S.off[9] = 0;
-    if (d.fmt == ELA_CK_S16) CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, FQ, FQ>(h, a, rp, R, S)));
-    else CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, a, rp, R, S)));
+    if (role == 0) {
+      CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, a, rp, R, S)));
+    } else {
+      set_drv<T>(h, a, d, false);
+      if (role == 2) set_drv_pair<T>(h, a, d2);
+      a.grad = g32;
+      for (int c = 0; c < 9; ++c) {
+        if (a.drv) R.drv[c] = a.drv + c * np;
+        if (a.dq16) { R.dq16[c] = a.dq16 + c * np; R.dqs[c] = a.dqs + c * (np / ela::DQ_BLOCK); }
+      }
+      for (int m = 0; m < 8; ++m) R.grad[m] = g32 + m * np;
+      constexpr int FQ = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
+      if (d.fmt == ELA_CK_S16) CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, FQ, FQ>(h, a, rp, R, S)));
+      else CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, a, rp, R, S)));
+    }
     if (ds.advance) launch(h, ela::k_count, dim3(1), dim3(64), ds.k, ds.advance);
     av.swap();
     return ELA_OK;
@@ -1884,7 +1929,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
         auto adj_seg = [&]() -> int {
           Wave<T> wl = ad;
           for (int64_t kk = plan.K - 1; kk >= 0; --kk)
-            CHK(adj_step(wl, 0, drv(kk), DevStep{kst, (int)kk, 0}));
+            CHK(adj_step(wl, 0, drv(kk), drv(kk + 2), pair_role(plan.K - kk, plan.K), DevStep{kst, (int)kk, 0}));
           return ELA_OK;
         };
         hipGraphExec_t ex = nullptr;
@@ -1896,7 +1941,8 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
       } else {
         for (int64_t k = j0; k < j1; ++k)
           CHK((grad_fwd_step<T, true>(h, bg, sp, src_tr, k, drv(k - j0))));
-        for (int64_t k = j1 - 1; k >= j0; --k) CHK(adj_step(ad, k, drv(k - j0), DevStep()));
+        for (int64_t k = j1 - 1; k >= j0; --k)
+          CHK(adj_step(ad, k, drv(k - j0), drv(k - j0 + 2), pair_role(j1 - k, j1 - j0), DevStep()));
       }
       steps += 2 * (j1 - j0);
       CHK(fold_gradient<T>(h, g32, g64));
@@ -1973,24 +2019,30 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   g.grad = (T*)h->g32.p;
   constexpr int FQS = sizeof(T) == 4 ? ela::F_STORE | ela::F_Q16 : ela::F_STORE;
   constexpr int FQG = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
+  set_drv_pair<T>(h, g, slot);
+  // half of the transposed steps image (two levels each), half do not
+  bool image = false;
   auto step = [&](int which) -> int {
+    image = !image;
     if (which == 0) return launch_step_m<T, ela::MODE_FWD, 0, 0>(h, f);
     if (which == 1) {
       if (dfmt == ELA_CK_S16) return launch_step_m<T, ela::MODE_FWD, FQS, FQS>(h, r);
       return launch_step_m<T, ela::MODE_FWD, ela::F_STORE, ela::F_STORE>(h, r);
     }
+    if (!image) return launch_step_m<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, g);
     if (dfmt == ELA_CK_S16) return launch_step_m<T, ela::MODE_BORN_ADJ_PM, FQG, FQG>(h, g);
     return launch_step_m<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, g);
   };
   for (int k = 0; k < 3; ++k) {
     CHK(step(k));  // warm caches and code
     HIPCHK(hipEventRecord(h->ev0, h->stream));
-    for (int i = 0; i < reps; ++i) CHK(step(k));
+    const int n = k == 2 ? reps + reps % 2 : reps;   // as many imaging as other transposed steps
+    for (int i = 0; i < n; ++i) CHK(step(k));
     HIPCHK(hipEventRecord(h->ev1, h->stream));
     HIPCHK(hipEventSynchronize(h->ev1));
     float t = 0.f;
     HIPCHK(hipEventElapsedTime(&t, h->ev0, h->ev1));
-    ms3[k] = t / reps;
+    ms3[k] = t / n;
   }
   HIPCHK(hipGetLastError());
   return ELA_OK;

@@ -45,6 +45,15 @@ enum { MODE_FWD = 0,       // n = w(w o + M D c)        stepFwdGpu_3D
 };
 
 // Optional work fused into a stepper launch (bit flags).
+//
+// F_ACC and F_GRAD read and rewrite up to 18 and 8 arrays for values the step
+// has in registers anyway: the new level n+1 and, in o, the level n-1 it
+// replaces. So they run in every other step only and take both levels (pair;
+// the schedule is pair_role), which halves that traffic:
+//   Born transposed step: 75 -> 57 arrays a step on average (Born adjoint of
+//   232x328x324, 40 steps: 105 -> 80 ms, the clearing of the targets gone too),
+//   gradient transposed step: 64 -> 56 arrays (gradient of 232x328x324, 40
+//   steps: 110 -> 108 ms).
 enum { F_SS = 1,     // add the secondary sources ssl/ssr (Born forward)
        F_ACC = 2,    // accumulate the new level into accl/accr (coarse-time interpolation)
        F_STORE = 4,  // write the step's derivative combinations to dst (gradient recomputation)
@@ -89,6 +98,12 @@ struct StepArgs {
   double tdt64;         // F_MED3: 2 dtw in FP64 (FP32 steppers form buoyancies and normal moduli in FP64)
   T ssfl, ssfr;         // filter weights for the secondary source
   T accfl, accfr;       // filter weights for the accumulation
+  T acc2l, acc2r;       // F_ACC with pair: those of the level in o
+  const T* drv2;        // F_GRAD with pair: the derivative combinations of the level in o
+  const int16_t* dq16b; // F_GRAD | F_Q16 with pair: the same as int16
+  const float* dqsb;
+  int pair;             // accumulate / image the level in o (n-1, complete) as well as the new one
+  int accfirst;         // F_ACC: the left (1) or right (2) target holds nothing yet: written, not read
   T cx[4], cy[4], cz[4];
   const T* taper;       // [min_pad]
   int min_pad;
@@ -813,18 +828,28 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
       // used, which holds fewer registers (2 waves per SIMD)
       T o3[3], m3[3], ss3[3], al3[3], ar3[3], g3[3], d3[3];
       auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
+      auto load_acc = [&](int f) {
+        al3[f] = a.accfirst == 1 ? T(0) : *at(fam(a.accl, f, np), i);
+        ar3[f] = a.accfirst == 2 ? T(0) : *at(fam(a.accr, f, np), i);
+        if (a.pair) { al3[f] += o3[f] * a.acc2l; ar3[f] += o3[f] * a.acc2r; }
+      };
+      auto load_grad = [&](int f) {  // BX_/BY_/BZ_ == VX/VY/VZ
+        g3[f] = *at(fam(a.grad, f, np), i);
+        if constexpr (Q16) d3[f] = load_dq16(fam(a.dq16, f, np), fam(a.dqs, f, np / DQ_BLOCK), i);
+        else d3[f] = ld_nt(fam(a.drv, f, np), i);
+        if (a.pair) {
+          if constexpr (Q16) g3[f] += o3[f] * load_dq16(fam(a.dq16b, f, np), fam(a.dqsb, f, np / DQ_BLOCK), i);
+          else g3[f] += o3[f] * ld_nt(fam(a.drv2, f, np), i);
+        }
+      };
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
         o3[f] = ld_nt(fam(a.o, f, np), i);
         if (!MED3 && MODE != MODE_BORN_ADJ) m3[f] = ld_nt(fam(a.m, f, np), i);
         if constexpr (HOIST) {
           if (SS) ss3[f] = load_ss(f);
-          if (ACC) { al3[f] = *at(fam(a.accl, f, np), i); ar3[f] = *at(fam(a.accr, f, np), i); }
-          if (F & F_GRAD) {  // BX_/BY_/BZ_ == VX/VY/VZ
-            g3[f] = *at(fam(a.grad, f, np), i);
-            if constexpr (Q16) d3[f] = load_dq16(fam(a.dq16, f, np), fam(a.dqs, f, np / DQ_BLOCK), i);
-            else d3[f] = ld_nt(fam(a.drv, f, np), i);
-          }
+          if (ACC) load_acc(f);
+          if (F & F_GRAD) load_grad(f);
         }
       }
       if (MED3) {
@@ -854,8 +879,8 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
         else u = w * o3[f] - s3[f];
         if constexpr (!HOIST) {
           if (SS) ss3[f] = load_ss(f);
-          if (ACC) { al3[f] = *at(fam(a.accl, f, np), i); ar3[f] = *at(fam(a.accr, f, np), i); }
-          if (F & F_GRAD) { g3[f] = *at(fam(a.grad, f, np), i); d3[f] = ld_nt(fam(a.drv, f, np), i); }
+          if (ACC) load_acc(f);
+          if (F & F_GRAD) load_grad(f);
         }
         if (SS) u += ss3[f];
         u *= w;
@@ -1018,21 +1043,47 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
       // FP32: every per-cell operand is loaded before the first store (see velocity_block)
       T o6[6], ss6[6], al6[6], ar6[6], g5[5], d6[6];
       auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
+      auto load_acc = [&](int k) {
+        const int f = SXX + k;
+        al6[k] = a.accfirst == 1 ? T(0) : *at(fam(a.accl, f, np), i);
+        ar6[k] = a.accfirst == 2 ? T(0) : *at(fam(a.accr, f, np), i);
+        if (a.pair) { al6[k] += o6[k] * a.acc2l; ar6[k] += o6[k] * a.acc2r; }
+      };
+      // g5 += the image of level v with the derivative combinations d:
+      // lamb2MuDtw multiplies exx, eyy, ezz in sxx, syy, szz; lambDtw the
+      // other two normal strains; the shear moduli one shear strain each
+      auto image = [&](const T* v, const T* d) {
+        const T l2 = v[0] * d[0] + v[1] * d[1] + v[2] * d[2];
+        g5[0] += l2;
+        g5[1] += (v[0] + v[1] + v[2]) * (d[0] + d[1] + d[2]) - l2;
+        g5[2] += v[3] * d[3];
+        g5[3] += v[4] * d[4];
+        g5[4] += v[5] * d[5];
+      };
       auto load_grad = [&]() {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) g5[m] = *at(fam(a.grad, L2M + m, np), i);
+        if (a.pair) {
+          T e6[6];
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            if constexpr (Q16) e6[k] = load_dq16(fam(a.dq16b, SXX + k, np), fam(a.dqsb, SXX + k, np / DQ_BLOCK), i);
+            else e6[k] = ld_nt(fam(a.drv2, SXX + k, np), i);
+          }
+          image(o6, e6);
+        }
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
           if constexpr (Q16) d6[k] = load_dq16(fam(a.dq16, SXX + k, np), fam(a.dqs, SXX + k, np / DQ_BLOCK), i);
           else d6[k] = ld_nt(fam(a.drv, SXX + k, np), i);
         }
-#pragma unroll
-        for (int m = 0; m < 5; ++m) g5[m] = *at(fam(a.grad, L2M + m, np), i);
       };
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
         o6[k] = ld_nt(fam(a.o, SXX + k, np), i);
         if constexpr (HOIST) {
           if (SS) ss6[k] = load_ss(SXX + k);
-          if (ACC) { al6[k] = *at(fam(a.accl, SXX + k, np), i); ar6[k] = *at(fam(a.accr, SXX + k, np), i); }
+          if (ACC) load_acc(k);
         }
       }
       if constexpr (HOIST && (F & F_GRAD) != 0) load_grad();
@@ -1092,7 +1143,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         const int f = SXX + k;
         if constexpr (!HOIST) {
           if (SS) ss6[k] = load_ss(f);
-          if (ACC) { al6[k] = *at(fam(a.accl, f, np), i); ar6[k] = *at(fam(a.accr, f, np), i); }
+          if (ACC) load_acc(k);
         }
         T v = u[k];
         if (SS) v += ss6[k];
@@ -1114,16 +1165,10 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         st_nt(fam(a.qn, SYZ, np), i, u[5] * myz);
       }
       if (F & F_GRAD) {
-        // lamb2MuDtw multiplies exx, eyy, ezz in sxx, syy, szz; lambDtw the
-        // other two normal strains; the shear moduli one shear strain each
         if constexpr (!HOIST) load_grad();
-        const T dxx = d6[0], dyy = d6[1], dzz = d6[2];
-        const T l2 = u[0] * dxx + u[1] * dyy + u[2] * dzz;
-        *at(fam(a.grad, L2M, np), i) = g5[0] + l2;
-        *at(fam(a.grad, LAM, np), i) = g5[1] + ((u[0] + u[1] + u[2]) * (dxx + dyy + dzz) - l2);
-        *at(fam(a.grad, MXZ, np), i) = g5[2] + u[3] * d6[3];
-        *at(fam(a.grad, MXY, np), i) = g5[3] + u[4] * d6[4];
-        *at(fam(a.grad, MYZ, np), i) = g5[4] + u[5] * d6[5];
+        image(u, d6);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) *at(fam(a.grad, L2M + m, np), i) = g5[m];
       }
     }
 #pragma unroll

@@ -404,8 +404,8 @@ int ela_time_step_kernels(ela_handle* h, int reps, double* ms_velocity, double* 
 /* Mean milliseconds of the three kernel pairs of an adjoint-state gradient
  * step on the handle's grid and launch shape, over `reps` launches each:
  * ms3[0] the forward step, ms3[1] the recomputing step with derivative store
- * (in the handle's derivative format), ms3[2] the transposed step with
- * imaging. Overwrites the wavefields and allocates the gradient's step
+ * (in the handle's derivative format), ms3[2] the transposed step (the mean of
+ * one that images two levels and one that images none, which alternate). Overwrites the wavefields and allocates the gradient's step
  * buffers (kept, as after a gradient; the Born adjoint's automatic storage
  * plan counts them as free and releases them); stored checkpoints are kept.
  * For the launch-shape tuner of the gradient. No counterpart in the

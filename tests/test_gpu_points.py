@@ -33,6 +33,7 @@ def make_prop(g, precision):
 # points per list: 9 (few, one box), 56 (504 over the 9 components: still in the blocks), 57 (513: separate launch)
 @pytest.mark.parametrize("n", [9, 56, 57])
 @pytest.mark.parametrize("precision,nts,sub,graph", [("f64", 2, 1, False), ("f64", 3, 3, False), ("f64", 4, 2, True),
+                                                     ("f64", 3, 6, False), ("f64", 3, 7, False),
                                                      ("f32", 3, 4, True), ("f32", 3, 2, False)])
 def test_points_in_the_steps_blocks(n, precision, nts, sub, graph):
     g = grid(nts, sub)
