@@ -196,6 +196,7 @@ struct ela_handle {
   std::vector<double> filt; // 2*(sub+1)
   int64_t last_steps = 0;
   int by_x = 4;             // x extent of a tile (initial launch shape: initial_shape)
+  bool narrow = false;      // 256-thread blocks are narrow tiles (narrow_tiles)
   int by_x_t = 0;           // x extent of the premultiplied transposed steps' tiles (0: by_x)
   int ychunk = 8;           // y planes per block
   int remap = 3;            // tile order (ela_set_tile_order)
@@ -396,10 +397,11 @@ int ensure_chunks(ela_handle* h) {
   return ELA_OK;
 }
 
-Tiles tiles_for(const ela_handle* h, int bx, int ychunk) {
+Tiles tiles_for(const ela_handle* h, int shape, int ychunk) {
   Tiles t;
   const int64_t iz = h->cfg.nz - 2 * ela::FAT, ix = h->cfg.nx - 2 * ela::FAT, iy = h->cfg.ny - 2 * ela::FAT;
-  t.nbz = (int)((iz + ela::TZ - 1) / ela::TZ);
+  const int bz = ela::tile_z(shape), bx = ela::tile_x(shape);
+  t.nbz = (int)((iz + bz - 1) / bz);
   t.nbx = (int)((ix + bx - 1) / bx);
   t.nby = h->win_y0.empty() ? (int)((iy + ychunk - 1) / ychunk) : h->nchunks;
   t.nblocks = t.nbz * t.nbx * t.nby;
@@ -421,9 +423,27 @@ Tiles tiles_for(const ela_handle* h, int bx, int ychunk) {
 // ones): 72x72x72 18.6 us a step with 8 planes, 15.5 with 2; 40x36x44 15.8
 // -> 10.8. 7/8 of the residency counts as full: 88x97x90 (1012 blocks of 1024)
 // 28.8 us with 8 planes, 29.4 with 4; a march of 1 gains nothing over 2.
+// Whether 256-thread blocks are narrow tiles (32 z x 8 x cells) instead of
+// wide ones (64 x 4). FP64: always; the 8 rows share their x halo (2 rows read
+// per row owned instead of 3) and the planes take 3/4 of the LDS: forward step
+// 152x152x148 219 -> 188 us, 232x328x324 1490 -> 1300, 328x472x468 (z extent
+// 320, no padding either way) 4050 -> 3860. FP32: where 32-cell tiles leave
+// fewer lanes idle past the last z cell: 232x328x324 (224 cells) 634 -> 596
+// us, 201x187x143 (193) 149 -> 145, 152x152x148 (144) 92 -> 91; with equal
+// padding the second row's loads and the z halo per 32 cells cost more than
+// the x halo saves: 110x93x121 37.5 -> 39.5, 72x72x72 12.3 -> 14.1.
+bool narrow_tiles(int esize, int64_t iz) {
+  return esize == 8 || (iz + 31) / 32 * 32 < (iz + 63) / 64 * 64;
+}
+
+// Tile shape for an x tile set by ela_set_tiling.
+int shape_of(const ela_handle* h, int bx) { return bx == 4 && h->narrow ? ela::TILE_NARROW : bx; }
+
 void initial_shape(ela_handle* h) {
   const int64_t iz = h->cfg.nz - 2 * ela::FAT, ix = h->cfg.nx - 2 * ela::FAT, iy = h->cfg.ny - 2 * ela::FAT;
-  const int64_t cols = ((iz + ela::TZ - 1) / ela::TZ) * ((ix + h->by_x - 1) / h->by_x);
+  h->narrow = narrow_tiles(h->esize, iz);
+  const int bz = ela::tile_z(shape_of(h, h->by_x)), bx = ela::tile_x(shape_of(h, h->by_x));
+  const int64_t cols = ((iz + bz - 1) / bz) * ((ix + bx - 1) / bx);
   const int64_t resident = 256 * (h->esize == 4 ? 4 : 2);
   const int planes[] = {8, 6, 4, 3, 2};
   for (int yc : planes) {
@@ -463,17 +483,17 @@ ela::StepArgs<T> base_args(ela_handle* h, T* o[9], T* c[9]) {
 
 // which: bit 0 = velocity blocks, bit 1 = stress blocks; FV / FS: the
 // ela::F_* work fused into them.
-template <typename T, int BX, int MODE, int FV, int FS>
-int launch_step_bx(ela_handle* h, ela::StepArgs<T> a, int which, const ela::PointArgs<T>& inj,
+template <typename T, int S, int MODE, int FV, int FS>
+int launch_step_s(ela_handle* h, ela::StepArgs<T> a, int which, const ela::PointArgs<T>& inj,
                    const ela::PointArgs<T>& rec) {
-  Tiles t = tiles_for(h, BX, a.ychunk);
+  Tiles t = tiles_for(h, S, a.ychunk);
   a.nbz = t.nbz; a.nbx = t.nbx; a.nby = t.nby;
-  dim3 block(ela::TZ, BX);
+  dim3 block(ela::WAVE, ela::tile_threads(S) / ela::WAVE);
   a.first = which & 1 ? 0 : t.nblocks;
   // recording blocks follow the stress blocks (a recorded step runs both halves)
-  const unsigned nrec = (unsigned)((rec.off[9] + ela::TZ * BX - 1) / (ela::TZ * BX));
+  const unsigned nrec = (unsigned)((rec.off[9] + ela::tile_threads(S) - 1) / ela::tile_threads(S));
   const unsigned nb = (unsigned)(which == 3 ? 2 * t.nblocks : t.nblocks);
-  launch(h, ela::k_step<T, BX, MODE, FV, FS>, dim3(nb + nrec), block, a, inj, rec);
+  launch(h, ela::k_step<T, S, MODE, FV, FS>, dim3(nb + nrec), block, a, inj, rec);
   return ELA_OK;
 }
 
@@ -486,11 +506,14 @@ int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::
   // FP64 and the steps with per-cell extra operands spill there (Born adjoint
   // of 232x328x324 69-97 ms with 16 rows, 60 with 4) and run 4 rows instead
   constexpr bool wide = sizeof(T) == 4 && ((FV | FS) & (ela::F_SS | ela::F_ACC | ela::F_GRAD)) == 0;
-  if (bx == 8) return launch_step_bx<T, 8, MODE, FV, FS>(h, a, which, inj, rec);
+  if (bx == 8) return launch_step_s<T, 8, MODE, FV, FS>(h, a, which, inj, rec);
   if constexpr (wide) {
-    if (bx == 16) return launch_step_bx<T, 16, MODE, FV, FS>(h, a, which, inj, rec);
+    if (bx == 16) return launch_step_s<T, 16, MODE, FV, FS>(h, a, which, inj, rec);
   }
-  return launch_step_bx<T, 4, MODE, FV, FS>(h, a, which, inj, rec);
+  if constexpr (sizeof(T) == 4) {
+    if (!h->narrow) return launch_step_s<T, 4, MODE, FV, FS>(h, a, which, inj, rec);
+  }
+  return launch_step_s<T, ela::TILE_NARROW, MODE, FV, FS>(h, a, which, inj, rec);
 }
 
 // Forward, nonlinear-adjoint and premultiplied transposed steps form the
@@ -572,7 +595,9 @@ bool fuse_injection(const ela_handle* h, const DevPoints& p, const int* box) {
   const int64_t n = total_points(p);
   if (n == 0 || n > kFusePoints) return false;
   const auto tiles = [](int lo_top, int hi, int64_t tile) { return (int64_t)(hi - (ela::POS_TOP - lo_top)) / tile + 2; };
-  return tiles(box[0], box[1], ela::TZ) * tiles(box[2], box[3], h->by_x) * tiles(box[4], box[5], h->ychunk) <= 1024;
+  const int S = shape_of(h, h->by_x);
+  return tiles(box[0], box[1], ela::tile_z(S)) * tiles(box[2], box[3], ela::tile_x(S)) *
+             tiles(box[4], box[5], h->ychunk) <= 1024;
 }
 
 // Copies (host) or reads (device) the caller's int64 positions, converts them

@@ -14,8 +14,8 @@
 //   the swap is the previous level damped a second time.
 //
 // Mapping to the CDNA4 execution model:
-//   - a block is 64 (z, one wave row, coalesced) x BX (x) threads and owns a
-//     64 x BX column tile that it marches along y over a chunk of planes;
+//   - a block owns a tile of 64 (z, one wave, coalesced) x 4, 8 or 16 (x)
+//     cells, or of 32 x 8, which it marches along y over a chunk of planes;
 //   - fields needing x or z derivatives are staged per plane in LDS with a
 //     4-cell halo; y derivatives come from an 8-deep register queue per
 //     thread, so each plane of each field is read from HBM once per tile;
@@ -31,7 +31,18 @@
 namespace ela {
 
 constexpr int FAT = 4;
-constexpr int TZ = 64;       // z extent of a tile = one wavefront
+constexpr int WAVE = 64;
+constexpr int TZ = 64;       // z extent of the wide tiles = one wavefront
+
+// Tile shapes S: 4, 8 and 16 are wide tiles of 64 (z) x S (x) cells, a wave
+// covering one x row; TILE_NARROW is 32 x 8 cells, a wave covering two x rows
+// of 32 (one 128-byte FP32 line each). Which grids
+// take them, and what it measured, stands at narrow_tiles.
+constexpr int TILE_NARROW = 32 + 8;
+constexpr int tile_z(int S) { return S == TILE_NARROW ? 32 : TZ; }
+constexpr int tile_x(int S) { return S == TILE_NARROW ? 8 : S; }
+constexpr int tile_threads(int S) { return tile_z(S) * tile_x(S); }
+constexpr int wave_rows(int S) { return WAVE / tile_z(S); }   // x rows per wave
 constexpr int NXCD = 8;      // MI355X: 8 XCDs, blocks dealt round-robin
 
 enum { VX = 0, VY, VZ, SXX, SYY, SZZ, SXZ, SXY, SYZ };
@@ -166,27 +177,27 @@ __device__ __forceinline__ T dq(const T* q, const T* c) {
 }
 
 // LDS plane with a 4-cell halo on both sides in x (rows) and z (columns).
-template <typename T, int BX>
-using Plane = T[BX + 2 * FAT][TZ + 2 * FAT];
+template <typename T, int S>
+using Plane = T[tile_x(S) + 2 * FAT][tile_z(S) + 2 * FAT];
 
 // D+ / D- along z (columns) and x (rows) of an LDS plane, at (r, col) = (ty+4, tz+4).
-template <typename T, int BX>
-__device__ __forceinline__ T dpz(const Plane<T, BX>& p, int r, int q, const T* c) {
+template <typename T, int S>
+__device__ __forceinline__ T dpz(const Plane<T, S>& p, int r, int q, const T* c) {
   return c[0] * (p[r][q + 1] - p[r][q]) + c[1] * (p[r][q + 2] - p[r][q - 1]) +
          c[2] * (p[r][q + 3] - p[r][q - 2]) + c[3] * (p[r][q + 4] - p[r][q - 3]);
 }
-template <typename T, int BX>
-__device__ __forceinline__ T dmz(const Plane<T, BX>& p, int r, int q, const T* c) {
+template <typename T, int S>
+__device__ __forceinline__ T dmz(const Plane<T, S>& p, int r, int q, const T* c) {
   return c[0] * (p[r][q] - p[r][q - 1]) + c[1] * (p[r][q + 1] - p[r][q - 2]) +
          c[2] * (p[r][q + 2] - p[r][q - 3]) + c[3] * (p[r][q + 3] - p[r][q - 4]);
 }
-template <typename T, int BX>
-__device__ __forceinline__ T dpx(const Plane<T, BX>& p, int r, int q, const T* c) {
+template <typename T, int S>
+__device__ __forceinline__ T dpx(const Plane<T, S>& p, int r, int q, const T* c) {
   return c[0] * (p[r + 1][q] - p[r][q]) + c[1] * (p[r + 2][q] - p[r - 1][q]) +
          c[2] * (p[r + 3][q] - p[r - 2][q]) + c[3] * (p[r + 4][q] - p[r - 3][q]);
 }
-template <typename T, int BX>
-__device__ __forceinline__ T dmx(const Plane<T, BX>& p, int r, int q, const T* c) {
+template <typename T, int S>
+__device__ __forceinline__ T dmx(const Plane<T, S>& p, int r, int q, const T* c) {
   return c[0] * (p[r][q] - p[r - 1][q]) + c[1] * (p[r + 1][q] - p[r - 2][q]) +
          c[2] * (p[r + 2][q] - p[r - 3][q]) + c[3] * (p[r + 3][q] - p[r - 4][q]);
 }
@@ -245,6 +256,27 @@ __device__ __forceinline__ void st_nt(T* base, uint32_t i, T v) {
 // precedes the block's next barrier.
 __device__ __forceinline__ void row_to_lds(const float* base, uint32_t i, float* row) {
   __builtin_amdgcn_global_load_lds(at(base, i), (__attribute__((address_space(3))) void*)row, 4, 0, 0);
+}
+
+// The rows of a tile plane that a wave loads: plane[row][col ...] and, of a
+// narrow tile, plane[row + 1][col ...] by the upper half of the lanes (lane l
+// writes 4 l bytes past the row given, hence the shift by half a wave). The
+// two comments in the assembly keep the compiler from merging the branches
+// into one load whose LDS row, a wave-uniform operand, would be the lower
+// half's for every lane.
+template <int S, typename P>
+__device__ __forceinline__ void rows_to_lds(const float* base, uint32_t i, P& plane, int row, int col) {
+  if constexpr (wave_rows(S) == 1) {
+    row_to_lds(base, i, &plane[row][col]);
+  } else {
+    if (threadIdx.x < WAVE / 2) {
+      row_to_lds(base, i, &plane[row][col]);
+      asm volatile("; lower lanes");
+    } else {
+      row_to_lds(base, i, &plane[row + 1][col] - WAVE / 2);
+      asm volatile("; upper lanes");
+    }
+  }
 }
 
 // Largest magnitude over each 32-lane half of the wave (one DQ_BLOCK), in
@@ -363,9 +395,10 @@ struct TileCoord {
 // columns (`xgroup` adjacent columns of nbz tiles), so that z (and, with
 // xgroup > 1, x) neighbours share an L2 while the grid is swept in the
 // hardware order.
-template <int BX>
+template <int S>
 __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int nby, int ychunk, int nz, int nzi,
                                                 int zoff, int nx, int ny, int order, int xgroup, const int* chunks) {
+  constexpr int BX = tile_x(S), BZ = tile_z(S);
   const int nb = nbz * nbx * nby;
   const int lb = order == 3 ? xcd_group(bid, nb, nbz * xgroup) : order ? xcd_remap(bid, nb) : bid;
   int bz, bx, by;
@@ -384,9 +417,9 @@ __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int n
     by = lb / (nbz * nbx);
   }
   TileCoord t;
-  t.tz = threadIdx.x;
-  t.ty = threadIdx.y;
-  t.z0 = zoff + FAT + bz * TZ;
+  t.tz = wave_rows(S) == 1 ? threadIdx.x : threadIdx.x % BZ;
+  t.ty = wave_rows(S) == 1 ? threadIdx.y : threadIdx.y * wave_rows(S) + threadIdx.x / BZ;
+  t.z0 = zoff + FAT + bz * BZ;
   t.x0 = FAT + bx * BX;
   t.iz = t.z0 + t.tz;
   t.izo = t.iz - zoff;
@@ -409,8 +442,8 @@ __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int n
   t.okxl = t.xh && t.izo < nz;
   t.okxh = t.okxl && ixhi < nx;
   t.zh = t.tz < 2 * FAT;
-  const int izh = t.tz < FAT ? t.z0 - FAT + t.tz : t.z0 + TZ + (t.tz - FAT);
-  t.colh = t.tz < FAT ? t.tz : TZ + t.tz;
+  const int izh = t.tz < FAT ? t.z0 - FAT + t.tz : t.z0 + BZ + (t.tz - FAT);
+  t.colh = t.tz < FAT ? t.tz : BZ + t.tz;
   t.okzh = t.zh && (izh - zoff) < nz && t.ix < nx;
   // Lanes past the last z cell and rows past the last x row read the last
   // one: no interior stencil uses their values, and without the clamp they
@@ -612,7 +645,7 @@ constexpr int POS_TOP = 1 << 30;
 // trace back, and the tile worked out again from the block index: kept live
 // across the march they cost scalar registers, whose spills take vector
 // registers (130 instead of 128, i.e. 3 waves per SIMD, in some steps).
-template <typename T, int BX, bool ACC, bool GRAD, bool PM>
+template <typename T, int S, bool ACC, bool GRAD, bool PM>
 __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
 #define ELA_KERNARG __attribute__((address_space(4)))
   uint64_t seg = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
@@ -622,13 +655,14 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
 #undef ELA_KERNARG
   if (a.off[9] == 0) return;  // kernel-uniform
   const int bid = (int)blockIdx.x + s.first - half * s.nbz * s.nbx * s.nby;
-  const TileCoord t = tile_coord<BX>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
+  const TileCoord t = tile_coord<S>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
   const int* b = a.box;
-  const bool hit = POS_TOP - b[0] < t.z0 + TZ && b[1] >= t.z0 && POS_TOP - b[2] < t.x0 + BX && b[3] >= t.x0 &&
+  constexpr int BX = tile_x(S), BZ = tile_z(S);
+  const bool hit = POS_TOP - b[0] < t.z0 + BZ && b[1] >= t.z0 && POS_TOP - b[2] < t.x0 + BX && b[3] >= t.x0 &&
                    POS_TOP - b[4] < t.y1 && b[5] >= t.y0;
   if (!hit) return;  // block-uniform
   __syncthreads();
-  for (int g = (int)a.off[c0] + t.ty * TZ + t.tz; g < (int)a.off[c1]; g += TZ * BX) {
+  for (int g = (int)a.off[c0] + t.ty * BZ + t.tz; g < (int)a.off[c1]; g += BZ * BX) {
     int c = c0;
 #pragma nounroll   // one offset at a time in a scalar register
     for (int k = c0 + 1; k < c1; ++k) c += g >= (int)a.off[k] ? 1 : 0;
@@ -636,7 +670,7 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
     const int32_t p = a.pos[c][k];
     if (p < 0) continue;
     const int row = p / a.nzi, z = p - row * a.nzi, y = row / a.nx, x = row - y * a.nx;
-    if (z >= t.z0 && z < t.z0 + TZ && x >= t.x0 && x < t.x0 + BX && y >= t.y0 && y < t.y1)
+    if (z >= t.z0 && z < t.z0 + BZ && x >= t.x0 && x < t.x0 + BX && y >= t.y0 && y < t.y1)
       inject_point<T, ACC, GRAD, PM>(a, c, k);
   }
 }
@@ -651,10 +685,10 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
 // ---------------------------------------------------------------------------
 // The velocity stepper's LDS: double-buffered planes of sxx, szz, sxy, sxz,
 // syz and (F_MED3) density planes with the low x row and low z column.
-template <typename T, int BX, bool MED3>
+template <typename T, int S, bool MED3>
 struct VelLds {
-  Plane<T, BX> xx[2], zz[2], xy[2], xz[2], yz[2];
-  T rho[2][MED3 ? BX + 1 : 1][MED3 ? TZ + 1 : 1];
+  Plane<T, S> xx[2], zz[2], xy[2], xz[2], yz[2];
+  T rho[2][MED3 ? tile_x(S) + 1 : 1][MED3 ? tile_z(S) + 1 : 1];
 };
 
 template <typename T>
@@ -710,8 +744,9 @@ __device__ __forceinline__ void normal_moduli(T tdt, double tdt64, T lam, T mu, 
   }
 }
 
-template <typename T, int BX, int MODE, int F>
-__device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, VelLds<T, BX, (F & F_MED3) != 0>& L) {
+template <typename T, int S, int MODE, int F>
+__device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, VelLds<T, S, (F & F_MED3) != 0>& L) {
+  constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
@@ -721,7 +756,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
                 "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
   auto& l_xx = L.xx; auto& l_zz = L.zz; auto& l_xy = L.xy; auto& l_xz = L.xz; auto& l_yz = L.yz;
   auto& l_rho = L.rho;
-  const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   int64_t np = a.np;
@@ -731,16 +766,16 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
   auto src = [&](int f) -> const T* { return fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np); };
   const int r = t.ty + FAT, q = t.tz + FAT;
-  // a wave is one row of the tile (blockDim.x == TZ == wavefront size): its row index is wave-uniform
+  // first x row of the wave (a wide tile's wave is one row), wave-uniform
   const int wy = __builtin_amdgcn_readfirstlane(t.ty), wr = wy + FAT;
 
   // plane p's values: LDS rows of buffer nb directly (DMA), the rest into v
   auto fetch = [&](VelStage<T>& v, int p, int nb) {
     const uint32_t pl = (uint32_t)p * ys;
     if constexpr (DMA) {
-      row_to_lds(src(SXX), pl + t.col, &l_xx[nb][wr][FAT]);
-      row_to_lds(src(SZZ), pl + t.col, &l_zz[nb][wr][FAT]);
-      row_to_lds(src(SXZ), pl + t.col, &l_xz[nb][wr][FAT]);
+      rows_to_lds<S>(src(SXX), pl + t.col, l_xx[nb], wr, FAT);
+      rows_to_lds<S>(src(SZZ), pl + t.col, l_zz[nb], wr, FAT);
+      rows_to_lds<S>(src(SXZ), pl + t.col, l_xz[nb], wr, FAT);
     } else {
       v.xx = S_().sxx(pl + t.col);
       v.zz = S_().szz(pl + t.col);
@@ -751,9 +786,9 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     v.nyz = S_().syz(pl + 4 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
-        row_to_lds(src(SXX), pl + t.cxl, &l_xx[nb][wy][FAT]); row_to_lds(src(SXX), pl + t.cxh, &l_xx[nb][wr + BX][FAT]);
-        row_to_lds(src(SXY), pl + t.cxl, &l_xy[nb][wy][FAT]); row_to_lds(src(SXY), pl + t.cxh, &l_xy[nb][wr + BX][FAT]);
-        row_to_lds(src(SXZ), pl + t.cxl, &l_xz[nb][wy][FAT]); row_to_lds(src(SXZ), pl + t.cxh, &l_xz[nb][wr + BX][FAT]);
+        rows_to_lds<S>(src(SXX), pl + t.cxl, l_xx[nb], wy, FAT); rows_to_lds<S>(src(SXX), pl + t.cxh, l_xx[nb], wr + BX, FAT);
+        rows_to_lds<S>(src(SXY), pl + t.cxl, l_xy[nb], wy, FAT); rows_to_lds<S>(src(SXY), pl + t.cxh, l_xy[nb], wr + BX, FAT);
+        rows_to_lds<S>(src(SXZ), pl + t.cxl, l_xz[nb], wy, FAT); rows_to_lds<S>(src(SXZ), pl + t.cxh, l_xz[nb], wr + BX, FAT);
       } else {
         v.hxx0 = S_().sxx(pl + t.cxl); v.hxx1 = S_().sxx(pl + t.cxh);
         v.hxy0 = S_().sxy(pl + t.cxl); v.hxy1 = S_().sxy(pl + t.cxh);
@@ -766,8 +801,8 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     if (MED3) {
       // the column's own cell and its x - 1 / z - 1 neighbours
       if constexpr (DMA) {
-        row_to_lds(fam(a.ep, 0, np), pl + t.col, &l_rho[nb][wy + 1][1]);
-        if (wy == 0) row_to_lds(fam(a.ep, 0, np), pl + t.col - (uint32_t)a.nzi, &l_rho[nb][0][1]);
+        rows_to_lds<S>(fam(a.ep, 0, np), pl + t.col, l_rho[nb], wy + 1, 1);
+        if (t.ty == 0) row_to_lds(fam(a.ep, 0, np), pl + t.col - (uint32_t)a.nzi, &l_rho[nb][0][1]);
       } else {
         v.rho = *at(fam(a.ep, 0, np), pl + t.col);
         if (t.ty == 0) v.rho_hx = *at(fam(a.ep, 0, np), pl + t.col - (uint32_t)a.nzi);
@@ -858,9 +893,9 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
         m3[1] = stag_buoy(a, rc, rho_prev);
         m3[2] = stag_buoy(a, rc, l_rho[b][t.ty + 1][t.tz]);
       }
-      const T sx = dmx<T, BX>(l_xx[b], r, q, cx) + dq(qxy, cy) + dpz<T, BX>(l_xz[b], r, q, cz);
-      const T sy = dpx<T, BX>(l_xy[b], r, q, cx) + dq(qyy, cy) + dpz<T, BX>(l_yz[b], r, q, cz);
-      const T sz = dpx<T, BX>(l_xz[b], r, q, cx) + dq(qyz, cy) + dmz<T, BX>(l_zz[b], r, q, cz);
+      const T sx = dmx<T, S>(l_xx[b], r, q, cx) + dq(qxy, cy) + dpz<T, S>(l_xz[b], r, q, cz);
+      const T sy = dpx<T, S>(l_xy[b], r, q, cx) + dq(qyy, cy) + dpz<T, S>(l_yz[b], r, q, cz);
+      const T sz = dpx<T, S>(l_xz[b], r, q, cx) + dq(qyz, cy) + dmz<T, S>(l_zz[b], r, q, cz);
       T w = T(0);
       if (!QS || t.active) w = damp_w(a, t.izo, t.ix, iy, t.wy0, t.wny, t.wnx);
       const T s3[3] = {sx, sy, sz};
@@ -904,7 +939,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     __syncthreads();
     b ^= 1;
   }
-  inject_tile<T, BX, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
+  inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
 }
 
 // ---------------------------------------------------------------------------
@@ -912,10 +947,10 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
 // ---------------------------------------------------------------------------
 // The stress stepper's LDS: double-buffered planes of vx, vy, vz and (F_MED3)
 // shear-modulus planes with the low x row and low z column.
-template <typename T, int BX, bool MED3>
+template <typename T, int S, bool MED3>
 struct StressLds {
-  Plane<T, BX> vx[2], vy[2], vz[2];
-  T mu[2][MED3 ? BX + 1 : 1][MED3 ? TZ + 1 : 1];
+  Plane<T, S> vx[2], vy[2], vz[2];
+  T mu[2][MED3 ? tile_x(S) + 1 : 1][MED3 ? tile_z(S) + 1 : 1];
 };
 
 template <typename T>
@@ -925,8 +960,9 @@ struct StressStage {
   T mu, mu_hx, mu_hz, mu_hc; // F_MED3: shear modulus of the column, row x0 - 1, z0 - 1 and both
 };
 
-template <typename T, int BX, int MODE, int F>
-__device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, StressLds<T, BX, (F & F_MED3) != 0>& L) {
+template <typename T, int S, int MODE, int F>
+__device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, StressLds<T, S, (F & F_MED3) != 0>& L) {
+  constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
@@ -935,7 +971,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   static_assert(!MED3 || MODE == MODE_FWD || MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_PM,
                 "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz; auto& l_mu = L.mu;
-  const TileCoord t = tile_coord<BX>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   int64_t np = a.np;
@@ -954,9 +990,9 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
     v.nz = V_().v(VZ, pl + 3 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
-        row_to_lds(src(VX), pl + t.cxl, &l_vx[nb][wy][FAT]); row_to_lds(src(VX), pl + t.cxh, &l_vx[nb][wr + BX][FAT]);
-        row_to_lds(src(VY), pl + t.cxl, &l_vy[nb][wy][FAT]); row_to_lds(src(VY), pl + t.cxh, &l_vy[nb][wr + BX][FAT]);
-        row_to_lds(src(VZ), pl + t.cxl, &l_vz[nb][wy][FAT]); row_to_lds(src(VZ), pl + t.cxh, &l_vz[nb][wr + BX][FAT]);
+        rows_to_lds<S>(src(VX), pl + t.cxl, l_vx[nb], wy, FAT); rows_to_lds<S>(src(VX), pl + t.cxh, l_vx[nb], wr + BX, FAT);
+        rows_to_lds<S>(src(VY), pl + t.cxl, l_vy[nb], wy, FAT); rows_to_lds<S>(src(VY), pl + t.cxh, l_vy[nb], wr + BX, FAT);
+        rows_to_lds<S>(src(VZ), pl + t.cxl, l_vz[nb], wy, FAT); rows_to_lds<S>(src(VZ), pl + t.cxh, l_vz[nb], wr + BX, FAT);
       } else {
 #pragma unroll
         for (int f = 0; f < 3; ++f) { v.hlo[f] = V_().v(f, pl + t.cxl); v.hhi[f] = V_().v(f, pl + t.cxh); }
@@ -971,8 +1007,8 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
   auto fetch_mu = [&](StressStage<T>& v, int p, int nb) {
     const uint32_t pl = (uint32_t)p * ys, nzi = (uint32_t)a.nzi;
     if constexpr (DMA) {
-      row_to_lds(fam(a.ep, 2, np), pl + t.col, &l_mu[nb][wy + 1][1]);
-      if (wy == 0) row_to_lds(fam(a.ep, 2, np), pl + t.col - nzi, &l_mu[nb][0][1]);
+      rows_to_lds<S>(fam(a.ep, 2, np), pl + t.col, l_mu[nb], wy + 1, 1);
+      if (t.ty == 0) row_to_lds(fam(a.ep, 2, np), pl + t.col - nzi, &l_mu[nb][0][1]);
     } else {
       v.mu = *at(fam(a.ep, 2, np), pl + t.col);
       if (t.ty == 0) v.mu_hx = *at(fam(a.ep, 2, np), pl + t.col - nzi);
@@ -1103,12 +1139,12 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
         l2m = ld_nt(fam(a.m, L2M, np), i); lam = ld_nt(fam(a.m, LAM, np), i);
         mxz = ld_nt(fam(a.m, MXZ, np), i); mxy = ld_nt(fam(a.m, MXY, np), i); myz = ld_nt(fam(a.m, MYZ, np), i);
       }
-      const T exx = dpx<T, BX>(l_vx[b], r, q, cx);
+      const T exx = dpx<T, S>(l_vx[b], r, q, cx);
       const T eyy = dq(qy, cy);
-      const T ezz = dpz<T, BX>(l_vz[b], r, q, cz);
-      const T gxy = dq(qx, cy) + dmx<T, BX>(l_vy[b], r, q, cx);
-      const T gxz = dmz<T, BX>(l_vx[b], r, q, cz) + dmx<T, BX>(l_vz[b], r, q, cx);
-      const T gyz = dq(qz, cy) + dmz<T, BX>(l_vy[b], r, q, cz);
+      const T ezz = dpz<T, S>(l_vz[b], r, q, cz);
+      const T gxy = dq(qx, cy) + dmx<T, S>(l_vy[b], r, q, cx);
+      const T gxz = dmz<T, S>(l_vx[b], r, q, cz) + dmx<T, S>(l_vz[b], r, q, cx);
+      const T gyz = dq(qz, cy) + dmz<T, S>(l_vy[b], r, q, cz);
       T w = T(0);
       if (!QS || t.active) w = damp_w(a, t.izo, t.ix, iy, t.wy0, t.wny, t.wnx);
       if (F & F_STORE) {
@@ -1188,7 +1224,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
     __syncthreads();
     b ^= 1;
   }
-  inject_tile<T, BX, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
+  inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1208,21 +1244,21 @@ constexpr int step_waves() {
   return sizeof(T) == 4 && ((FV | FS) & (F_SS | F_ACC | F_GRAD)) == 0 ? 4 : 1;
 }
 
-template <typename T, int BX, int MODE, int FV, int FS>
-__global__ void __launch_bounds__(TZ * BX, (step_waves<T, FV, FS>())) k_step(StepArgs<T> a, PointArgs<T> inj, PointArgs<T> rec) {
+template <typename T, int S, int MODE, int FV, int FS>
+__global__ void __launch_bounds__(tile_threads(S), (step_waves<T, FV, FS>())) k_step(StepArgs<T> a, PointArgs<T> inj, PointArgs<T> rec) {
   // one LDS object: the compiler's wait analysis then tells the rows the
   // direct loads fill (buffer b ^ 1) from the rows the stencil reads (buffer b)
   union Lds {
-    VelLds<T, BX, (FV & F_MED3) != 0> v;
-    StressLds<T, BX, (FS & F_MED3) != 0> s;
+    VelLds<T, S, (FV & F_MED3) != 0> v;
+    StressLds<T, S, (FS & F_MED3) != 0> s;
   };
   __shared__ Lds L;
   (void)inj;  // read by inject_tile
   static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
-  if (bid < nb) velocity_block<T, BX, MODE, FV>(a, bid, L.v);
-  else if (bid < 2 * nb) stress_block<T, BX, MODE, FS>(a, bid - nb, L.s);
-  else record_point(rec, (int64_t)(bid - 2 * nb) * (TZ * BX) + threadIdx.y * TZ + threadIdx.x);
+  if (bid < nb) velocity_block<T, S, MODE, FV>(a, bid, L.v);
+  else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, bid - nb, L.s);
+  else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
 }
 
 // The injection by itself: lists too long or too spread for a step's blocks.
@@ -1283,9 +1319,9 @@ struct ImagingArgs {
 
 // The imaging kernels' LDS: double-buffered planes of the coarse vx, vy, vz
 // slice V[its] (one LDS object, see k_step).
-template <typename T, int BX>
+template <typename T, int S>
 struct ImagingLds {
-  Plane<T, BX> vx[2], vy[2], vz[2];
+  Plane<T, S> vx[2], vy[2], vz[2];
 };
 
 // Secondary sources (forward) or images (adjoint) of coarse sample its. The
@@ -1299,11 +1335,12 @@ struct ImagingLds {
 // V[its - 1] and V[its + 1] (not at the ends of the record) and the 8
 // perturbations (forward, writing 9 secondary sources) or the 9 adjoint
 // slices and the 8 FP64 images (adjoint, rewriting the images).
-template <typename T, int BX, bool ADJ>
-__global__ void __launch_bounds__(TZ * BX) k_imaging(ImagingArgs<T> a) {
-  __shared__ ImagingLds<T, BX> L;
+template <typename T, int S, bool ADJ>
+__global__ void __launch_bounds__(tile_threads(S)) k_imaging(ImagingArgs<T> a) {
+  constexpr int BX = tile_x(S);
+  __shared__ ImagingLds<T, S> L;
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz;
-  const TileCoord t = tile_coord<BX>(blockIdx.x, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
+  const TileCoord t = tile_coord<S>(blockIdx.x, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4;
@@ -1322,9 +1359,9 @@ __global__ void __launch_bounds__(TZ * BX) k_imaging(ImagingArgs<T> a) {
     v.nz = *at(a.c[2], pl + 3 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders are whole waves
       if constexpr (DMA) {
-        row_to_lds(a.c[0], pl + t.cxl, &l_vx[nb][wy][FAT]); row_to_lds(a.c[0], pl + t.cxh, &l_vx[nb][wr + BX][FAT]);
-        row_to_lds(a.c[1], pl + t.cxl, &l_vy[nb][wy][FAT]); row_to_lds(a.c[1], pl + t.cxh, &l_vy[nb][wr + BX][FAT]);
-        row_to_lds(a.c[2], pl + t.cxl, &l_vz[nb][wy][FAT]); row_to_lds(a.c[2], pl + t.cxh, &l_vz[nb][wr + BX][FAT]);
+        rows_to_lds<S>(a.c[0], pl + t.cxl, l_vx[nb], wy, FAT); rows_to_lds<S>(a.c[0], pl + t.cxh, l_vx[nb], wr + BX, FAT);
+        rows_to_lds<S>(a.c[1], pl + t.cxl, l_vy[nb], wy, FAT); rows_to_lds<S>(a.c[1], pl + t.cxh, l_vy[nb], wr + BX, FAT);
+        rows_to_lds<S>(a.c[2], pl + t.cxl, l_vz[nb], wy, FAT); rows_to_lds<S>(a.c[2], pl + t.cxh, l_vz[nb], wr + BX, FAT);
       } else {
 #pragma unroll
         for (int f = 0; f < 3; ++f) { v.hlo[f] = *at(a.c[f], pl + t.cxl); v.hhi[f] = *at(a.c[f], pl + t.cxh); }
@@ -1388,15 +1425,15 @@ __global__ void __launch_bounds__(TZ * BX) k_imaging(ImagingArgs<T> a) {
         for (int k = 0; k < 8; ++k) dmo[k] = a.dmo[k][i];   // 64-bit indexing: FP64 offsets can pass 4 GiB
       }
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
-      const T exx = dpx<T, BX>(l_vx[b], r, q, cx);
+      const T exx = dpx<T, S>(l_vx[b], r, q, cx);
       const T eyy = dq(qy, cy);
-      const T ezz = dpz<T, BX>(l_vz[b], r, q, cz);
-      const T gxy = dq(qx, cy) + dmx<T, BX>(l_vy[b], r, q, cx);
-      const T gxz = dmz<T, BX>(l_vx[b], r, q, cz) + dmx<T, BX>(l_vz[b], r, q, cx);
+      const T ezz = dpz<T, S>(l_vz[b], r, q, cz);
+      const T gxy = dq(qx, cy) + dmx<T, S>(l_vy[b], r, q, cx);
+      const T gxz = dmz<T, S>(l_vx[b], r, q, cz) + dmx<T, S>(l_vz[b], r, q, cx);
       // yz term: the reference uses the xz derivative pattern
       // (kernelsElaGpu_3D.cu:1419-1431, :1622-1634); physics mode the yz one
       // of the stepper's syz update (D-y vz + D-z vy)
-      const T gyz = a.physics ? dq(qz, cy) + dmz<T, BX>(l_vy[b], r, q, cz) : gxz;
+      const T gyz = a.physics ? dq(qz, cy) + dmz<T, S>(l_vy[b], r, q, cz) : gxz;
       if constexpr (!ADJ) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) st_nt(a.ss[k], i, dm[k] * dv[k] * a.dts_inv);

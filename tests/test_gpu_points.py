@@ -84,3 +84,31 @@ def test_fused_and_separate_injection_give_the_same_bits(precision):
         prop.set_tiling(tx, yc)
         out.append(prop.nl_forward(pos, src, pos) + [prop.born_adjoint(pos, src, src, pos)])
     assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+# z interiors of one 32-cell tile, one cell more, a ragged last tile, and one
+# where FP32 keeps the 64-cell tiles; x interiors below, at and past 8 rows
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("iz,ix", [(32, 8), (33, 9), (90, 7), (64, 17), (1, 1)])
+def test_narrow_tiles(precision, iz, ix):
+    """32 x 8 tiles (4 rows set) against 64 x 8 tiles bit for bit, and the
+    oracle, for the forward, the gradient (derivative store and paired
+    imaging) and the Born pair."""
+    g = O.Grid(nz=iz + 8, nx=ix + 8, ny=17, nts=3, sub=4, dz=10.0, dx=10.0, dy=10.0, dts=0.002, minPad=2, alphaCos=0.95)
+    P = random_problem(g, seed=iz, nsrc=1, nrec=1)
+    prop = make_prop(g, precision)
+    prop.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+    prop.set_gradient_checkpoints(4, 0, "native")
+    out = []
+    for tx, yc in ((4, 3), (8, 4)):
+        prop.set_tiling(tx, yc)
+        rec = prop.gradient_forward(P["spos"], P["src"], P["rpos"])
+        g8, gs = prop.gradient_backward(P["spos"], P["src"], P["rpos"], P["rec"])
+        out.append([*rec, g8, *gs, *prop.nl_adjoint(P["spos"], P["rec"], P["rpos"]),
+                    *prop.born_forward(P["spos"], P["src"], P["dm"], P["rpos"]),
+                    prop.born_adjoint(P["spos"], P["src"], P["rec"], P["rpos"])])
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    fwd = O.lib_nl_forward(g, P["med"], P["src"], P["spos"], P["rpos"])
+    g8_ref, gs_ref = O.lib_gradient(g, P["med"], P["src"], P["spos"], P["rec"], P["rpos"])
+    assert rel(rec, fwd) < TOL[precision]
+    assert rel(g8, g8_ref) < 2 * TOL[precision] and rel(gs, gs_ref) < 2 * TOL[precision]
