@@ -654,7 +654,7 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
   const auto& a = *(const ELA_KERNARG PointArgs<T>*)(seg + sizeof(StepArgs<T>));
 #undef ELA_KERNARG
   if (a.off[9] == 0) return;  // kernel-uniform
-  const int bid = (int)blockIdx.x + s.first - half * s.nbz * s.nbx * s.nby;
+  const int nb = s.nbz * s.nbx * s.nby, b0 = (int)blockIdx.x + s.first, bid = half ? b0 - nb : nb - 1 - b0;
   const TileCoord t = tile_coord<S>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
   const int* b = a.box;
   constexpr int BX = tile_x(S), BZ = tile_z(S);
@@ -1235,6 +1235,13 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
 // 110x93x121 49.8 -> 43.4 us, 152x152x148 105.8 -> 96.9 us (FP32, tile 8x8,
 // order 3/2). Large grids gain only the first half's tail (232x328x324 638.7
 // -> 637.2 us, 328x472x468 1721.8 -> 1718.6 us): they are bound by HBM.
+//
+// The velocity blocks run through the tiles backwards: the stress blocks of
+// the launch before ended at the last tiles, and what they wrote and read
+// there (sigma n, v n-1, 9 of the 13 arrays a velocity block touches) is
+// still in the 256 MB Infinity Cache. Forward 328x472x468, 80 steps, 144.1
+// -> 140.2 ms, adjoint 232x328x324 64.7 -> 62.9 ms, Born adjoint 83.2 -> 78.1
+// ms; nothing at 152x152x148, which the cache does not limit.
 // ---------------------------------------------------------------------------
 // Waves per SIMD asked of the compiler: the FP32 steps without per-cell extra
 // operands need 115-129 VGPRs and run at 4 (at most 128); the others hold more
@@ -1256,7 +1263,7 @@ __global__ void __launch_bounds__(tile_threads(S), (step_waves<T, FV, FS>())) k_
   (void)inj;  // read by inject_tile
   static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
-  if (bid < nb) velocity_block<T, S, MODE, FV>(a, bid, L.v);
+  if (bid < nb) velocity_block<T, S, MODE, FV>(a, nb - 1 - bid, L.v);
   else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, bid - nb, L.s);
   else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
 }
