@@ -408,21 +408,6 @@ Tiles tiles_for(const ela_handle* h, int shape, int ychunk) {
   return t;
 }
 
-// Launch shape of a new handle (until ela_set_tiling / ela_set_tile_order).
-// 256-thread blocks of 4 x rows, whole z columns in groups of 4 x columns per
-// XCD: the fastest or within 1 % of it on every grid and step kind measured
-// but the recomputation with derivative store (2 % behind 8 rows) and the
-// FP64 forward of large grids (3 % behind 8x16); against the former 16x8 in
-// hardware order, us per FP32 step with (rho, lambda, mu): 152x152x148 100.8
-// -> 96, 201x187x143 173 -> 155, 232x328x324 661 -> 631, 328x472x468 1736 ->
-// 1712; its transposed step with imaging 1572 -> 1186 (232x328x324), where 16
-// rows spill. Planes per block: 8, the prologue's 7 planes of queue values
-// being paid once per block, unless the blocks of the two halves then leave
-// CUs idle; a shorter march has less latency to pay as long as the blocks are
-// resident together (256 CUs x 4 waves per SIMD of FP32 blocks, 2 of FP64
-// ones): 72x72x72 18.6 us a step with 8 planes, 15.5 with 2; 40x36x44 15.8
-// -> 10.8. 7/8 of the residency counts as full: 88x97x90 (1012 blocks of 1024)
-// 28.8 us with 8 planes, 29.4 with 4; a march of 1 gains nothing over 2.
 // Whether 256-thread blocks are narrow tiles (32 z x 8 x cells) instead of
 // wide ones (64 x 4). FP64: always; the 8 rows share their x halo (2 rows read
 // per row owned instead of 3) and the planes take 3/4 of the LDS: forward step
@@ -439,16 +424,44 @@ bool narrow_tiles(int esize, int64_t iz) {
 // Tile shape for an x tile set by ela_set_tiling.
 int shape_of(const ela_handle* h, int bx) { return bx == 4 && h->narrow ? ela::TILE_NARROW : bx; }
 
+// Launch shape of a new handle (until ela_set_tiling / ela_set_tile_order).
+// 256-thread blocks, whole z columns in groups of 4 x columns per XCD: the
+// fastest or within 1 % of it on every grid and step kind measured but the
+// recomputation with derivative store (2 % behind 8 rows); against 16 rows in
+// hardware order, us per FP32 step with (rho, lambda, mu): 152x152x148 100.8
+// -> 96, 201x187x143 173 -> 155, 232x328x324 661 -> 631, 328x472x468 1736 ->
+// 1712; its transposed step with imaging 1572 -> 1186 (232x328x324), where 16
+// rows spill.
+//
+// Planes per block: 8 where the blocks of the two halves fill the chip more
+// than 5 times over (the prologue's 7 planes of queue values are paid once a
+// block, and 6 to 16 planes then lie within 1 %). Below that whole rounds of
+// resident blocks count: a grid of 1.3 rounds takes as long as one of 2. A
+// round costs its march plus about 4 planes of launch, prologue and first
+// latency, so the least rounds x (planes + 4) is taken, rounds summed over the
+// resident blocks of the light steps (FP32: 4 waves per SIMD, 1024 blocks) and
+// of those with extra operands (3 waves, 768); FP64 steps have 2 (512). us per
+// step with 8 planes -> with the rule's: FP32 152x152x148 87.5 -> 82.8 (13
+// planes, 1.9 rounds), 110x93x121 37.1 -> 35.1 (7), 72x72x72 16.8 -> 14.5 (3),
+// 40x36x44 15.2 -> 8.7 (2); FP64 88x97x90 43.3 -> 37.7 (12), its transposed
+// step with imaging 62.6 -> 55.3, 110x93x121 74.7 -> 70.4 (11).
 void initial_shape(ela_handle* h) {
   const int64_t iz = h->cfg.nz - 2 * ela::FAT, ix = h->cfg.nx - 2 * ela::FAT, iy = h->cfg.ny - 2 * ela::FAT;
   h->narrow = narrow_tiles(h->esize, iz);
-  const int bz = ela::tile_z(shape_of(h, h->by_x)), bx = ela::tile_x(shape_of(h, h->by_x));
+  const int S = shape_of(h, h->by_x), bz = ela::tile_z(S), bx = ela::tile_x(S);
   const int64_t cols = ((iz + bz - 1) / bz) * ((ix + bx - 1) / bx);
-  const int64_t resident = 256 * (h->esize == 4 ? 4 : 2);
-  const int planes[] = {8, 6, 4, 3, 2};
-  for (int yc : planes) {
-    h->ychunk = yc;
-    if (2 * cols * ((iy + yc - 1) / yc) >= resident * 7 / 8) break;
+  const int64_t resident[2] = {256 * (h->esize == 4 ? 4 : 2), 256 * (h->esize == 4 ? 3 : 2)};
+  const auto blocks = [&](int64_t yc) { return 2 * cols * ((iy + yc - 1) / yc); };
+  h->ychunk = 8;
+  if (blocks(8) > 5 * resident[0]) return;
+  double best = 0;
+  for (int yc = 2; yc <= 13; ++yc) {
+    double cost = 0;
+    for (int64_t r : resident) {
+      const double rounds = double(blocks(yc)) / double(r);
+      cost += (rounds <= 4 ? std::ceil(rounds) : rounds + 0.5) * (yc + 4);
+    }
+    if (best == 0 || cost < best) { best = cost; h->ychunk = yc; }
   }
 }
 

@@ -630,16 +630,26 @@ __device__ __forceinline__ void record_point(const PointArgs<T>& a, int64_t g) {
 // Injection by a step's own blocks: after its march a block whose tile meets
 // the points' box adds the listed points inside its tile (components c0 ..
 // c1 - 1, those the block has written) with inject_point, so that a step with
-// few sources is one launch. With the recording moved into the step after
-// (step_with_points) that took 40x36x44, 100 steps through host arrays, from
-// 1.68 to 1.17 ms, 152x152x148 (200 steps) from 20.1 to 18.6 ms and
-// 328x472x468 with 2.9 M recorded points (80 steps) from 143.0 to 138.9 ms. The barrier orders the block's stores of the new
+// few sources is one launch. The barrier orders the block's stores of the new
 // level before the read-modify-writes; no other block touches these cells.
+// With the recording moved into the step after (step_with_points) that took
+// 40x36x44, 100 steps through host arrays, from 1.68 to 1.17 ms, 152x152x148
+// (200 steps) from 20.1 to 18.6 ms and 328x472x468 with 2.9 M recorded points
+// (80 steps) from 143.0 to 138.9 ms.
+//
 // box: the largest of (POS_TOP - z, z, POS_TOP - x, x, POS_TOP - y, y) over
-// the points, in internal z, so that a zeroed box holds nothing.
+// the points, in internal z, so that a zeroed box holds nothing. It is tested
+// during the prologue, where its load hides behind the stencil's (40x36x44: 8.16 -> 7.97 us a step).
 constexpr int POS_TOP = 1 << 30;
 
-//
+template <typename T, int S>
+__device__ __forceinline__ bool box_hit(const PointArgs<T>& a, const TileCoord& t) {
+  if (a.off[9] == 0) return false;
+  const int* b = a.box;
+  return POS_TOP - b[0] < t.z0 + tile_z(S) && b[1] >= t.z0 && POS_TOP - b[2] < t.x0 + tile_x(S) && b[3] >= t.x0 &&
+         POS_TOP - b[4] < t.y1 && b[5] >= t.y0;
+}
+
 // Everything is read again from the kernel's argument segment (k_step's
 // second argument is the injection) through an address the compiler cannot
 // trace back, and the tile worked out again from the block index: kept live
@@ -653,14 +663,9 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
   const auto& s = *(const ELA_KERNARG StepArgs<T>*)seg;
   const auto& a = *(const ELA_KERNARG PointArgs<T>*)(seg + sizeof(StepArgs<T>));
 #undef ELA_KERNARG
-  if (a.off[9] == 0) return;  // kernel-uniform
   const int nb = s.nbz * s.nbx * s.nby, b0 = (int)blockIdx.x + s.first, bid = half ? b0 - nb : nb - 1 - b0;
   const TileCoord t = tile_coord<S>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
-  const int* b = a.box;
   constexpr int BX = tile_x(S), BZ = tile_z(S);
-  const bool hit = POS_TOP - b[0] < t.z0 + BZ && b[1] >= t.z0 && POS_TOP - b[2] < t.x0 + BX && b[3] >= t.x0 &&
-                   POS_TOP - b[4] < t.y1 && b[5] >= t.y0;
-  if (!hit) return;  // block-uniform
   __syncthreads();
   for (int g = (int)a.off[c0] + t.ty * BZ + t.tz; g < (int)a.off[c1]; g += BZ * BX) {
     int c = c0;
@@ -745,7 +750,8 @@ __device__ __forceinline__ void normal_moduli(T tdt, double tdt64, T lam, T mu, 
 }
 
 template <typename T, int S, int MODE, int F>
-__device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, VelLds<T, S, (F & F_MED3) != 0>& L) {
+__device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
+                                               VelLds<T, S, (F & F_MED3) != 0>& L) {
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
@@ -839,10 +845,12 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     qyy[j] = S_().syy((uint32_t)(t.y0 - 4 + j) * ys + t.col);
     qyz[j] = S_().syz((uint32_t)(t.y0 - 3 + j) * ys + t.col);
   }
+  bool inj_hit;  // block-uniform
   {
     VelStage<T> v0;
     fetch(v0, t.y0, 0);
     qxy[7] = v0.nxy; qyy[7] = v0.nyy; qyz[7] = v0.nyz;
+    inj_hit = box_hit<T, S>(inj, t);
     stage(0, v0, qxy[3], qyz[3]);
   }
   __syncthreads();
@@ -939,7 +947,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, int bid, Ve
     __syncthreads();
     b ^= 1;
   }
-  inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
 }
 
 // ---------------------------------------------------------------------------
@@ -961,7 +969,8 @@ struct StressStage {
 };
 
 template <typename T, int S, int MODE, int F>
-__device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, StressLds<T, S, (F & F_MED3) != 0>& L) {
+__device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
+                                             StressLds<T, S, (F & F_MED3) != 0>& L) {
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
@@ -1053,10 +1062,12 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
     muz_prev = *at(fam(a.ep, 2, np), pl + t.col - 1u);
     sx_prev = T(0.5) * (mu_prev + *at(fam(a.ep, 2, np), pl + t.col - (uint32_t)a.nzi));
   }
+  bool inj_hit;  // block-uniform
   {
     StressStage<T> v0;
     fetch(v0, t.y0, 0);
     qx[7] = v0.nx; qy[7] = v0.ny; qz[7] = v0.nz;
+    inj_hit = box_hit<T, S>(inj, t);
     stage(0, v0, qx[4], qy[3], qz[4]);
     if (MED3) {
       fetch_mu(v0, t.y0, 0);
@@ -1224,7 +1235,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, int bid, Stre
     __syncthreads();
     b ^= 1;
   }
-  inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1260,11 +1271,10 @@ __global__ void __launch_bounds__(tile_threads(S), (step_waves<T, FV, FS>())) k_
     StressLds<T, S, (FS & F_MED3) != 0> s;
   };
   __shared__ Lds L;
-  (void)inj;  // read by inject_tile
   static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
-  if (bid < nb) velocity_block<T, S, MODE, FV>(a, nb - 1 - bid, L.v);
-  else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, bid - nb, L.s);
+  if (bid < nb) velocity_block<T, S, MODE, FV>(a, inj, nb - 1 - bid, L.v);
+  else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, inj, bid - nb, L.s);
   else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
 }
 

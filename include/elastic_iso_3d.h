@@ -380,7 +380,7 @@ int ela_set_graph(ela_handle* h, int on);
 
 /* Tile shape of the stencil kernels: x extent of a 64-wide z tile (4, 8 or
  * 16 rows) and the number of y planes one block marches through (a new
- * handle: 4 rows and 2 to 8 planes, by the grid's size). 4 rows become 8 rows
+ * handle: 4 rows and 2 to 13 planes, by the grid's size). 4 rows become 8 rows
  * of a 32-wide z tile where that is faster (FP64, and z extents that leave
  * fewer cells idle), 16 rows become 4 in the steps whose registers do not
  * allow 16. Any setting gives the same result; it only changes speed. */
