@@ -1293,23 +1293,47 @@ __global__ void __launch_bounds__(256) k_record(PointArgs<T> a) {
   record_point(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-// Out-of-place transpose of a [rows][cols] block (row stride ld_in) into
-// [cols][rows] (row stride ld_out).
+// Caller traces tr[c] = [n[c]][nts] of the 9 components <-> the time-major
+// buffer tm = [nts][tot], component c at column off[c]. blockIdx.z = c.
 template <typename T>
-__global__ void __launch_bounds__(256) k_transpose(const T* __restrict__ in, T* __restrict__ out, int64_t rows,
-                                                   int64_t cols, int64_t ld_in, int64_t ld_out) {
+struct TransposeArgs {
+  T* tr[9];
+  T* tm;
+  int64_t n[9], off[9];
+  int64_t nts, tot;
+};
+
+template <typename T, bool TO_TM>
+__global__ void __launch_bounds__(256) k_transpose(TransposeArgs<T> a) {
   __shared__ T tile[32][33];
-  const int64_t c0 = (int64_t)blockIdx.x * 32, r0 = (int64_t)blockIdx.y * 32;
+  const int c = blockIdx.z;
+  const int64_t p0 = (int64_t)blockIdx.x * 32, n = a.n[c];
+  if (p0 >= n) return;  // block-uniform
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-  for (int j = ty; j < 32; j += 8) {
-    const int64_t rr = r0 + j, cc = c0 + tx;
-    if (rr < rows && cc < cols) tile[j][tx] = in[rr * ld_in + cc];
+  for (int64_t t0 = (int64_t)blockIdx.y * 32; t0 < a.nts; t0 += (int64_t)gridDim.y * 32) {
+    for (int j = ty; j < 32; j += 8) {
+      if (TO_TM ? (p0 + j < n && t0 + tx < a.nts) : (t0 + j < a.nts && p0 + tx < n))
+        tile[j][tx] = TO_TM ? a.tr[c][(p0 + j) * a.nts + t0 + tx] : a.tm[(t0 + j) * a.tot + a.off[c] + p0 + tx];
+    }
+    __syncthreads();
+    for (int j = ty; j < 32; j += 8) {
+      if (TO_TM) {
+        if (t0 + j < a.nts && p0 + tx < n) a.tm[(t0 + j) * a.tot + a.off[c] + p0 + tx] = tile[tx][j];
+      } else if (p0 + j < n && t0 + tx < a.nts) {
+        a.tr[c][(p0 + j) * a.nts + t0 + tx] = tile[tx][j];
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  for (int j = ty; j < 32; j += 8) {
-    const int64_t cc = c0 + j, rr = r0 + tx;
-    if (rr < rows && cc < cols) out[cc * ld_out + rr] = tile[tx][j];
-  }
+}
+
+// The 9 trace arrays cleared (blockIdx.y = component).
+template <typename T>
+__global__ void __launch_bounds__(256) k_clear_traces(TransposeArgs<T> a) {
+  const int c = blockIdx.y;
+  const int64_t n = a.n[c] * a.nts;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    a.tr[c][i] = T(0);
 }
 
 // Born forward secondary sources for coarse sample `its`
@@ -1488,25 +1512,38 @@ __global__ void __launch_bounds__(tile_threads(S)) k_imaging(ImagingArgs<T> a) {
 // the FD interior are replaced by -1 (skipped by the point kernels) and
 // reported through *bad; box (or null) becomes the box of the others (see
 // inject_tile).
-__global__ void __launch_bounds__(256) k_convert_pos(const int64_t* __restrict__ in, int32_t* __restrict__ out,
-                                                     int64_t n, int nz, int nx, int ny, int nzi, int zoff,
-                                                     const int* ytab, int* bad, int* box) {
+struct ConvertArgs {
+  const int64_t* in[14];   // 7 source lists, 7 receiver lists
+  int64_t off[15];         // prefix offsets over the lists
+  int32_t* out;            // the converted lists, one after another
+  int nz, nx, ny, nzi, zoff;
+  const int* ytab;
+  int* bad;
+  int* box[2];             // of the sources and of the receivers, or null
+};
+
+__global__ void __launch_bounds__(256) k_convert_pos(ConvertArgs a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t p = in[i];
+  if (i >= a.off[14]) return;
+  int l = 0;
+#pragma unroll
+  for (int k = 1; k < 14; ++k) l += i >= a.off[k] ? 1 : 0;
+  const int64_t p = a.in[l][i - a.off[l]];
+  const int nz = a.nz, nx = a.nx, ny = a.ny;
   const int64_t ys = (int64_t)nz * nx;
   const int64_t iy = (p >= 0 && p < ys * ny) ? p / ys : -1;
   const int64_t r = p - iy * ys;
   const int64_t ix = r / nz, iz = r - ix * nz;
   bool ok = iy >= FAT && iy < ny - FAT && ix >= FAT && ix < nx - FAT && iz >= FAT && iz < nz - FAT;
-  if (ok && ytab) {  // inside the interior of its window
-    const int wy0 = ytab[4 * iy], wny = ytab[4 * iy + 1], wnx = ytab[4 * iy + 2];
+  if (ok && a.ytab) {  // inside the interior of its window
+    const int wy0 = a.ytab[4 * iy], wny = a.ytab[4 * iy + 1], wnx = a.ytab[4 * iy + 2];
     ok = wny > 0 && iy >= wy0 + FAT && iy < wy0 + wny - FAT && ix < wnx - FAT;
   }
-  out[i] = ok ? (int32_t)(iy * nx * nzi + ix * nzi + iz + zoff) : -1;
-  if (!ok) atomicOr(bad, 1);
+  a.out[i] = ok ? (int32_t)(iy * nx * a.nzi + ix * a.nzi + iz + a.zoff) : -1;
+  int* box = a.box[l >= 7];
+  if (!ok) atomicOr(a.bad, 1);
   else if (box) {
-    const int c[3] = {(int)iz + zoff, (int)ix, (int)iy};
+    const int c[3] = {(int)iz + a.zoff, (int)ix, (int)iy};
     for (int k = 0; k < 3; ++k) { atomicMax(box + 2 * k, POS_TOP - c[k]); atomicMax(box + 2 * k + 1, c[k]); }
   }
 }

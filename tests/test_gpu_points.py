@@ -112,3 +112,23 @@ def test_narrow_tiles(precision, iz, ix):
     g8_ref, gs_ref = O.lib_gradient(g, P["med"], P["src"], P["spos"], P["rec"], P["rpos"])
     assert rel(rec, fwd) < TOL[precision]
     assert rel(g8, g8_ref) < 2 * TOL[precision] and rel(gs, gs_ref) < 2 * TOL[precision]
+
+
+# 16 points x 300 samples: packed (173 kB of receiver traces); x 1000: past the packed size, copied array by array
+@pytest.mark.parametrize("nts", [300, 1000])
+def test_host_traces_packed_and_direct(nts):
+    """Host-memory calls against the same call on device tensors, bit for
+    bit, for trace blocks that travel in one pinned copy and larger ones."""
+    import torch
+    g = O.Grid(nz=20, nx=19, ny=18, nts=nts, sub=1, dz=10.0, dx=10.0, dy=10.0, dts=0.0005, minPad=3, alphaCos=0.95)
+    P = random_problem(g, seed=9, nsrc=2, nrec=16)
+    prop = make_prop(g, "f32")
+    prop.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+    dev = lambda xs, dt: [torch.tensor(np.asarray(x), dtype=dt, device="cuda") for x in xs]  # noqa: E731
+    sp, rp = dev(P["spos"], torch.int64), dev(P["rpos"], torch.int64)
+    src, rec = dev(P["src"], torch.float32), dev(P["rec"], torch.float32)
+    for _ in range(2):
+        pairs = [(prop.nl_forward(P["spos"], P["src"], P["rpos"]), prop.nl_forward(sp, src, rp)),
+                 (prop.nl_adjoint(P["spos"], P["rec"], P["rpos"]), prop.nl_adjoint(sp, rec, rp))]
+        for host, device in pairs:
+            assert all(np.array_equal(a, b.cpu().numpy()) for a, b in zip(host, device))
