@@ -1165,9 +1165,10 @@ int bg_coarse_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_
 // V[its+1] (null outside 0..nts-1).
 template <typename T>
 ela::ImagingArgs<T> imaging_args(ela_handle* h, const T* Vo, const T* Vc, const T* Vn, int64_t its, const T* dm,
-                                 double* dmo, T* const ss[9]) {
+                                 double* dmo, T* const ss[9], bool init = false) {
   ela::ImagingArgs<T> a;
   std::memset(&a, 0, sizeof(a));
+  a.init = init;
   const int64_t np = h->stride;
   for (int k = 0; k < 3; ++k) {
     a.o[k] = Vo ? Vo + k * np : nullptr;
@@ -1218,13 +1219,13 @@ struct BornPlan {
 
 // Arrays (of h->stride elements) the Born adjoint needs besides V and the
 // checkpoints: medium 8, background wavefield 18, adjoint wavefield with its
-// premultiplied levels 36, secondary sources 18, images 8 (FP32 handles: and
-// their FP64 accumulator, 16 more).
+// premultiplied levels 36, secondary sources 18, the device copy of a host
+// call's images 8 and their FP64 sums (16 in FP32, 8 in FP64).
 int64_t born_seg_start(const BornPlan& p, int64_t ncoarse, int64_t s) {
   return std::max<int64_t>(0, ncoarse - (p.S - s) * p.K);
 }
 
-int64_t born_fixed_arrays(const ela_handle* h) { return 8 + 18 + 36 + 18 + 8 + (h->esize == 4 ? 16 : 0); }
+int64_t born_fixed_arrays(const ela_handle* h) { return 8 + 18 + 36 + 18 + 8 + (h->esize == 4 ? 16 : 8); }
 
 int born_plan(ela_handle* h, BornPlan& p) {
   const int64_t nts = h->cfg.nts, ncoarse = nts - 1;
@@ -1280,7 +1281,6 @@ int born_forward_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
   Wave<T> bg = wave_ptrs<T>(h->wave, np), sc = wave_ptrs<T>(h->wave2, np);
   CHK(fill<T>(h, h->wave.p, 18 * np));
   CHK(fill<T>(h, h->wave2.p, 18 * np));
-  CHK(fill<T>(h, h->ss.p, 18 * np));
   CHK(fill<T>(h, ring, 4 * 3 * np));
   CHK(fill<T>(h, tm, nrec_tot * nts));
   const double* f = h->filt.data();
@@ -1392,7 +1392,7 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
 
   // adjoint sweep
   CHK(fill<T>(h, h->wave2.p, 36 * np));
-  CHK(fill<T>(h, h->ss.p, 18 * np));
+  CHK(fill<T>(h, ssR[0], 9 * np));   // ssL is written before it is read
   auto adjoint_step = [&](int64_t its) -> int {
     bool first = true;   // ssL holds nothing of this coarse sample yet
     for (int64_t it2 = sub - 1; it2 >= 0; --it2) {
@@ -1418,7 +1418,8 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
       }
       ad.swap();
     }
-    launch_imaging<T, true>(h, imaging_args<T>(h, V(its), V(its + 1), V(its + 2), its + 1, nullptr, dm, ssR));
+    launch_imaging<T, true>(h, imaging_args<T>(h, V(its), V(its + 1), V(its + 2), its + 1, nullptr, dm, ssR,
+                                                its == nts - 2));
     for (int k = 0; k < 9; ++k) std::swap(ssL[k], ssR[k]);
     steps += sub;
     return ELA_OK;
@@ -1452,6 +1453,9 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
   return ELA_OK;
 }
 
+template <typename T, typename U>
+void add_out(ela_handle* h, const double* acc, const T* part, U* out);
+
 template <typename T>
 int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, const void* dmod_in,
              void* dmod_out, const ela_points* rp_in, const ela_traces* rt_in, bool adjoint, int mem) {
@@ -1469,36 +1473,37 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
   T* rec_tr[9];
   for (int c = 0; c < 9; ++c) { src_tr[c] = (T*)ds[c]; rec_tr[c] = (T*)dr[c]; }
 
-  // perturbations (forward) / incoming images (adjoint, accumulated) in the library layout
-  CHK(h->dmod.alloc(8 * np * sizeof(T)));
+  // forward: the perturbations in the library layout (read at interior cells
+  // only); adjoint: the image to add to, the caller's or its device copy
+  if (!adjoint || mem == ELA_MEM_HOST) CHK(h->dmod.alloc(8 * np * sizeof(T)));
   T* dm = (T*)h->dmod.p;
-  CHK(fill<T>(h, dm, 8 * np));
-  CHK(copy_in_3d(h, dm, adjoint ? dmod_out : dmod_in, 8, mem));
+  const size_t img_bytes = (size_t)8 * h->n_model * sizeof(T);
+  if (!adjoint) {
+    CHK(copy_in_3d(h, dm, dmod_in, 8, mem));
+  } else if (mem == ELA_MEM_HOST) {
+    HIPCHK(hipMemcpyAsync(dm, dmod_out, img_bytes, hipMemcpyHostToDevice, h->stream));
+  } else {
+    CHK(check_dev_ptr(dmod_out, "the image"));
+    dm = (T*)dmod_out;
+  }
 
   const int64_t nrec_tot = total_points(rp);
   CHK(h->scratch_tm.alloc(std::max<int64_t>(1, nrec_tot * nts) * sizeof(T)));
   T* tm = (T*)h->scratch_tm.p;
 
   if (adjoint) launch_transpose<T, true>(h, rp, rec_tr, tm);
-  // the adjoint sums its image over every coarse sample in FP64 (FP32
-  // handles: in an FP64 copy of the incoming image, narrowed at the end)
+  // the adjoint sums its image over every coarse sample in FP64, then adds it
+  // to the caller's
   double* dm64 = nullptr;
   if (adjoint) {
-    if constexpr (sizeof(T) == 8) {
-      dm64 = reinterpret_cast<double*>(dm);
-    } else {
-      CHK(h->dmod64.alloc(8 * np * sizeof(double)));
-      dm64 = (double*)h->dmod64.p;
-      CHK(fill<double>(h, dm64, 8 * np));
-      launch(h, ela::k_fold<T>, dim3((unsigned)std::min<int64_t>((8 * np + 255) / 256, 65536)), dim3(256), dm, dm64, 8 * np);
-    }
+    CHK(h->dmod64.alloc(8 * np * sizeof(double)));
+    dm64 = (double*)h->dmod64.p;
   }
   HIPCHK(hipEventRecord(h->ev0, h->stream));
   if (!adjoint) CHK(born_forward_run<T>(h, sp, src_tr, rp, tm, nrec_tot, dm));
   else CHK(born_adjoint_run<T>(h, sp, src_tr, rp, tm, nrec_tot, dm64));
   HIPCHK(hipEventRecord(h->ev1, h->stream));
-  if (adjoint && sizeof(T) == 4)
-    launch(h, ela::k_narrow<T>, dim3((unsigned)std::min<int64_t>((8 * np + 255) / 256, 65536)), dim3(256), dm64, dm, 8 * np);
+  if (adjoint) add_out<T, T>(h, dm64, nullptr, dm);
   HIPCHK(hipGetLastError());
 
   if (!adjoint) {
@@ -1506,7 +1511,7 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
     HIPCHK(hipGetLastError());
     if (mem == ELA_MEM_HOST) CHK(stage_out_traces(h, rp_in, dr, rt_in));
   } else {
-    CHK(copy_out_3d(h, dmod_out, dm, 8, mem));
+    if (mem == ELA_MEM_HOST) HIPCHK(hipMemcpyAsync(dmod_out, dm, img_bytes, hipMemcpyDeviceToHost, h->stream));
   }
   if (mem == ELA_MEM_HOST) HIPCHK(hipStreamSynchronize(h->stream));
   return ELA_OK;
@@ -1750,25 +1755,34 @@ int grad_fwd_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_t
   return ELA_OK;
 }
 
-// g64 += g32; g32 = 0 over the 8 medium arrays: FP32 over the FD interior four
-// values per lane when the interior z extent allows it, else element-wise
+// out (caller layout, device) += the FP64 sums acc and the partial sums part
+// of 8 arrays, over the FD interior.
+template <typename T, typename U>
+void add_out(ela_handle* h, const double* acc, const T* part, U* out) {
+  Wave<T> w{};
+  const ela::CkArgs<T> a = ck_args<T>(h, w);
+  launch(h, ela::k_add_out<T, U>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 8192), 8), dim3(256), a, acc, part,
+         h->stride, out, (int)h->cfg.nz, (int)h->cfg.nx, h->n_model);
+}
+
+// g64 (+)= g32; g32 = 0 over the 8 medium arrays: FP32 over the FD interior
+// four values per lane when the interior z extent allows it, else element-wise
 // over the whole arrays.
-template <typename T>
-int fold_gradient(ela_handle* h, T* g32, double* g64) {
+template <typename T, bool FIRST>
+void fold_gradient(ela_handle* h, T* g32, double* g64) {
   const int64_t np = h->stride;
   if constexpr (sizeof(T) == 4) {
     if ((h->cfg.nz - 2 * ela::FAT) % 4 == 0) {
       Wave<T> w{};
       ela::CkArgs<T> a = ck_args<T>(h, w);
       for (int m = 0; m < 8; ++m) a.f[m] = g32 + m * np;
-      launch(h, ela::k_fold_v4, dim3((unsigned)std::min<int64_t>((a.nI / 4 + 255) / 256, 4096), 8), dim3(256), a,
+      launch(h, ela::k_fold_v4<FIRST>, dim3((unsigned)std::min<int64_t>((a.nI / 4 + 255) / 256, 4096), 8), dim3(256), a,
              g64, np);
-      return ELA_OK;
+      return;
     }
   }
   const int64_t n8 = 8 * np;
-  launch(h, ela::k_fold<T>, dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, 65536)), dim3(256), g32, g64, n8);
-  return ELA_OK;
+  launch(h, ela::k_fold<T, FIRST>, dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, 65536)), dim3(256), g32, g64, n8);
 }
 
 // Device fine-step counter of the gradient's graph replays.
@@ -1963,8 +1977,15 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   T* g32 = (T*)h->g32.p;
   double* g64 = (double*)h->g64.p;
   CHK(fill<T>(h, g32, 8 * np));
-  CHK(fill<double>(h, g64, 8 * np));
-  CHK(copy_in_3d(h, g64, grad8, 8, mem, sizeof(double)));
+  // a device call adds its sums to the caller's arrays at the end; a host
+  // call's arrays are the start of the sums
+  bool summed = mem == ELA_MEM_HOST;   // g64 holds something
+  if (mem == ELA_MEM_HOST) {
+    CHK(fill<double>(h, g64, 8 * np));
+    CHK(copy_in_3d(h, g64, grad8, 8, mem, sizeof(double)));
+  } else {
+    CHK(check_dev_ptr(grad8, "the gradient"));
+  }
   CHK(fill<T>(h, h->wave2.p, 36 * np));
   Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = wave_ptrs<T>(h->wave2, np, true);
   const double* f = h->filt.data();
@@ -2056,13 +2077,17 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
           CHK(adj_step(ad, k, drv(k - j0), drv(k - j0 + 2), pair_role(j1 - k, j1 - j0), DevStep()));
       }
       steps += 2 * (j1 - j0);
-      CHK(fold_gradient<T>(h, g32, g64));
+      if (mem == ELA_MEM_DEVICE && s1 == 0 && s2 == 0) break;   // the last partial sums go out with the rest
+      if (summed) fold_gradient<T, false>(h, g32, g64);
+      else fold_gradient<T, true>(h, g32, g64);
+      summed = true;
     }
   }
   launch_record<T>(h, make_points<T>(h, sp, ad.p1, TmViews<T>(tm_src).v, true, nsrc_tot), 0, f[0], f[hh]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   h->last_steps = steps;
-  CHK(copy_out_3d(h, grad8, g64, 8, mem, sizeof(double)));
+  if (mem == ELA_MEM_DEVICE) add_out<T, double>(h, summed ? g64 : nullptr, g32, grad8);
+  else CHK(copy_out_3d(h, grad8, g64, 8, mem, sizeof(double)));
   launch_transpose<T, false>(h, sp, gs_tr, tm_src);
   HIPCHK(hipGetLastError());
   if (mem == ELA_MEM_HOST) CHK(stage_out_traces(h, sp_in, (void* const*)gs_tr, gs_out));

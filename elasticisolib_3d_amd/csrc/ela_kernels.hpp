@@ -1350,6 +1350,7 @@ struct ImagingArgs {
   T cx[4], cy[4], cz[4];
   T dts_inv;
   int its, nts;
+  int init;         // adjoint: the images hold nothing yet (written, not read)
   int physics;      // 0: the yz term with the xz derivative pattern (reference); 1: the yz pattern
   int nz, nx, ny, nzi, zoff;
   int64_t ys;
@@ -1463,7 +1464,7 @@ __global__ void __launch_bounds__(tile_threads(S)) k_imaging(ImagingArgs<T> a) {
 #pragma unroll
         for (int k = 0; k < 9; ++k) ss[k] = *at(a.ss[k], i);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) dmo[k] = a.dmo[k][i];   // 64-bit indexing: FP64 offsets can pass 4 GiB
+        for (int k = 0; k < 8; ++k) dmo[k] = a.init ? 0.0 : a.dmo[k][i];   // 64-bit indexing: FP64 offsets can pass 4 GiB
       }
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
       const T exx = dpx<T, S>(l_vx[b], r, q, cx);
@@ -1866,7 +1867,9 @@ __global__ void __launch_bounds__(256) k_ck_unpack_s16_v8(CkArgs<float> a, const
 // interior only (the steppers and injections write nothing else): four
 // consecutive z values per lane (interior z extent a multiple of 4, rows
 // 16-byte aligned), array m = blockIdx.y of a.f (partial sums) and of acc
-// (FP64 sums, stride np); the partial sums are cleared.
+// (FP64 sums, stride np); the partial sums are cleared. FIRST: the FP64 sums
+// hold nothing yet (written, not read).
+template <bool FIRST>
 __global__ void __launch_bounds__(256) k_fold_v4(CkArgs<float> a, double* acc, int64_t np) {
   const int m = blockIdx.y;
   float* part = a.f[m];
@@ -1877,7 +1880,8 @@ __global__ void __launch_bounds__(256) k_fold_v4(CkArgs<float> a, double* acc, i
     float4* pp = reinterpret_cast<float4*>(part + o);
     double2* d = reinterpret_cast<double2*>(ac + o);
     const float4 p = *pp;
-    double2 d0 = d[0], d1 = d[1];
+    double2 d0 = make_double2(0.0, 0.0), d1 = d0;
+    if constexpr (!FIRST) { d0 = d[0]; d1 = d[1]; }
     d0.x += (double)p.x; d0.y += (double)p.y;
     d1.x += (double)p.z; d1.y += (double)p.w;
     d[0] = d0;
@@ -1886,20 +1890,33 @@ __global__ void __launch_bounds__(256) k_fold_v4(CkArgs<float> a, double* acc, i
   }
 }
 
-// out[i] = (T) in[i] (the Born adjoint's FP64 image handed back in T).
-template <typename T>
-__global__ void __launch_bounds__(256) k_narrow(const double* in, T* out, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = T(in[i]);
-}
-
-// acc[i] += (double) part[i]; part[i] = 0 (FP64 time accumulation of the
-// gradient from the per-segment partial sums).
-template <typename T>
+// acc[i] (+)= (double) part[i]; part[i] = 0 over whole arrays.
+template <typename T, bool FIRST>
 __global__ void __launch_bounds__(256) k_fold(T* part, double* acc, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    acc[i] += (double)part[i];
+    acc[i] = (FIRST ? 0.0 : acc[i]) + (double)part[i];
     part[i] = T(0);
+  }
+}
+
+// The sums of a call added to the caller's arrays [8][ny][nx][nz] over the FD
+// interior, in place: out = U(double(out) + acc (+ part)), acc the FP64 sums
+// (stride np; null: part alone), part the gradient's last partial sums (null:
+// none). Takes the place of copying the caller's arrays in, converting them,
+// adding and copying them out: Born adjoint 232x328x324 (40 steps) 77.2 ->
+// 75.5 ms, gradient 99.8 -> 98.3 ms.
+template <typename T, typename U>
+__global__ void __launch_bounds__(256) k_add_out(CkArgs<T> a, const double* acc, const T* part, int64_t np, U* out,
+                                                 int nz, int nx, int64_t n_model) {
+  const int m = blockIdx.y;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nI; q += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t q32 = (uint32_t)q, r = fdiv(q32, a.dz), iz = q32 - r * (uint32_t)a.nzI;
+    const uint32_t iy = fdiv(r, a.dx), ix = r - iy * (uint32_t)a.nxI;
+    const int64_t i = (int64_t)((iy + FAT) * (uint32_t)a.ys + (ix + FAT) * (uint32_t)a.nzi + (uint32_t)(a.zoff + FAT) + iz);
+    double s = acc ? acc[m * np + i] : 0.0;
+    if (part) s += (double)part[m * np + i];
+    U* o = out + m * n_model + ((int64_t)(iy + FAT) * nx + (ix + FAT)) * nz + FAT + iz;
+    *o = U((double)*o + s);
   }
 }
 
