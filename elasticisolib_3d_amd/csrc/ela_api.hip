@@ -219,6 +219,7 @@ struct ela_handle {
   DevBuf elastic;           // rho, lambda, mu (ela_set_elastic)
   bool have_elastic = false;  // the steppers form the medium from `elastic` (F_MED3)
   double tdt = 0.0;         // 2 dtw of ela_set_elastic
+  bool solid = false;       // the transposed steps of this call are MODE_BORN_ADJ_Q (check_solid)
   DevBuf taper;             // min_pad values
   DevBuf scratch_tm;        // time-major trace buffer
   void* scratch_dev = nullptr;  // device address of ela_scratch on cfg.device (resolved in ela_create)
@@ -553,7 +554,8 @@ template <typename T, int MODE, int FV, int FS>
 int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::PointArgs<T>& inj,
                 const ela::PointArgs<T>& rec) {
   // the premultiplied transposed steps (Born adjoint, gradient) may take a tile of their own
-  const int bx = MODE == ela::MODE_BORN_ADJ_PM && h->by_x_t ? h->by_x_t : h->by_x;
+  const bool transposed = MODE == ela::MODE_BORN_ADJ_PM || MODE == ela::MODE_BORN_ADJ_Q;
+  const int bx = transposed && h->by_x_t ? h->by_x_t : h->by_x;
   // 16 rows (1024 threads, at most 128 registers) only where the step fits:
   // FP64 and the steps with per-cell extra operands spill there (Born adjoint
   // of 232x328x324 69-97 ms with 16 rows, 60 with 4) and run 4 rows instead
@@ -576,7 +578,7 @@ int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::
 template <typename T, int MODE, int FV, int FS>
 int launch_step_m(ela_handle* h, const ela::StepArgs<T>& a, int which = 3,
                   const ela::PointArgs<T>& inj = ela::PointArgs<T>{}, const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
-  if constexpr (MODE == ela::MODE_FWD || MODE == ela::MODE_ADJ || MODE == ela::MODE_BORN_ADJ_PM) {
+  if constexpr (MODE != ela::MODE_BORN_ADJ) {
     if (h->have_elastic) return launch_step<T, MODE, FV | ela::F_MED3, FS | ela::F_MED3>(h, a, which, inj, rec);
   }
   return launch_step<T, MODE, FV, FS>(h, a, which, inj, rec);
@@ -652,13 +654,17 @@ bool fuse_injection(const ela_handle* h, const DevPoints& p, const int* box) {
              tiles(box[4], box[5], h->ychunk) <= 1024;
 }
 
-// Copies (host) or reads (device) the caller's int64 positions, converts them
-// to internal int32 offsets on the GPU and checks that every point lies in the
-// FD interior.
+// The device's answer of k_check_solid about the medium that is set.
+int* fluid_flag(ela_handle* h) { return static_cast<int*>(h->counter.p) + 8; }
+
 // Bytes of scratch that convert_points uses for `total` points of a
 // device-memory call (int32 positions and the flag).
 size_t point_scratch_bytes(int64_t total) { return (size_t)round_up(total * 4, 256) + 256; }
 
+// Copies (host) or reads (device) the caller's int64 positions, converts them
+// to internal int32 offsets on the GPU and checks that every point lies in the
+// FD interior.
+// Fetches the answer of k_check_solid too.
 int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, int mem, DevPoints& ds, DevPoints& dr,
                    void* scratch = nullptr) {
   int64_t total = 0;
@@ -677,7 +683,7 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   int64_t* s64 = (int64_t*)base;
   int32_t* s32 = (int32_t*)(base + b64);
   int* flag = (int*)(base + b64 + b32);
-  launch(h, ela::k_fill<int>, dim3(1), dim3(64), flag, (int64_t)64, 0);  // flag[0]; boxes at 8 and 16
+  launch(h, ela::k_clear_flags, dim3(1), dim3(64), flag, fluid_flag(h));  // flag[0]; boxes at 8 and 16
   if (mem == ELA_MEM_HOST && total) {
     char* pin = h->pinned.room((size_t)total * 8);
     int64_t off = 0;
@@ -719,6 +725,7 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   int host[24];
   HIPCHK(hipMemcpyAsync(host, flag, sizeof(host), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
+  h->solid = !host[1];
   ds.fuse = ds.box && fuse_injection(h, ds, host + 8);
   dr.fuse = dr.box && fuse_injection(h, dr, host + 16);
   if (host[0]) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
@@ -795,7 +802,7 @@ int step_with_points(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& 
   if (ip.fuse || inj.off[9] == 0) return ELA_OK;
   const unsigned nb = (unsigned)((inj.off[9] + 255) / 256);
   launch(h, ela::k_inject<T, ((FV | FS) & ela::F_ACC) != 0, ((FV | FS) & ela::F_GRAD) != 0,
-                          MODE == ela::MODE_BORN_ADJ_PM>, dim3(nb), dim3(256), inj);
+                          MODE == ela::MODE_BORN_ADJ_PM || MODE == ela::MODE_BORN_ADJ_Q>, dim3(nb), dim3(256), inj);
   return ELA_OK;
 }
 
@@ -947,18 +954,63 @@ Wave<T> wave_ptrs(DevBuf& b, int64_t stride, bool premultiplied = false) {
   return w;
 }
 
-// Premultiplied Born-adjoint step arguments: read M c from q1, write M n to q0.
+// The transposed wavefield of the Born adjoint and the gradient. The steppers
+// take derivatives of M n, so the general steps write it beside n and read both
+// levels of both (MODE_BORN_ADJ_PM, 36 arrays). The sponge being a scalar, q =
+// M n follows the recursion q' = w (w q - M D c) by itself. On a solid medium
+// (check_solid) the velocities and shear stresses, whose M is one factor, hold
+// q alone, and n = q / M where it is accumulated, imaged or recorded
+// (MODE_BORN_ADJ_Q, 24 arrays): a step touches 6 arrays less (39 -> 33 without,
+// 73 -> 67 with two levels imaged): Born adjoint 232x328x324 80.6 -> 75.7 ms per
+// 80 steps, gradient 101.7 -> 95.3 ms, FP64 gradient 88x97x90 11.4 -> 10.8 ms. The
+// normal stresses keep both: q alone is 3 to 4 % faster still, but the inverse
+// of their 3 x 3 block enlarges q's roundings by (3 lambda + 2 mu) / 2 mu, up to
+// 1.8 times the FP32 error at Vp / Vs = 4; as it is the error is the same.
 template <typename T>
-void set_pm(ela_handle* h, ela::StepArgs<T>& a, const Wave<T>& w) {
-  a.q = w.q1[0];
-  a.qn = w.q0[0];
-  (void)h;
+Wave<T> adj_wave(ela_handle* h) {
+  if (!h->solid) return wave_ptrs<T>(h->wave2, h->stride, true);
+  Wave<T> w{};
+  for (int k = 0; k < 9; ++k) {
+    w.q0[k] = arr<T>(h->wave2, h->stride, k);
+    w.q1[k] = arr<T>(h->wave2, h->stride, 9 + k);
+  }
+  for (int k = 0; k < 3; ++k) {
+    w.p0[ela::SXX + k] = arr<T>(h->wave2, h->stride, 18 + k);
+    w.p1[ela::SXX + k] = arr<T>(h->wave2, h->stride, 21 + k);
+  }
+  return w;
 }
 
+int64_t adj_arrays(const ela_handle* h) { return h->solid ? 24 : 36; }
+
+// Step arguments: reads M c from q1, writes M n to q0 and n to p0.
 template <typename T>
-void set_pm(ela_handle* h, ela::PointArgs<T>& a, const Wave<T>& w) {
-  for (int k = 0; k < 9; ++k) a.q[k] = w.q0[k];
+ela::StepArgs<T> adj_args(ela_handle* h, Wave<T>& w) {
+  ela::StepArgs<T> a = h->solid ? base_args<T>(h, w.q0, w.q1) : base_args<T>(h, w.p0, w.p1);
+  if (h->solid) {
+    a.qn = w.p0[ela::SXX];
+  } else {
+    a.q = w.q1[0];
+    a.qn = w.q0[0];
+  }
+  return a;
+}
+
+// Points of the level (p, q) of the transposed wavefield.
+template <typename T>
+ela::PointArgs<T> adj_points(ela_handle* h, const DevPoints& pts, T* const p[9], T* const q[9], T* tm, int64_t n) {
+  T* const tr[9] = {tm, tm, tm, tm, tm, tm, tm, tm, tm};
+  ela::PointArgs<T> a = make_points<T>(h, pts, p, tr, true, n);
+  for (int k = 0; k < 9; ++k) a.q[k] = q[k];
   for (int k = 0; k < 8; ++k) a.m[k] = arr<T>(h->med, h->stride, k);
+  return a;
+}
+
+template <typename T, int FV, int FS>
+int adj_launch(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& rp, const ela::PointArgs<T>& inj,
+               const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
+  if (h->solid) return step_with_points<T, ela::MODE_BORN_ADJ_Q, FV, FS>(h, a, rp, inj, rec);
+  return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, a, rp, inj, rec);
 }
 
 // The 9 components of a time-major trace buffer share one base pointer
@@ -1218,9 +1270,10 @@ struct BornPlan {
 // the last segment's V slices in the window, where the adjoint sweep starts.
 
 // Arrays (of h->stride elements) the Born adjoint needs besides V and the
-// checkpoints: medium 8, background wavefield 18, adjoint wavefield with its
-// premultiplied levels 36, secondary sources 18, the device copy of a host
-// call's images 8 and their FP64 sums (16 in FP32, 8 in FP64).
+// checkpoints: medium 8, background wavefield 18, adjoint wavefield 36 (a
+// solid medium's takes 24; the plan does not depend on it), secondary sources
+// 18, the device copy of a host call's images 8 and their FP64 sums (16 in
+// FP32, 8 in FP64).
 int64_t born_seg_start(const BornPlan& p, int64_t ncoarse, int64_t s) {
   return std::max<int64_t>(0, ncoarse - (p.S - s) * p.K);
 }
@@ -1337,14 +1390,14 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
   }
   CHK(h->ckpt.alloc(ck_bytes));
   CHK(h->coarse.alloc(v_bytes));
-  CHK(h->wave2.alloc(36 * np * sizeof(T)));
+  CHK(h->wave2.alloc(adj_arrays(h) * np * sizeof(T)));
   CHK(h->ss.alloc(18 * np * sizeof(T)));
   T* pool = (T*)h->coarse.p;
   T* ck = (T*)h->ckpt.p;
   T* ssL[9];
   T* ssR[9];
   for (int k = 0; k < 9; ++k) { ssL[k] = arr<T>(h->ss, np, k); ssR[k] = arr<T>(h->ss, np, 9 + k); }
-  Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = wave_ptrs<T>(h->wave2, np, true);
+  Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = adj_wave<T>(h);
   const double* f = h->filt.data();
   int64_t steps = 0;
 
@@ -1391,19 +1444,17 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
   }
 
   // adjoint sweep
-  CHK(fill<T>(h, h->wave2.p, 36 * np));
+  CHK(fill<T>(h, h->wave2.p, adj_arrays(h) * np));
   CHK(fill<T>(h, ssR[0], 9 * np));   // ssL is written before it is read
   auto adjoint_step = [&](int64_t its) -> int {
     bool first = true;   // ssL holds nothing of this coarse sample yet
     for (int64_t it2 = sub - 1; it2 >= 0; --it2) {
-      ela::StepArgs<T> a = base_args<T>(h, ad.p0, ad.p1);
-      set_pm<T>(h, a, ad);
-      ela::PointArgs<T> R = make_points<T>(h, rp, ad.p0, TmViews<T>(tm).v, true, nrec_tot);
-      set_pm<T>(h, R, ad);
+      ela::StepArgs<T> a = adj_args<T>(h, ad);
+      ela::PointArgs<T> R = adj_points<T>(h, rp, ad.p0, ad.q0, tm, nrec_tot);
       set_time(R, (int)its, f[it2 + 1], f[hh + it2 + 1]);
       const int role = pair_role(sub - it2, sub);
       if (role == 0) {
-        CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, a, rp, R)));
+        CHK((adj_launch<T, 0, 0>(h, a, rp, R)));
       } else {
         a.accl = ssL[0];
         a.accr = ssR[0];
@@ -1414,7 +1465,7 @@ int born_adjoint_run(ela_handle* h, const DevPoints& sp, T* const src_tr[9], con
         first = false;
         for (int k = 0; k < 9; ++k) { R.accl[k] = ssL[k]; R.accr[k] = ssR[k]; }
         R.accfl = a.accfl; R.accfr = a.accfr;
-        CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_ACC, ela::F_ACC>(h, a, rp, R)));
+        CHK((adj_launch<T, ela::F_ACC, ela::F_ACC>(h, a, rp, R)));
       }
       ad.swap();
     }
@@ -1971,7 +2022,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   CHK(h->drv.alloc((size_t)plan.K * plan.drv_bytes));
   CHK(h->g32.alloc((size_t)8 * np * sizeof(T)));
   CHK(h->g64.alloc((size_t)8 * np * sizeof(double)));
-  CHK(h->wave2.alloc((size_t)36 * np * sizeof(T)));
+  CHK(h->wave2.alloc((size_t)adj_arrays(h) * np * sizeof(T)));
   // derivative combinations of inner step kk of a segment
   auto drv = [&](int64_t kk) { return DrvSlot{(char*)h->drv.p + kk * plan.drv_bytes, plan.dfmt}; };
   T* g32 = (T*)h->g32.p;
@@ -1986,8 +2037,8 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   } else {
     CHK(check_dev_ptr(grad8, "the gradient"));
   }
-  CHK(fill<T>(h, h->wave2.p, 36 * np));
-  Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = wave_ptrs<T>(h->wave2, np, true);
+  CHK(fill<T>(h, h->wave2.p, adj_arrays(h) * np));
+  Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = adj_wave<T>(h);
   const double* f = h->filt.data();
   const float* scales = (const float*)h->ckscale.p;
   int64_t steps = 0;
@@ -1997,12 +2048,10 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   // combinations of the one it replaces
   auto adj_step = [&](Wave<T>& av, int64_t k, DrvSlot d, DrvSlot d2, int role, DevStep ds) -> int {
     const int its = (int)(k / sub), i2 = (int)(k % sub);
-    ela::StepArgs<T> a = base_args<T>(h, av.p0, av.p1);
-    set_pm<T>(h, a, av);
-    ela::PointArgs<T> R = make_points<T>(h, rp, av.p0, TmViews<T>(tm_adj).v, true, nrec_tot);
-    set_pm<T>(h, R, av);
+    ela::StepArgs<T> a = adj_args<T>(h, av);
+    ela::PointArgs<T> R = adj_points<T>(h, rp, av.p0, av.q0, tm_adj, nrec_tot);
     // the level step k reads, which step k + 1 left (none before the first)
-    ela::PointArgs<T> S = make_points<T>(h, sp, av.p1, TmViews<T>(tm_src).v, true, nsrc_tot);
+    ela::PointArgs<T> S = adj_points<T>(h, sp, av.p1, av.q1, tm_src, nsrc_tot);
     if (ds.k) { set_step(h, R, ds.k, ds.off, 1); set_step(h, S, ds.k, ds.off + 1, 0); }
     S.nmax = (int)N;
     set_time(R, its, f[i2 + 1], f[hh + i2 + 1]);
@@ -2010,7 +2059,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
     set_time(S, (int)(kr / sub), f[ir], f[hh + ir]);
     if (!ds.k && k == N - 1) S.off[9] = 0;
     if (role == 0) {
-      CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, a, rp, R, S)));
+      CHK((adj_launch<T, 0, 0>(h, a, rp, R, S)));
     } else {
       set_drv<T>(h, a, d, false);
       if (role == 2) set_drv_pair<T>(h, a, d2);
@@ -2021,8 +2070,8 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
       }
       for (int m = 0; m < 8; ++m) R.grad[m] = g32 + m * np;
       constexpr int FQ = sizeof(T) == 4 ? ela::F_GRAD | ela::F_Q16 : ela::F_GRAD;
-      if (d.fmt == ELA_CK_S16) CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, FQ, FQ>(h, a, rp, R, S)));
-      else CHK((step_with_points<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, a, rp, R, S)));
+      if (d.fmt == ELA_CK_S16) CHK((adj_launch<T, FQ, FQ>(h, a, rp, R, S)));
+      else CHK((adj_launch<T, ela::F_GRAD, ela::F_GRAD>(h, a, rp, R, S)));
     }
     if (ds.advance) launch(h, ela::k_count, dim3(1), dim3(64), ds.k, ds.advance);
     av.swap();
@@ -2083,7 +2132,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
       summed = true;
     }
   }
-  launch_record<T>(h, make_points<T>(h, sp, ad.p1, TmViews<T>(tm_src).v, true, nsrc_tot), 0, f[0], f[hh]);
+  launch_record<T>(h, adj_points<T>(h, sp, ad.p1, ad.q1, tm_src, nsrc_tot), 0, f[0], f[hh]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   h->last_steps = steps;
   if (mem == ELA_MEM_DEVICE) add_out<T, double>(h, summed ? g64 : nullptr, g32, grad8);
@@ -2127,19 +2176,24 @@ template <typename T>
 int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   const int64_t np = h->stride;
   const int dfmt = drv_format(h);
-  CHK(h->wave2.alloc((size_t)36 * np * sizeof(T)));
+  int fluid = 1;
+  HIPCHK(hipMemcpyAsync(&fluid, fluid_flag(h), sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipStreamSynchronize(h->stream));
+  h->solid = !fluid;
+  CHK(h->wave2.alloc((size_t)adj_arrays(h) * np * sizeof(T)));
   CHK(h->drv.alloc(drv_step_bytes(h, dfmt)));
   CHK(h->g32.alloc((size_t)8 * np * sizeof(T)));
-  CHK(fill<T>(h, h->wave2.p, 36 * np));
+  CHK(fill<T>(h, h->wave2.p, adj_arrays(h) * np));
   CHK(fill<T>(h, h->g32.p, 8 * np));
   CHK(fill<float>(h, h->drv.p, (int64_t)drv_step_bytes(h, dfmt) / 4));  // a multiple of 4 bytes
-  Wave<T> w = wave_ptrs<T>(h->wave, np), ad = wave_ptrs<T>(h->wave2, np, true);
+  Wave<T> w = wave_ptrs<T>(h->wave, np), ad = adj_wave<T>(h);
+  const DevPoints none{};
+  const ela::PointArgs<T> nopts{};
   const DrvSlot slot{(char*)h->drv.p, dfmt};
   ela::StepArgs<T> f = base_args<T>(h, w.p0, w.p1);
   ela::StepArgs<T> r = base_args<T>(h, w.p0, w.p1);
   set_drv<T>(h, r, slot, true);
-  ela::StepArgs<T> g = base_args<T>(h, ad.p0, ad.p1);
-  set_pm<T>(h, g, ad);
+  ela::StepArgs<T> g = adj_args<T>(h, ad);
   set_drv<T>(h, g, slot, false);
   g.grad = (T*)h->g32.p;
   constexpr int FQS = sizeof(T) == 4 ? ela::F_STORE | ela::F_Q16 : ela::F_STORE;
@@ -2154,9 +2208,9 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
       if (dfmt == ELA_CK_S16) return launch_step_m<T, ela::MODE_FWD, FQS, FQS>(h, r);
       return launch_step_m<T, ela::MODE_FWD, ela::F_STORE, ela::F_STORE>(h, r);
     }
-    if (!image) return launch_step_m<T, ela::MODE_BORN_ADJ_PM, 0, 0>(h, g);
-    if (dfmt == ELA_CK_S16) return launch_step_m<T, ela::MODE_BORN_ADJ_PM, FQG, FQG>(h, g);
-    return launch_step_m<T, ela::MODE_BORN_ADJ_PM, ela::F_GRAD, ela::F_GRAD>(h, g);
+    if (!image) return adj_launch<T, 0, 0>(h, g, none, nopts);
+    if (dfmt == ELA_CK_S16) return adj_launch<T, FQG, FQG>(h, g, none, nopts);
+    return adj_launch<T, ela::F_GRAD, ela::F_GRAD>(h, g, none, nopts);
   };
   for (int k = 0; k < 3; ++k) {
     CHK(step(k));  // warm caches and code
@@ -2169,6 +2223,24 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
     HIPCHK(hipEventElapsedTime(&t, h->ev0, h->ev1));
     ms3[k] = t / n;
   }
+  HIPCHK(hipGetLastError());
+  return ELA_OK;
+}
+
+// Whether the transposed steps may divide by M (adj_wave): every buoyancy and
+// shear modulus of the interior is positive, the shear moduli at least 2^-20 of
+// lamb2MuDtw (in a fluid M n says nothing of a shear stress n, and far below
+// that it may underflow).
+// The answer about the 8 scaled arrays stays on the device (a medium may be set
+// in a captured graph); convert_points fetches it with its own flag.
+template <typename T>
+int check_solid(ela_handle* h) {
+  Wave<T> w{};
+  ela::CkArgs<T> a = ck_args<T>(h, w);
+  for (int k = 0; k < 8; ++k) a.f[k] = arr<T>(h->med, h->stride, k);
+  launch(h, ela::k_fill<int>, dim3(1), dim3(64), fluid_flag(h), (int64_t)1, 0);
+  launch(h, ela::k_check_solid<T>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 4096)), dim3(256), a,
+         fluid_flag(h));
   HIPCHK(hipGetLastError());
   return ELA_OK;
 }
@@ -2204,7 +2276,7 @@ int set_elastic(ela_handle* h, const void* rlm3, double dtw, int mem) {
   const int64_t n = h->cfg.nz * h->cfg.nx * h->cfg.ny;
   launch(h, ela::k_scale_medium<T>, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1 << 20)), dim3(256), a);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(h->stream));
+  CHK(check_solid<T>(h));
   h->tdt = 2.0 * dtw;
   return ELA_OK;
 }
@@ -2364,7 +2436,7 @@ int ela_set_medium(ela_handle* h, const void* med8, int mem) {
     if (!h || !med8) return fail(ELA_ERR_ARG, "null argument");
     DeviceGuard dg(h->cfg.device);
     CHK(copy_in_3d(h, h->med.p, med8, 8, mem));
-    HIPCHK(hipStreamSynchronize(h->stream));
+    CHK(h->esize == 4 ? check_solid<float>(h) : check_solid<double>(h));
     h->have_medium = true;
     h->have_elastic = false;   // the steppers read these 8 arrays
     h->grad_ready = false;

@@ -52,7 +52,8 @@ enum { BX_ = 0, BY_, BZ_, L2M, LAM, MXZ, MXY, MYZ };
 enum { MODE_FWD = 0,       // n = w(w o + M D c)        stepFwdGpu_3D
        MODE_ADJ = 1,       // n = w(w o - M D c)        stepAdjGpu_3D
        MODE_BORN_ADJ = 2,  // n = w(w o - D (M c))      stepAdjGpuBorn_3D
-       MODE_BORN_ADJ_PM = 3  // the same with M c read premultiplied (q) and M n written (qn)
+       MODE_BORN_ADJ_PM = 3, // the same with M c read premultiplied (q) and M n written (qn)
+       MODE_BORN_ADJ_Q = 4   // the same on q = M n alone but for the normal stresses: q' = w(w q - M D c) (adj_wave)
 };
 
 // Optional work fused into a stepper launch (bit flags).
@@ -100,7 +101,7 @@ struct StepArgs {
   const T* drv;         // F_GRAD: the same combinations stored by the matching forward step
   T* grad;              // F_GRAD: gradient accumulators, one per medium array
   const T* q;           // MODE_BORN_ADJ_PM: M c of the current level
-  T* qn;                // MODE_BORN_ADJ_PM: M n of the new level (written)
+  T* qn;                // MODE_BORN_ADJ_PM: M n of the new level (written); MODE_BORN_ADJ_Q: n of the 3 normal stresses
   const T* ep;          // F_MED3: rho, lambda, mu
   int16_t* dq16;        // F_Q16: int16 derivative combinations (written by F_STORE, read by F_GRAD)
   float* dqs;           // F_Q16: their scales, one per DQ_BLOCK elements
@@ -566,7 +567,7 @@ __device__ __forceinline__ void inject_point(const PA& a, int c, int64_t k) {
     return taper * fma(tr[(int64_t)its * a.tr_stride_t], fa, tr[(int64_t)(its + 1) * a.tr_stride_t] * fb);
   };
   const T v = injected(c);
-  a.field[c][p] += v;
+  if (!PM || a.field[c]) a.field[c][p] += v;  // MODE_BORN_ADJ_Q: the normal stresses alone hold n
   if (ACC && a.accl[c]) {
     a.accl[c][p] += v * a.accfl;
     a.accr[c][p] += v * a.accfr;
@@ -607,6 +608,15 @@ __device__ __forceinline__ void inject_point(const PA& a, int c, int64_t k) {
   }
 }
 
+// n = M^-1 q of a velocity or shear component of MODE_BORN_ADJ_Q. Not
+// contracted with what forms m, so that a loaded medium and one formed in the
+// step give the same bits.
+template <typename T>
+__device__ __forceinline__ T level_of(T q, T m) {
+#pragma clang fp contract(off)
+  return q * (T(1) / m);
+}
+
 // tr[its] += field[pos] fa ; tr[its+1] += field[pos] fb
 // (ker_record_interp_data_* / ker_record_source_*, kernelsElaGpu_3D.cu:61-104).
 template <typename T>
@@ -616,10 +626,11 @@ __device__ __forceinline__ void record_point(const PointArgs<T>& a, int64_t g) {
   const int64_t k = g - a.off[c];
   const int32_t p = a.pos[c][k];
   if (p < 0) return;
-  const T v = a.field[c][p];
   int its;
   T fa, fb;
   if (!point_time<T>(a, its, fa, fb)) return;
+  // MODE_BORN_ADJ_Q holds no n of the velocities and shear stresses
+  const T v = a.field[c] ? a.field[c][p] : level_of(a.q[c][p], a.m[c < 3 ? c : MXZ + (c - SXZ)][p]);
   T* tr = a.tr[c] + k * a.tr_stride_pt;
   T& t0 = tr[(int64_t)its * a.tr_stride_t];
   T& t1 = tr[(int64_t)(its + 1) * a.tr_stride_t];
@@ -752,14 +763,14 @@ __device__ __forceinline__ void normal_moduli(T tdt, double tdt64, T lam, T mu, 
 template <typename T, int S, int MODE, int F>
 __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
                                                VelLds<T, S, (F & F_MED3) != 0>& L) {
+  constexpr bool PREMULT = MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q;  // injections go into M n too
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
   static_assert(!QS || (!SS && !ACC && (F & F_GRAD) == 0 && MODE == MODE_FWD), "F_Q16 stores: MODE_FWD recomputation");
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
-  static_assert(!MED3 || MODE == MODE_FWD || MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_PM,
-                "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
+  static_assert(!MED3 || MODE != MODE_BORN_ADJ, "MODE_BORN_ADJ reads the scaled medium");
   auto& l_xx = L.xx; auto& l_zz = L.zz; auto& l_xy = L.xy; auto& l_xz = L.xz; auto& l_yz = L.yz;
   auto& l_rho = L.rho;
   const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
@@ -869,22 +880,23 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
       // stores could alias them as far as the compiler knows, and a load
       // issued after a store waits for it); FP64 loads them where they are
       // used, which holds fewer registers (2 waves per SIMD)
-      T o3[3], m3[3], ss3[3], al3[3], ar3[3], g3[3], d3[3];
+      T o3[3], m3[3], ss3[3], al3[3], ar3[3], g3[3], d3[3], e3[3];
       auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
       auto load_acc = [&](int f) {
         al3[f] = a.accfirst == 1 ? T(0) : *at(fam(a.accl, f, np), i);
         ar3[f] = a.accfirst == 2 ? T(0) : *at(fam(a.accr, f, np), i);
-        if (a.pair) { al3[f] += o3[f] * a.acc2l; ar3[f] += o3[f] * a.acc2r; }
       };
       auto load_grad = [&](int f) {  // BX_/BY_/BZ_ == VX/VY/VZ
         g3[f] = *at(fam(a.grad, f, np), i);
         if constexpr (Q16) d3[f] = load_dq16(fam(a.dq16, f, np), fam(a.dqs, f, np / DQ_BLOCK), i);
         else d3[f] = ld_nt(fam(a.drv, f, np), i);
         if (a.pair) {
-          if constexpr (Q16) g3[f] += o3[f] * load_dq16(fam(a.dq16b, f, np), fam(a.dqsb, f, np / DQ_BLOCK), i);
-          else g3[f] += o3[f] * ld_nt(fam(a.drv2, f, np), i);
+          if constexpr (Q16) e3[f] = load_dq16(fam(a.dq16b, f, np), fam(a.dqsb, f, np / DQ_BLOCK), i);
+          else e3[f] = ld_nt(fam(a.drv2, f, np), i);
         }
       };
+      // the level n of a value of this step's arrays (MODE_BORN_ADJ_Q: they hold M n)
+      auto level = [&](T v, int f) { return MODE == MODE_BORN_ADJ_Q ? level_of(v, m3[f]) : v; };
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
         o3[f] = ld_nt(fam(a.o, f, np), i);
@@ -918,7 +930,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
       for (int f = 0; f < 3; ++f) {
         T u;
         if (MODE == MODE_FWD) u = w * o3[f] + m3[f] * s3[f];
-        else if (MODE == MODE_ADJ) u = w * o3[f] - m3[f] * s3[f];
+        else if (MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_Q) u = w * o3[f] - m3[f] * s3[f];
         else u = w * o3[f] - s3[f];
         if constexpr (!HOIST) {
           if (SS) ss3[f] = load_ss(f);
@@ -930,11 +942,18 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
         if (QS && !t.active) continue;
         st_nt(fam(a.o, f, np), i, u);
         if (MODE == MODE_BORN_ADJ_PM) st_nt(fam(a.qn, f, np), i, u * m3[f]);
-        if (ACC) {
-          *at(fam(a.accl, f, np), i) = al3[f] + u * a.accfl;
-          *at(fam(a.accr, f, np), i) = ar3[f] + u * a.accfr;
+        if (ACC || (F & F_GRAD)) {
+          const T n = level(u, f), n2 = a.pair ? level(o3[f], f) : T(0);
+          if (ACC) {
+            if (a.pair) { al3[f] += n2 * a.acc2l; ar3[f] += n2 * a.acc2r; }
+            *at(fam(a.accl, f, np), i) = al3[f] + n * a.accfl;
+            *at(fam(a.accr, f, np), i) = ar3[f] + n * a.accfr;
+          }
+          if (F & F_GRAD) {
+            if (a.pair) g3[f] += n2 * e3[f];
+            *at(fam(a.grad, f, np), i) = g3[f] + n * d3[f];
+          }
         }
-        if (F & F_GRAD) *at(fam(a.grad, f, np), i) = g3[f] + u * d3[f];
       }
     }
     if (MED3) rho_prev = l_rho[b][t.ty + 1][t.tz + 1];
@@ -947,7 +966,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
     __syncthreads();
     b ^= 1;
   }
-  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(0, VX, SXX);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, PREMULT>(0, VX, SXX);
 }
 
 // ---------------------------------------------------------------------------
@@ -971,14 +990,14 @@ struct StressStage {
 template <typename T, int S, int MODE, int F>
 __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
                                              StressLds<T, S, (F & F_MED3) != 0>& L) {
+  constexpr bool PREMULT = MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q;  // injections go into M n too
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
   static_assert(!QS || (!SS && !ACC && (F & F_GRAD) == 0 && MODE == MODE_FWD), "F_Q16 stores: MODE_FWD recomputation");
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
-  static_assert(!MED3 || MODE == MODE_FWD || MODE == MODE_ADJ || MODE == MODE_BORN_ADJ_PM,
-                "F_MED3 needs MODE_FWD, MODE_ADJ or MODE_BORN_ADJ_PM");
+  static_assert(!MED3 || MODE != MODE_BORN_ADJ, "MODE_BORN_ADJ reads the scaled medium");
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz; auto& l_mu = L.mu;
   const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
@@ -1088,53 +1107,70 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
       const uint32_t i = (uint32_t)iy * ys + (QS ? t.colu : t.col);
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
       // FP32: every per-cell operand is loaded before the first store (see velocity_block)
-      T o6[6], ss6[6], al6[6], ar6[6], g5[5], d6[6];
+      T o6[6], ss6[6], al6[6], ar6[6], g5[5], d6[6], e6[6];
       auto load_ss = [&](int f) { return *at(fam(a.ssl, f, np), i) * a.ssfl + *at(fam(a.ssr, f, np), i) * a.ssfr; };
+      T l2m = 0, lam = 0, mxz = 0, mxy = 0, myz = 0;
       auto load_acc = [&](int k) {
         const int f = SXX + k;
         al6[k] = a.accfirst == 1 ? T(0) : *at(fam(a.accl, f, np), i);
         ar6[k] = a.accfirst == 2 ? T(0) : *at(fam(a.accr, f, np), i);
-        if (a.pair) { al6[k] += o6[k] * a.acc2l; ar6[k] += o6[k] * a.acc2r; }
+      };
+      // the level n of a value v of shear stress k (MODE_BORN_ADJ_Q holds M n)
+      auto level = [&](T v, int k) {
+        if constexpr (MODE == MODE_BORN_ADJ_Q) return level_of(v, k == 3 ? mxz : k == 4 ? mxy : myz);
+        else return v;
       };
       // g5 += the image of level v with the derivative combinations d:
       // lamb2MuDtw multiplies exx, eyy, ezz in sxx, syy, szz; lambDtw the
       // other two normal strains; the shear moduli one shear strain each
-      auto image = [&](const T* v, const T* d) {
+      auto image_normal = [&](const T* v, const T* d) {
         const T l2 = v[0] * d[0] + v[1] * d[1] + v[2] * d[2];
         g5[0] += l2;
         g5[1] += (v[0] + v[1] + v[2]) * (d[0] + d[1] + d[2]) - l2;
-        g5[2] += v[3] * d[3];
-        g5[3] += v[4] * d[4];
-        g5[4] += v[5] * d[5];
       };
-      auto load_grad = [&]() {
+      auto image_shear = [&](const T* v, const T* d) {
+#pragma unroll
+        for (int k = 3; k < 6; ++k) g5[k - 1] += level(v[k], k) * d[k];
+      };
+      auto load_g = [&]() {
 #pragma unroll
         for (int m = 0; m < 5; ++m) g5[m] = *at(fam(a.grad, L2M + m, np), i);
-        if (a.pair) {
-          T e6[6];
+      };
+      auto load_e = [&]() {
 #pragma unroll
-          for (int k = 0; k < 6; ++k) {
-            if constexpr (Q16) e6[k] = load_dq16(fam(a.dq16b, SXX + k, np), fam(a.dqsb, SXX + k, np / DQ_BLOCK), i);
-            else e6[k] = ld_nt(fam(a.drv2, SXX + k, np), i);
-          }
-          image(o6, e6);
+        for (int k = 0; k < 6; ++k) {
+          if constexpr (Q16) e6[k] = load_dq16(fam(a.dq16b, SXX + k, np), fam(a.dqsb, SXX + k, np / DQ_BLOCK), i);
+          else e6[k] = ld_nt(fam(a.drv2, SXX + k, np), i);
         }
+      };
+      auto load_d = [&]() {
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
           if constexpr (Q16) d6[k] = load_dq16(fam(a.dq16, SXX + k, np), fam(a.dqs, SXX + k, np / DQ_BLOCK), i);
           else d6[k] = ld_nt(fam(a.drv, SXX + k, np), i);
         }
       };
+      // the arrays of the level that is replaced
+      auto level_at = [&](int k) {
+        return MODE == MODE_BORN_ADJ_Q && k < 3 ? fam(a.qn, k, np) : fam(a.o, SXX + k, np);
+      };
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
-        o6[k] = ld_nt(fam(a.o, SXX + k, np), i);
+        o6[k] = ld_nt(level_at(k), i);
         if constexpr (HOIST) {
           if (SS) ss6[k] = load_ss(SXX + k);
           if (ACC) load_acc(k);
         }
       }
-      if constexpr (HOIST && (F & F_GRAD) != 0) load_grad();
-      T l2m = 0, lam = 0, mxz = 0, mxy = 0, myz = 0;
+      if constexpr (HOIST && (F & F_GRAD) != 0) {
+        load_g();
+        if (a.pair) {
+          load_e();
+          image_normal(o6, e6);
+          if constexpr (MODE != MODE_BORN_ADJ_Q) image_shear(o6, e6);  // else below, with the medium
+        }
+        load_d();
+      }
       if (MED3) {
         const int rr = t.ty + 1, qq = t.tz + 1;
         const T mu_c = l_mu[b][rr][qq], mu_xm = l_mu[b][rr - 1][qq], mu_zm = l_mu[b][rr][qq - 1];
@@ -1169,18 +1205,22 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         }
       }
       T u[6];
-      if (MODE == MODE_BORN_ADJ || MODE == MODE_BORN_ADJ_PM) {
+      if (MODE == MODE_BORN_ADJ || MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q) {
         u[0] = w * o6[0] - exx;
         u[1] = w * o6[1] - eyy;
         u[2] = w * o6[2] - ezz;
-        u[3] = w * o6[3] - gxz;
-        u[4] = w * o6[4] - gxy;
-        u[5] = w * o6[5] - gyz;
       } else {
         const T sg = MODE == MODE_FWD ? T(1) : T(-1);
         u[0] = w * o6[0] + sg * (l2m * exx) + sg * (lam * (eyy + ezz));
         u[1] = w * o6[1] + sg * (l2m * eyy) + sg * (lam * (exx + ezz));
         u[2] = w * o6[2] + sg * (l2m * ezz) + sg * (lam * (exx + eyy));
+      }
+      if (MODE == MODE_BORN_ADJ || MODE == MODE_BORN_ADJ_PM) {
+        u[3] = w * o6[3] - gxz;
+        u[4] = w * o6[4] - gxy;
+        u[5] = w * o6[5] - gyz;
+      } else {
+        const T sg = MODE == MODE_FWD ? T(1) : T(-1);
         u[3] = w * o6[3] + sg * (mxz * gxz);
         u[4] = w * o6[4] + sg * (mxy * gxy);
         u[5] = w * o6[5] + sg * (myz * gyz);
@@ -1190,30 +1230,48 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         const int f = SXX + k;
         if constexpr (!HOIST) {
           if (SS) ss6[k] = load_ss(f);
-          if (ACC) load_acc(k);
         }
         T v = u[k];
         if (SS) v += ss6[k];
         v *= w;
         u[k] = v;
         if (QS && !t.active) continue;
-        st_nt(fam(a.o, f, np), i, v);
-        if (ACC) {
-          *at(fam(a.accl, f, np), i) = al6[k] + v * a.accfl;
-          *at(fam(a.accr, f, np), i) = ar6[k] + v * a.accfr;
+        st_nt(level_at(k), i, v);
+      }
+      if constexpr (ACC) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          const int f = SXX + k;
+          const T n = k < 3 ? u[k] : level(u[k], k);
+          if constexpr (!HOIST) load_acc(k);
+          if (a.pair) {
+            const T n2 = k < 3 ? o6[k] : level(o6[k], k);
+            al6[k] += n2 * a.acc2l; ar6[k] += n2 * a.acc2r;
+          }
+          *at(fam(a.accl, f, np), i) = al6[k] + n * a.accfl;
+          *at(fam(a.accr, f, np), i) = ar6[k] + n * a.accfr;
         }
       }
+      if (MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q) {
+        T* const qn = MODE == MODE_BORN_ADJ_Q ? a.o : a.qn;
+        st_nt(fam(qn, SXX, np), i, u[0] * l2m + (u[1] + u[2]) * lam);
+        st_nt(fam(qn, SYY, np), i, u[1] * l2m + (u[0] + u[2]) * lam);
+        st_nt(fam(qn, SZZ, np), i, u[2] * l2m + (u[0] + u[1]) * lam);
+      }
       if (MODE == MODE_BORN_ADJ_PM) {
-        st_nt(fam(a.qn, SXX, np), i, u[0] * l2m + (u[1] + u[2]) * lam);
-        st_nt(fam(a.qn, SYY, np), i, u[1] * l2m + (u[0] + u[2]) * lam);
-        st_nt(fam(a.qn, SZZ, np), i, u[2] * l2m + (u[0] + u[1]) * lam);
         st_nt(fam(a.qn, SXZ, np), i, u[3] * mxz);
         st_nt(fam(a.qn, SXY, np), i, u[4] * mxy);
         st_nt(fam(a.qn, SYZ, np), i, u[5] * myz);
       }
       if (F & F_GRAD) {
-        if constexpr (!HOIST) load_grad();
-        image(u, d6);
+        if constexpr (!HOIST) {
+          load_g();
+          if (a.pair) { load_e(); image_normal(o6, e6); }
+        }
+        if ((!HOIST || MODE == MODE_BORN_ADJ_Q) && a.pair) image_shear(o6, e6);
+        if constexpr (!HOIST) load_d();
+        image_normal(u, d6);
+        image_shear(u, d6);
 #pragma unroll
         for (int m = 0; m < 5; ++m) *at(fam(a.grad, L2M + m, np), i) = g5[m];
       }
@@ -1235,7 +1293,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
     __syncthreads();
     b ^= 1;
   }
-  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, MODE == MODE_BORN_ADJ_PM>(1, SXX, SYZ + 1);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, PREMULT>(1, SXX, SYZ + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1523,6 +1581,11 @@ struct ConvertArgs {
   int* box[2];             // of the sources and of the receivers, or null
 };
 
+// 64 flags of a call: [1] = *fluid (k_check_solid), the others 0 (one block of 64).
+__global__ void __launch_bounds__(64) k_clear_flags(int* flag, const int* fluid) {
+  flag[threadIdx.x] = threadIdx.x == 1 ? *fluid : 0;
+}
+
 __global__ void __launch_bounds__(256) k_convert_pos(ConvertArgs a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.off[14]) return;
@@ -1728,6 +1791,22 @@ __global__ void __launch_bounds__(256) k_scale_medium(MedArgs<T> a) {
     a.m[MXY][i] = outer(tx, tx_y, iy, a.ny) * a.tdt;
     a.m[MYZ][i] = outer(ty, ty_z, iz, a.nz) * a.tdt;
   }
+}
+
+// *fluid = 1 if any interior cell's buoyancies or shear moduli are not safely
+// divided by (see check_solid). NaN counts as such.
+template <typename T>
+__global__ void __launch_bounds__(256) k_check_solid(CkArgs<T> a, int* fluid) {
+  bool bad = false;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nI; q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t i = ck_offset(a, q);
+    const T least = a.f[L2M][i] * T(0x1p-20);
+    bool ok = least > T(0);
+    for (int k = MXZ; k <= MYZ; ++k) ok = ok && a.f[k][i] >= least;
+    for (int k = BX_; k <= BZ_; ++k) ok = ok && a.f[k][i] > T(0);
+    bad = bad || !ok;
+  }
+  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(fluid, 1);
 }
 
 // Streaming reference for the roofline: R arrays of n4 16-byte vectors are

@@ -132,3 +132,40 @@ def test_host_traces_packed_and_direct(nts):
                  (prop.nl_adjoint(P["spos"], P["rec"], P["rpos"]), prop.nl_adjoint(sp, rec, rp))]
         for host, device in pairs:
             assert all(np.array_equal(a, b.cpu().numpy()) for a, b in zip(host, device))
+
+
+# mu / (lambda + 2 mu) of the upper half: as drawn, a fluid, a soft solid, and on both sides of the rule's 2^-20
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("ratio", [None, 0.0, 0.01, 0.9e-6, 3e-6])
+def test_transposed_wavefield_kinds(precision, ratio):
+    """The transposed steps hold M n alone for the velocities and shear stresses
+    of a solid medium and n beside it otherwise: Born adjoint, gradient and
+    source gradient against the oracle on both sides of the rule, both medium
+    kinds, after a switch of the medium on one handle."""
+    g = grid(4, 4)
+    P = random_problem(g, seed=21, nsrc=2, nrec=9)
+    lam, mu = P["lam"].copy(), P["mu"].copy()
+    if ratio is not None:
+        top = np.zeros(g.shape, bool)
+        top[:, :, :NZ // 2] = True
+        p = lam + 2 * mu
+        mu = np.where(top, ratio * p, mu)
+        lam = p - 2 * mu
+    med = O.lib_scale_medium(P["rho"], lam, mu, g.dtw)
+    img = O.lib_born_adjoint(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+    g8_ref, gs_ref = O.lib_gradient(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+    prop = make_prop(g, precision)
+    prop.set_gradient_checkpoints(4, 0, "native")
+    prop.set_medium(P["med"])
+    prop.born_adjoint(P["spos"], P["src"], P["rec"], P["rpos"])
+    for kind in ("scaled", "elastic"):
+        if kind == "scaled":
+            prop.set_medium(med)
+        else:
+            prop.set_elastic(np.stack([P["rho"], lam, mu]), g.dtw)
+        out = prop.born_adjoint(P["spos"], P["src"], P["rec"], P["rpos"])
+        prop.gradient_forward(P["spos"], P["src"], P["rpos"])
+        g8, gs = prop.gradient_backward(P["spos"], P["src"], P["rpos"], P["rec"])
+        e = rel(out, img), rel(g8, g8_ref), rel(gs, gs_ref)
+        print(f"{precision} ratio {ratio} {kind}: image {e[0]:.2e} gradient {e[1]:.2e} source gradient {e[2]:.2e}", flush=True)
+        assert e[0] < 2 * TOL[precision] and e[1] < 2 * TOL[precision] and e[2] < 2 * TOL[precision]
