@@ -223,7 +223,7 @@ struct ela_handle {
   DevBuf taper;             // min_pad values
   DevBuf scratch_tm;        // time-major trace buffer
   void* scratch_dev = nullptr;  // device address of ela_scratch on cfg.device (resolved in ela_create)
-  DevBuf wave2;             // Born scattered / adjoint wavefield, 2 x 9 arrays
+  DevBuf wave2;             // Born scattered wavefield, 2 x 9 arrays, or the transposed one (adj_arrays)
   DevBuf coarse;            // Born coarse-time vx, vy, vz slices [slot][3][stride]
   DevBuf ckpt;              // Born adjoint checkpoints [segment][21][stride]
   DevBuf ss;                // Born secondary sources 2 x 9 arrays
@@ -543,6 +543,12 @@ int launch_step_s(ela_handle* h, ela::StepArgs<T> a, int which, const ela::Point
   a.nbz = t.nbz; a.nbx = t.nbx; a.nby = t.nby;
   dim3 block(ela::WAVE, ela::tile_threads(S) / ela::WAVE);
   a.first = which & 1 ? 0 : t.nblocks;
+  // velocity tiles backwards (k_step) where four layers of y chunks, 13 arrays
+  // each, stay in the Infinity Cache. 328x472x468, 80 steps: 16-plane chunks
+  // (145 MB a layer) 142.7 ms backwards, 139.7 forwards; 8-plane chunks (75 MB)
+  // 143.7 and 137.7 (144.2 and 143.5 on another GPU). 232x328x324 (35 MB):
+  // 64.3 and 64.9
+  a.rev = 4.0 * 13 * a.ychunk * double(a.ys) * sizeof(T) <= 256.0 * (1 << 20);
   // recording blocks follow the stress blocks (a recorded step runs both halves)
   const unsigned nrec = (unsigned)((rec.off[9] + ela::tile_threads(S) - 1) / ela::tile_threads(S));
   const unsigned nb = (unsigned)(which == 3 ? 2 * t.nblocks : t.nblocks);
@@ -2146,22 +2152,21 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
 template <typename T>
 int time_kernels(ela_handle* h, int reps, double* ms_v, double* ms_s) {
   Wave<T> w = wave_ptrs<T>(h->wave, h->stride);
-  ela::StepArgs<T> a = base_args<T>(h, w.p0, w.p1);
-  float tv = 0.f, ts = 0.f;
-  CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a, 3)));  // warm caches and code
-  HIPCHK(hipEventRecord(h->ev0, h->stream));
-  for (int r = 0; r < reps; ++r) CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a, 1)));
-  HIPCHK(hipEventRecord(h->ev1, h->stream));
-  HIPCHK(hipEventSynchronize(h->ev1));
-  HIPCHK(hipEventElapsedTime(&tv, h->ev0, h->ev1));
-  HIPCHK(hipEventRecord(h->ev0, h->stream));
-  for (int r = 0; r < reps; ++r) CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, a, 2)));
-  HIPCHK(hipEventRecord(h->ev1, h->stream));
-  HIPCHK(hipEventSynchronize(h->ev1));
-  HIPCHK(hipEventElapsedTime(&ts, h->ev0, h->ev1));
+  float t[4] = {0.f, 0.f, 0.f, 0.f};   // by halves launched: velocity, stress, both
+  CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, base_args<T>(h, w.p0, w.p1), 3)));  // warm caches and code
+  for (int which = 1; which <= 3; ++which) {
+    HIPCHK(hipEventRecord(h->ev0, h->stream));
+    for (int r = 0; r < reps; ++r) {
+      CHK((launch_step_m<T, ela::MODE_FWD, 0, 0>(h, base_args<T>(h, w.p0, w.p1), which)));
+      w.swap();   // as in a propagation: what stays in the caches from step to step counts
+    }
+    HIPCHK(hipEventRecord(h->ev1, h->stream));
+    HIPCHK(hipEventSynchronize(h->ev1));
+    HIPCHK(hipEventElapsedTime(&t[which], h->ev0, h->ev1));
+  }
   HIPCHK(hipGetLastError());
-  *ms_v = tv / reps;
-  *ms_s = ts / reps;
+  *ms_v = double(t[3]) * t[1] / (t[1] + t[2]) / reps;
+  *ms_s = double(t[3]) * t[2] / (t[1] + t[2]) / reps;
   return ELA_OK;
 }
 

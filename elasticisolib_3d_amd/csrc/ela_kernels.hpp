@@ -126,6 +126,7 @@ struct StepArgs {
   int nbz, nbx, nby;    // tile counts along z, x, y-chunks
   int first;            // first tile of the launch: 0, or the tile count (stress blocks alone)
   int remap;            // tile order (see tile_coord)
+  int rev;              // velocity blocks run backwards through the tiles (see k_step)
   int xgroup;           // x columns per group of the y-major order
   const int* chunks;    // stacked windows: per y chunk {y0, y1, window y0, window ny, window nx}, or null
 };
@@ -326,12 +327,11 @@ __device__ __forceinline__ float load_dq16(const int16_t* q, const float* sc, ui
 // halo and queue loads are one array per field as in the forward stepper.
 //
 // The loads are not predicated: a tile's columns, halo rows and halo column
-// may lie outside the grid (past nz in the row, past nx in the plane), where
-// no interior cell's stencil reaches, so those values are never used; every
-// library array ends with a guard of GUARD_ROWS rows plus GUARD_EXTRA elements
-// past its last plane, which holds the farthest such position (at most
-// (tile_x - 1) rows plus one tile height past the array's end), so the loads
-// stay inside the allocation.
+// past the grid are clamped to its last row and column (tile_coord), where no
+// interior cell's stencil reads them. That keeps them inside the arrays and
+// makes idle lanes read lines their neighbours read anyway (unclamped, behind
+// every array's guard of GUARD_ROWS rows plus GUARD_EXTRA elements, forward
+// 152x152x148 took 5 % longer).
 template <typename T, int MODE>
 struct StressVal {
   const StepArgs<T>& a;
@@ -674,7 +674,7 @@ __device__ __forceinline__ void inject_tile(int half, int c0, int c1) {
   const auto& s = *(const ELA_KERNARG StepArgs<T>*)seg;
   const auto& a = *(const ELA_KERNARG PointArgs<T>*)(seg + sizeof(StepArgs<T>));
 #undef ELA_KERNARG
-  const int nb = s.nbz * s.nbx * s.nby, b0 = (int)blockIdx.x + s.first, bid = half ? b0 - nb : nb - 1 - b0;
+  const int nb = s.nbz * s.nbx * s.nby, b0 = (int)blockIdx.x + s.first, bid = half ? b0 - nb : s.rev ? nb - 1 - b0 : b0;
   const TileCoord t = tile_coord<S>(bid, s.nbz, s.nbx, s.nby, s.ychunk, s.nz, s.nzi, s.zoff, s.nx, s.ny, s.remap, s.xgroup, s.chunks);
   constexpr int BX = tile_x(S), BZ = tile_z(S);
   __syncthreads();
@@ -1305,12 +1305,14 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
 // order 3/2). Large grids gain only the first half's tail (232x328x324 638.7
 // -> 637.2 us, 328x472x468 1721.8 -> 1718.6 us): they are bound by HBM.
 //
-// The velocity blocks run through the tiles backwards: the stress blocks of
-// the launch before ended at the last tiles, and what they wrote and read
-// there (sigma n, v n-1, 9 of the 13 arrays a velocity block touches) is
-// still in the 256 MB Infinity Cache. Forward 328x472x468, 80 steps, 144.1
-// -> 140.2 ms, adjoint 232x328x324 64.7 -> 62.9 ms, Born adjoint 83.2 -> 78.1
-// ms; nothing at 152x152x148, which the cache does not limit.
+// With a.rev the velocity blocks run through the tiles backwards: the stress
+// blocks of the launch before ended at the last tiles, and what they wrote and
+// read there (sigma n, v n-1, 9 of the 13 arrays a velocity block touches) is
+// still in the 256 MB Infinity Cache. Adjoint 232x328x324 64.9 -> 64.3 ms in one
+// process and 64.7 -> 62.9 in another, Born adjoint 83.2 -> 78.1 ms; nothing at
+// 152x152x148, which the cache does not limit. It costs the planes that a block
+// shares with the y chunk after it, which then were read two layers of chunks
+// ago instead of just now: launch_step_s reverses where four layers fit.
 // ---------------------------------------------------------------------------
 // Waves per SIMD asked of the compiler: the FP32 steps without per-cell extra
 // operands need 115-129 VGPRs and run at 4 (at most 128); the others hold more
@@ -1331,7 +1333,7 @@ __global__ void __launch_bounds__(tile_threads(S), (step_waves<T, FV, FS>())) k_
   __shared__ Lds L;
   static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
-  if (bid < nb) velocity_block<T, S, MODE, FV>(a, inj, nb - 1 - bid, L.v);
+  if (bid < nb) velocity_block<T, S, MODE, FV>(a, inj, a.rev ? nb - 1 - bid : bid, L.v);
   else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, inj, bid - nb, L.s);
   else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
 }

@@ -396,10 +396,10 @@ int ela_get_tiling(const ela_handle* h, int* tile_x, int* y_chunk);
  * L2. */
 int ela_set_tile_order(ela_handle* h, int order, int x_group);
 
-/* Diagnostic timing: launch the velocity and the stress stencil kernels of a
- * forward fine step `reps` times each on the handle's current wavefields and
- * return the mean duration of one launch of each [ms] (HIP events on the
- * handle's stream). The wavefields are overwritten; no counterpart in the
+/* Diagnostic timing: launch the velocity half, the stress half and the whole of
+ * a forward fine step `reps` times each on the handle's current wavefields and
+ * return the mean duration of a whole step [ms], divided as the two halves
+ * take when launched alone (HIP events on the handle's stream). The wavefields are overwritten; no counterpart in the
  * reference. */
 int ela_time_step_kernels(ela_handle* h, int reps, double* ms_velocity, double* ms_stress);
 /* Mean milliseconds of the three kernel pairs of an adjoint-state gradient

@@ -169,3 +169,20 @@ def test_transposed_wavefield_kinds(precision, ratio):
         e = rel(out, img), rel(g8, g8_ref), rel(gs, gs_ref)
         print(f"{precision} ratio {ratio} {kind}: image {e[0]:.2e} gradient {e[1]:.2e} source gradient {e[2]:.2e}", flush=True)
         assert e[0] < 2 * TOL[precision] and e[1] < 2 * TOL[precision] and e[2] < 2 * TOL[precision]
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_velocity_tile_direction(precision):
+    """Velocity tiles run backwards where the layers of y chunks are small
+    and forwards where they are not (600-plane chunks): the same bits, and the
+    oracle's data, with sources in the step's blocks."""
+    g = grid(3, 4)
+    P = random_problem(g, seed=33, nsrc=5, nrec=9)
+    out = []
+    for planes in (4, 600):
+        prop = make_prop(g, precision)
+        prop.set_tiling(4, planes)
+        prop.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+        out.append(prop.nl_forward(P["spos"], P["src"], P["rpos"]))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert rel(out[0], O.lib_nl_forward(g, P["med"], P["src"], P["spos"], P["rpos"])) < TOL[precision]
