@@ -87,8 +87,8 @@ def autotune(prop, reps: int = 10, candidates: Optional[Iterable[Candidate]] = N
     """Time every candidate launch shape on `prop` (its medium must be set),
     apply the fastest and return {tile_x, y_chunk, order, x_group, ms_step,
     table}. The wavefields of the handle are overwritten. `target`
-    "forward" ranks the shapes by a forward step (velocity + stress
-    launches); "gradient" by the three kernel pairs of an adjoint-state
+    "forward" ranks the shapes by a forward step (both halves in one
+    launch); "gradient" by the three kernel pairs of an adjoint-state
     gradient step (forward, recomputation with derivative store, transposed
     step with imaging: ela_time_gradient_kernels), which do not share the
     forward's best shape: for every y chunk and block order it takes the

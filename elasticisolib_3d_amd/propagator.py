@@ -376,8 +376,9 @@ class Propagator:
         return tx.value
 
     def time_step_kernels(self, reps: int = 50):
-        """Mean launch duration [ms] of the velocity and stress stencil kernels
-        (HIP events on the handle's stream; overwrites the wavefields)."""
+        """Mean duration [ms] of a forward step's launch, divided between its
+        velocity and stress halves as they take when launched alone (HIP
+        events on the handle's stream; overwrites the wavefields)."""
         mv, ms = ctypes.c_double(), ctypes.c_double()
         self._mem_of()
         check(self.lib.ela_time_step_kernels(self.h, int(reps), ctypes.byref(mv), ctypes.byref(ms)),
