@@ -1813,13 +1813,14 @@ int grad_fwd_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_t
 }
 
 // out (caller layout, device) += the FP64 sums acc and the partial sums part
-// of 8 arrays, over the FD interior.
+// of 8 arrays, over the FD interior or the windows' interiors.
 template <typename T, typename U>
 void add_out(ela_handle* h, const double* acc, const T* part, U* out) {
   Wave<T> w{};
   const ela::CkArgs<T> a = ck_args<T>(h, w);
   launch(h, ela::k_add_out<T, U>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 8192), 8), dim3(256), a, acc, part,
-         h->stride, out, (int)h->cfg.nz, (int)h->cfg.nx, h->n_model);
+         h->stride, out, (int)h->cfg.nz, (int)h->cfg.nx, h->n_model,
+         (const int*)(h->win_y0.empty() ? nullptr : h->ytab.p));
 }
 
 // g64 (+)= g32; g32 = 0 over the 8 medium arrays: FP32 over the FD interior

@@ -1670,6 +1670,13 @@ __device__ __forceinline__ int64_t ck_offset(const CkArgs<T>& a, int64_t q) {
   return (int64_t)((iy + FAT) * (uint32_t)a.ys + (ix + FAT) * (uint32_t)a.nzi + (uint32_t)(a.zoff + FAT) + iz);
 }
 
+// Whether an interior cell of the grid lies in the interior of a window
+// (ytab: per plane {window y0, ny, nx, 0}, zeros between the windows).
+__device__ __forceinline__ bool in_window(const int* ytab, int ix, int iy) {
+  const int wy0 = ytab[4 * iy], wny = ytab[4 * iy + 1], wnx = ytab[4 * iy + 2];
+  return iy >= wy0 + FAT && iy < wy0 + wny - FAT && ix < wnx - FAT;
+}
+
 __device__ __forceinline__ uint16_t f32_to_bf16(float x) {
   uint32_t u = __float_as_uint(x);
   u += 0x7FFFu + ((u >> 16) & 1u);
@@ -1981,18 +1988,20 @@ __global__ void __launch_bounds__(256) k_fold(T* part, double* acc, int64_t n) {
 }
 
 // The sums of a call added to the caller's arrays [8][ny][nx][nz] over the FD
-// interior, in place: out = U(double(out) + acc (+ part)), acc the FP64 sums
-// (stride np; null: part alone), part the gradient's last partial sums (null:
-// none). Takes the place of copying the caller's arrays in, converting them,
+// interior (ytab: over the windows' interiors, the only cells whose sums the
+// steps write), in place: out = U(double(out) + acc (+ part)), acc the FP64
+// sums (stride np; null: part alone), part the gradient's last partial sums
+// (null: none). Takes the place of copying the caller's arrays in, converting them,
 // adding and copying them out: Born adjoint 232x328x324 (40 steps) 77.2 ->
 // 75.5 ms, gradient 99.8 -> 98.3 ms.
 template <typename T, typename U>
 __global__ void __launch_bounds__(256) k_add_out(CkArgs<T> a, const double* acc, const T* part, int64_t np, U* out,
-                                                 int nz, int nx, int64_t n_model) {
+                                                 int nz, int nx, int64_t n_model, const int* ytab) {
   const int m = blockIdx.y;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nI; q += (int64_t)gridDim.x * blockDim.x) {
     const uint32_t q32 = (uint32_t)q, r = fdiv(q32, a.dz), iz = q32 - r * (uint32_t)a.nzI;
     const uint32_t iy = fdiv(r, a.dx), ix = r - iy * (uint32_t)a.nxI;
+    if (ytab && !in_window(ytab, (int)ix + FAT, (int)iy + FAT)) continue;
     const int64_t i = (int64_t)((iy + FAT) * (uint32_t)a.ys + (ix + FAT) * (uint32_t)a.nzi + (uint32_t)(a.zoff + FAT) + iz);
     double s = acc ? acc[m * np + i] : 0.0;
     if (part) s += (double)part[m * np + i];

@@ -1,0 +1,118 @@
+"""Transposed operators on stacked windows: every window gives what it gives
+alone, and the cells outside the windows' interiors stay the caller's."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.problems import FAT, random_problem, rel
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"f64": 1e-11, "f32": 1e-5}      # twice the parity suite's bars, as for its images and gradients
+NZ, NX, NY, NTS, SUB = 27, 31, 79, 4, 4
+# first plane, planes and x columns: a gap before, between and behind, one window of the grid's width
+WINDOWS = ((1, 25, 26), (29, 21, NX), (51, 23, 22))
+
+
+def grid(nx, ny):
+    return O.Grid(nz=NZ, nx=nx, ny=ny, nts=NTS, sub=SUB, dz=10.0, dx=10.0, dy=10.0, dts=0.002, minPad=4, alphaCos=0.95)
+
+
+def make_prop(g, precision, graph=False):
+    from elasticisolib_3d_amd.propagator import Propagator
+    prop = Propagator(g.nz, g.nx, g.ny, g.nts, g.sub, g.dz, g.dx, g.dy, g.dts, g.minPad, g.alphaCos, precision)
+    prop.set_gradient_checkpoints(4, 0, "native")
+    prop.set_graph(graph)
+    return prop
+
+
+def window_problems(nrec, fluid=()):
+    """One problem per window; the upper third of the windows listed in `fluid` has mu = 0."""
+    out = []
+    for k, (_, ny, nx) in enumerate(WINDOWS):
+        g = grid(nx, ny)
+        P = random_problem(g, seed=40 + k, nsrc=2, nrec=nrec)
+        if k in fluid:
+            top = np.zeros(g.shape, bool)
+            top[:, :, :NZ // 3] = True
+            P["lam"] = np.where(top, P["lam"] + 2 * P["mu"], P["lam"])
+            P["mu"] = np.where(top, 0.0, P["mu"])
+            P["med"] = O.lib_scale_medium(P["rho"], P["lam"], P["mu"], g.dtw)
+        out.append((g, P))
+    return out
+
+
+def box(k):
+    y0, ny, nx = WINDOWS[k]
+    return np.s_[..., y0:y0 + ny, :nx, :]
+
+
+def interior():
+    m = np.zeros((NY, NX, NZ), bool)
+    for y0, ny, nx in WINDOWS:
+        m[y0 + FAT:y0 + ny - FAT, FAT:nx - FAT, FAT:NZ - FAT] = True
+    return m
+
+
+def stack(probs, key, fill):
+    a = np.full((len(probs[0][1][key]) if key == "med" else 3, NY, NX, NZ), fill)
+    for k, (_, P) in enumerate(probs):
+        a[box(k)] = P["med"] if key == "med" else np.stack([P["rho"], P["lam"], P["mu"]])
+    return a
+
+
+def stack_points(probs, key):
+    out = [[] for _ in range(7)]
+    for k, (g, P) in enumerate(probs):
+        for j in range(7):
+            y, r = np.divmod(P[key][j], g.nx * NZ)
+            x, z = np.divmod(r, NZ)
+            out[j].append(((y + WINDOWS[k][0]) * NX + x) * NZ + z)
+    return [np.concatenate(p) for p in out]
+
+
+def stack_traces(probs, key):
+    return [np.concatenate([P[key][c] for _, P in probs]) for c in range(9)]
+
+
+def set_windows(prop):
+    prop.set_windows(*zip(*WINDOWS))
+
+
+@pytest.mark.parametrize("device", [False, True])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_born_adjoint_adds_inside_the_windows_only(precision, device):
+    """A Born adjoint over the whole grid first (its sums stay in the handle's
+    buffer), then with windows onto an image that holds something: each window
+    against the oracle and, to the bit, its own propagation; every other cell,
+    the windows' own FAT layers included, as the caller left it."""
+    import torch
+    dt = np.float32 if precision == "f32" else np.float64
+    to = (lambda x, t=dt: torch.tensor(np.ascontiguousarray(x, t), device="cuda")) if device else \
+        (lambda x, t=dt: np.ascontiguousarray(x, t))
+    back = (lambda x: x.cpu().numpy()) if device else (lambda x: x)
+    probs = window_problems(nrec=5)
+    spos, rpos = stack_points(probs, "spos"), stack_points(probs, "rpos")
+    if device:
+        spos, rpos = [[torch.tensor(p, device="cuda") for p in q] for q in (spos, rpos)]
+    src, rec = [[to(t) for t in stack_traces(probs, k)] for k in ("src", "rec")]
+    full = grid(NX, NY)
+    prop = make_prop(full, precision)
+    prop.set_medium(to(random_problem(full, seed=1)["med"]))
+    prop.born_adjoint(spos, src, rec, rpos)
+    set_windows(prop)
+    prop.set_medium(to(stack(probs, "med", 1.0)))
+    # an image of whole numbers times the size of the windows' images, exact in both precisions
+    start = np.rint(np.random.default_rng(2).standard_normal((8, NY, NX, NZ)) * 8).astype(dt)
+    img = back(prop.born_adjoint(spos, src, rec, rpos, to(start.copy())))
+    out = ~interior()
+    assert np.array_equal(img[:, out], start[:, out])
+    for k, (g, P) in enumerate(probs):
+        alone = make_prop(g, precision)
+        alone.set_medium(to(P["med"]))
+        own = back(alone.born_adjoint(P["spos"], [to(t) for t in P["src"]], [to(t) for t in P["rec"]], P["rpos"],
+                                      to(start[box(k)])))
+        assert np.array_equal(img[box(k)], own)
+        ref = O.lib_born_adjoint(g, P["med"], P["src"], P["spos"], P["rec"], P["rpos"])
+        fresh = back(alone.born_adjoint(P["spos"], [to(t) for t in P["src"]], [to(t) for t in P["rec"]], P["rpos"]))
+        assert rel(fresh, ref) < TOL[precision]
