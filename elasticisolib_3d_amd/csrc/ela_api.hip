@@ -403,6 +403,14 @@ int check_points(const ela_points* p, const char* what) {
   return ELA_OK;
 }
 
+// Every component with points needs its trace array: host calls copy from and
+// to it with memcpy, device calls hand it to kernels.
+int check_traces(const ela_points* p, const ela_traces* t, const char* what) {
+  for (int c = 0; c < 9; ++c)
+    if (p->n[kCompGrid[c]] > 0 && !t->tr[c]) return fail(ELA_ERR_ARG, "%s component %d: null trace array", what, c);
+  return ELA_OK;
+}
+
 template <typename T>
 void set_coefs(const ela_handle* h, T* cx, T* cy, T* cz) {
   for (int k = 0; k < 4; ++k) {
@@ -883,6 +891,8 @@ int stage_in_traces(ela_handle* h, const ela_points* p, const ela_traces* host, 
 // (device calls) or library staging copies (host calls).
 int stage_traces(ela_handle* h, const ela_points* sp, const ela_traces* st, const ela_points* rp,
                  const ela_traces* rt, bool copy_src, bool copy_rec, int mem, void* dsrc[9], void* drec[9]) {
+  CHK(check_traces(sp, st, "source"));
+  CHK(check_traces(rp, rt, "receiver"));
   if (mem == ELA_MEM_DEVICE) {
     for (int c = 0; c < 9; ++c) {
       if (sp->n[kCompGrid[c]]) CHK(check_dev_ptr(st->tr[c], "a source trace array"));
@@ -2001,6 +2011,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   T* adj_tr[9];
   for (int c = 0; c < 9; ++c) { src_tr[c] = (T*)ds[c]; adj_tr[c] = (T*)dr[c]; }
   // source-trace gradient outputs: the caller's arrays or host-call staging
+  CHK(check_traces(sp_in, gs_out, "source gradient"));
   T* gs_tr[9];
   if (mem == ELA_MEM_DEVICE) {
     for (int c = 0; c < 9; ++c) {
