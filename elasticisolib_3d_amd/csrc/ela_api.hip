@@ -201,6 +201,19 @@ int check_dev_ptr(const void* p, const char* what) {
   return ELA_OK;
 }
 
+// Whether p is memory of GPU `dev` itself. Output sums are added by a kernel
+// in place there; memory that the GPU may reach otherwise or not at all (another
+// GPU's, pinned host, managed) is copied in and out by the runtime.
+bool own_memory(const void* p, int dev) {
+  hipPointerAttribute_t attr;
+  std::memset(&attr, 0, sizeof(attr));
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && attr.device == dev;
+}
+
 }  // namespace
 
 struct ela_handle {
@@ -227,7 +240,7 @@ struct ela_handle {
   DevBuf coarse;            // Born coarse-time vx, vy, vz slices [slot][3][stride]
   DevBuf ckpt;              // Born adjoint checkpoints [segment][21][stride]
   DevBuf ss;                // Born secondary sources 2 x 9 arrays
-  DevBuf dmod;              // Born perturbations / images, 8 arrays
+  DevBuf dmod;              // Born perturbations / images not added to in place, 8 arrays
   DevBuf dmod64;            // FP32 handles: the Born adjoint's FP64 image accumulator, 8 arrays
   DevBuf pos;               // converted positions (int32) and an error flag
   DevBuf staging;           // device copies of host-memory arguments
@@ -1542,16 +1555,17 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
 
   // forward: the perturbations in the library layout (read at interior cells
   // only); adjoint: the image to add to, the caller's or its device copy
-  if (!adjoint || mem == ELA_MEM_HOST) CHK(h->dmod.alloc(8 * np * sizeof(T)));
+  const bool in_place = adjoint && mem == ELA_MEM_DEVICE && own_memory(dmod_out, h->cfg.device);
+  if (!in_place) CHK(h->dmod.alloc(8 * np * sizeof(T)));
   T* dm = (T*)h->dmod.p;
   const size_t img_bytes = (size_t)8 * h->n_model * sizeof(T);
   if (!adjoint) {
     CHK(copy_in_3d(h, dm, dmod_in, 8, mem));
-  } else if (mem == ELA_MEM_HOST) {
-    HIPCHK(hipMemcpyAsync(dm, dmod_out, img_bytes, hipMemcpyHostToDevice, h->stream));
-  } else {
-    CHK(check_dev_ptr(dmod_out, "the image"));
+  } else if (in_place) {
     dm = (T*)dmod_out;
+  } else {
+    if (mem == ELA_MEM_DEVICE) CHK(check_dev_ptr(dmod_out, "the image"));
+    HIPCHK(hipMemcpyAsync(dm, dmod_out, img_bytes, hipMemcpyDefault, h->stream));
   }
 
   const int64_t nrec_tot = total_points(rp);
@@ -1577,8 +1591,8 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
     launch_transpose<T, false>(h, rp, rec_tr, tm);
     HIPCHK(hipGetLastError());
     if (mem == ELA_MEM_HOST) CHK(stage_out_traces(h, rp_in, dr, rt_in));
-  } else {
-    if (mem == ELA_MEM_HOST) HIPCHK(hipMemcpyAsync(dmod_out, dm, img_bytes, hipMemcpyDeviceToHost, h->stream));
+  } else if (!in_place) {
+    HIPCHK(hipMemcpyAsync(dmod_out, dm, img_bytes, hipMemcpyDefault, h->stream));
   }
   if (mem == ELA_MEM_HOST) HIPCHK(hipStreamSynchronize(h->stream));
   return ELA_OK;
@@ -2046,14 +2060,13 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   T* g32 = (T*)h->g32.p;
   double* g64 = (double*)h->g64.p;
   CHK(fill<T>(h, g32, 8 * np));
-  // a device call adds its sums to the caller's arrays at the end; a host
-  // call's arrays are the start of the sums
-  bool summed = mem == ELA_MEM_HOST;   // g64 holds something
-  if (mem == ELA_MEM_HOST) {
+  // a call on this GPU's memory adds its sums to the caller's arrays at the
+  // end; other arrays are the start of the sums
+  const bool in_place = mem == ELA_MEM_DEVICE && own_memory(grad8, h->cfg.device);
+  bool summed = !in_place;   // g64 holds something
+  if (!in_place) {
     CHK(fill<double>(h, g64, 8 * np));
     CHK(copy_in_3d(h, g64, grad8, 8, mem, sizeof(double)));
-  } else {
-    CHK(check_dev_ptr(grad8, "the gradient"));
   }
   CHK(fill<T>(h, h->wave2.p, adj_arrays(h) * np));
   Wave<T> bg = wave_ptrs<T>(h->wave, np), ad = adj_wave<T>(h);
@@ -2144,7 +2157,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
           CHK(adj_step(ad, k, drv(k - j0), drv(k - j0 + 2), pair_role(j1 - k, j1 - j0), DevStep()));
       }
       steps += 2 * (j1 - j0);
-      if (mem == ELA_MEM_DEVICE && s1 == 0 && s2 == 0) break;   // the last partial sums go out with the rest
+      if (in_place && s1 == 0 && s2 == 0) break;   // the last partial sums go out with the rest
       if (summed) fold_gradient<T, false>(h, g32, g64);
       else fold_gradient<T, true>(h, g32, g64);
       summed = true;
@@ -2153,7 +2166,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   launch_record<T>(h, adj_points<T>(h, sp, ad.p1, ad.q1, tm_src, nsrc_tot), 0, f[0], f[hh]);
   HIPCHK(hipEventRecord(h->ev1, h->stream));
   h->last_steps = steps;
-  if (mem == ELA_MEM_DEVICE) add_out<T, double>(h, summed ? g64 : nullptr, g32, grad8);
+  if (in_place) add_out<T, double>(h, summed ? g64 : nullptr, g32, grad8);
   else CHK(copy_out_3d(h, grad8, g64, 8, mem, sizeof(double)));
   launch_transpose<T, false>(h, sp, gs_tr, tm_src);
   HIPCHK(hipGetLastError());

@@ -59,3 +59,38 @@ def test_null_trace_arrays_are_refused(device):
     again = prop.nl_forward(spos, src, rpos)
     assert all((np.asarray(x.cpu() if device else x) == np.asarray(y.cpu() if device else y)).all()
                for x, y in zip(want, again))
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_outputs_in_pinned_host_memory(precision):
+    """Device-memory calls whose image and gradient lie in pinned host memory,
+    which no kernel adds to in place: the same bits as in the GPU's own memory,
+    onto what the arrays hold."""
+    import torch
+    P = random_problem(G, seed=5)
+    prop = make_prop(precision)
+    prop.set_gradient_checkpoints(2, 0, "native")
+    td = torch.float32 if precision == "f32" else torch.float64
+    dev = lambda x, t=td: torch.tensor(np.asarray(x), dtype=t, device="cuda")  # noqa: E731
+    spos, rpos = [[dev(p, torch.int64) for p in P[k]] for k in ("spos", "rpos")]
+    src, rec = [[dev(x) for x in P[k]] for k in ("src", "rec")]
+    prop.set_medium(dev(P["med"]))
+    prop.gradient_forward(spos, src, rpos)
+    mem = prop._mem_of(*src)
+    sp, rp = prop._points(spos, mem), prop._points(rpos, mem)
+    st, rt = prop._traces(src, prop._counts(spos)), prop._traces(rec, prop._counts(rpos))
+    gs = prop._alloc_traces(prop._counts(spos), True)
+    gt = prop._traces(gs, prop._counts(spos))
+    ref = ctypes.byref
+    torch.manual_seed(1)
+    held = torch.randn((8,) + G.shape, dtype=td)
+    zero = torch.zeros((8,) + G.shape, dtype=torch.float64)   # sums of several segments: equal bits from zero
+    out = []
+    for pin in (False, True):
+        img, g8 = (x.pin_memory() if pin else x.cuda() for x in (held, zero))
+        assert prop.lib.ela_born_adjoint(prop.h, ref(sp), ref(st), img.data_ptr(), ref(rp), ref(rt), mem) == 0
+        assert prop.lib.ela_gradient_backward(prop.h, ref(sp), ref(st), ref(rp), ref(rt), g8.data_ptr(), ref(gt), mem) == 0
+        torch.cuda.synchronize()
+        out.append((img.cpu(), g8.cpu()))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    assert float(out[0][1].abs().max()) > 0 and not torch.equal(out[0][0], held)
