@@ -681,19 +681,38 @@ bool fuse_injection(const ela_handle* h, const DevPoints& p, const int* box) {
              tiles(box[4], box[5], h->ychunk) <= 1024;
 }
 
-// The device's answer of k_check_solid about the medium that is set.
-int* fluid_flag(ela_handle* h) { return static_cast<int*>(h->counter.p) + 8; }
-
 // Bytes of scratch that convert_points uses for `total` points of a
 // device-memory call (int32 positions and the flag).
 size_t point_scratch_bytes(int64_t total) { return (size_t)round_up(total * 4, 256) + 256; }
 
+template <typename T>
+ela::CkArgs<T> interior_args(const ela_handle* h);
+
+// Whether the transposed steps may divide by M (adj_wave): every buoyancy and
+// shear modulus that is stepped is positive, the shear moduli at least 2^-20 of
+// lamb2MuDtw (in a fluid M n says nothing of a shear stress n, and far below
+// that it may underflow). Looked at in every transposed call (one read of the
+// medium, 0.2 ms of the 70 to 90 ms of 40 steps of 232x328x324), not when the
+// medium is set: it depends on the windows too, and a medium may be set by a
+// replayed graph.
+template <typename T>
+int check_solid(ela_handle* h, int* fluid) {
+  ela::CkArgs<T> a = interior_args<T>(h);
+  for (int k = 0; k < 8; ++k) a.f[k] = arr<T>(h->med, h->stride, k);
+  launch(h, ela::k_check_solid<T>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 4096)), dim3(256), a,
+         (const int*)(h->win_y0.empty() ? nullptr : h->ytab.p), fluid);
+  return ELA_OK;
+}
+
+int check_solid(ela_handle* h, int* fluid) {
+  return h->esize == 4 ? check_solid<float>(h, fluid) : check_solid<double>(h, fluid);
+}
+
 // Copies (host) or reads (device) the caller's int64 positions, converts them
 // to internal int32 offsets on the GPU and checks that every point lies in the
-// FD interior.
-// Fetches the answer of k_check_solid too.
+// FD interior. A transposed call asks whether the medium is solid by the way.
 int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, int mem, DevPoints& ds, DevPoints& dr,
-                   void* scratch = nullptr) {
+                   void* scratch = nullptr, bool transposed = false) {
   int64_t total = 0;
   for (int g = 0; g < 7; ++g) total += sp->n[g] + rp->n[g];
   if (mem == ELA_MEM_DEVICE)
@@ -710,7 +729,8 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   int64_t* s64 = (int64_t*)base;
   int32_t* s32 = (int32_t*)(base + b64);
   int* flag = (int*)(base + b64 + b32);
-  launch(h, ela::k_clear_flags, dim3(1), dim3(64), flag, fluid_flag(h));  // flag[0]; boxes at 8 and 16
+  CHK(fill<int>(h, flag, 64));  // flag[0] bad position, flag[1] fluid; boxes at 8 and 16
+  if (transposed) CHK(check_solid(h, flag + 1));
   if (mem == ELA_MEM_HOST && total) {
     char* pin = h->pinned.room((size_t)total * 8);
     int64_t off = 0;
@@ -1545,7 +1565,7 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
   CHK(check_points(rp_in, "receiver"));
   const int64_t nts = h->cfg.nts, np = h->stride;
   DevPoints sp, rp;
-  CHK(convert_points(h, sp_in, rp_in, mem, sp, rp));
+  CHK(convert_points(h, sp_in, rp_in, mem, sp, rp, nullptr, adjoint));
   void* ds[9];
   void* dr[9];
   CHK(stage_traces(h, sp_in, st_in, rp_in, rt_in, true, adjoint, mem, ds, dr));
@@ -1742,9 +1762,8 @@ ela::FastDiv fast_div(uint32_t d) {
 }
 
 template <typename T>
-ela::CkArgs<T> ck_args(ela_handle* h, const Wave<T>& w) {
-  ela::CkArgs<T> a;
-  for (int k = 0; k < 9; ++k) { a.f[k] = w.p0[k]; a.f[9 + k] = w.p1[k]; }
+ela::CkArgs<T> interior_args(const ela_handle* h) {
+  ela::CkArgs<T> a{};
   a.nzI = (int)(h->cfg.nz - 2 * ela::FAT);
   a.nxI = (int)(h->cfg.nx - 2 * ela::FAT);
   a.nyI = (int)(h->cfg.ny - 2 * ela::FAT);
@@ -1754,6 +1773,13 @@ ela::CkArgs<T> ck_args(ela_handle* h, const Wave<T>& w) {
   a.nI = interior_count(h);
   a.dz = fast_div((uint32_t)a.nzI);
   a.dx = fast_div((uint32_t)a.nxI);
+  return a;
+}
+
+template <typename T>
+ela::CkArgs<T> ck_args(ela_handle* h, const Wave<T>& w) {
+  ela::CkArgs<T> a = interior_args<T>(h);
+  for (int k = 0; k < 9; ++k) { a.f[k] = w.p0[k]; a.f[9 + k] = w.p1[k]; }
   return a;
 }
 
@@ -1840,8 +1866,7 @@ int grad_fwd_step(ela_handle* h, Wave<T>& w, const DevPoints& sp, T* const src_t
 // of 8 arrays, over the FD interior or the windows' interiors.
 template <typename T, typename U>
 void add_out(ela_handle* h, const double* acc, const T* part, U* out) {
-  Wave<T> w{};
-  const ela::CkArgs<T> a = ck_args<T>(h, w);
+  const ela::CkArgs<T> a = interior_args<T>(h);
   launch(h, ela::k_add_out<T, U>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 8192), 8), dim3(256), a, acc, part,
          h->stride, out, (int)h->cfg.nz, (int)h->cfg.nx, h->n_model,
          (const int*)(h->win_y0.empty() ? nullptr : h->ytab.p));
@@ -1855,8 +1880,7 @@ void fold_gradient(ela_handle* h, T* g32, double* g64) {
   const int64_t np = h->stride;
   if constexpr (sizeof(T) == 4) {
     if ((h->cfg.nz - 2 * ela::FAT) % 4 == 0) {
-      Wave<T> w{};
-      ela::CkArgs<T> a = ck_args<T>(h, w);
+      ela::CkArgs<T> a = interior_args<T>(h);
       for (int m = 0; m < 8; ++m) a.f[m] = g32 + m * np;
       launch(h, ela::k_fold_v4<FIRST>, dim3((unsigned)std::min<int64_t>((a.nI / 4 + 255) / 256, 4096), 8), dim3(256), a,
              g64, np);
@@ -2017,7 +2041,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   plan.drv_bytes = drv_step_bytes(h, plan.dfmt);
 
   DevPoints sp, rp;
-  CHK(convert_points(h, sp_in, rp_in, mem, sp, rp));
+  CHK(convert_points(h, sp_in, rp_in, mem, sp, rp, nullptr, true));
   void* ds[9];
   void* dr[9];
   CHK(stage_traces(h, sp_in, st_in, rp_in, at_in, true, true, mem, ds, dr));
@@ -2207,7 +2231,10 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   const int64_t np = h->stride;
   const int dfmt = drv_format(h);
   int fluid = 1;
-  HIPCHK(hipMemcpyAsync(&fluid, fluid_flag(h), sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  int* flag = static_cast<int*>(h->counter.p) + 8;   // behind the step counters
+  CHK(fill<int>(h, flag, 1));
+  CHK(check_solid(h, flag));
+  HIPCHK(hipMemcpyAsync(&fluid, flag, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
   h->solid = !fluid;
   CHK(h->wave2.alloc((size_t)adj_arrays(h) * np * sizeof(T)));
@@ -2257,24 +2284,6 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   return ELA_OK;
 }
 
-// Whether the transposed steps may divide by M (adj_wave): every buoyancy and
-// shear modulus of the interior is positive, the shear moduli at least 2^-20 of
-// lamb2MuDtw (in a fluid M n says nothing of a shear stress n, and far below
-// that it may underflow).
-// The answer about the 8 scaled arrays stays on the device (a medium may be set
-// in a captured graph); convert_points fetches it with its own flag.
-template <typename T>
-int check_solid(ela_handle* h) {
-  Wave<T> w{};
-  ela::CkArgs<T> a = ck_args<T>(h, w);
-  for (int k = 0; k < 8; ++k) a.f[k] = arr<T>(h->med, h->stride, k);
-  launch(h, ela::k_fill<int>, dim3(1), dim3(64), fluid_flag(h), (int64_t)1, 0);
-  launch(h, ela::k_check_solid<T>, dim3((unsigned)std::min<int64_t>((a.nI + 255) / 256, 4096)), dim3(256), a,
-         fluid_flag(h));
-  HIPCHK(hipGetLastError());
-  return ELA_OK;
-}
-
 struct DeviceGuard {
   int prev = -1;
   explicit DeviceGuard(int dev) {
@@ -2306,7 +2315,6 @@ int set_elastic(ela_handle* h, const void* rlm3, double dtw, int mem) {
   const int64_t n = h->cfg.nz * h->cfg.nx * h->cfg.ny;
   launch(h, ela::k_scale_medium<T>, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1 << 20)), dim3(256), a);
   HIPCHK(hipGetLastError());
-  CHK(check_solid<T>(h));
   h->tdt = 2.0 * dtw;
   return ELA_OK;
 }
@@ -2466,7 +2474,6 @@ int ela_set_medium(ela_handle* h, const void* med8, int mem) {
     if (!h || !med8) return fail(ELA_ERR_ARG, "null argument");
     DeviceGuard dg(h->cfg.device);
     CHK(copy_in_3d(h, h->med.p, med8, 8, mem));
-    CHK(h->esize == 4 ? check_solid<float>(h) : check_solid<double>(h));
     h->have_medium = true;
     h->have_elastic = false;   // the steppers read these 8 arrays
     h->grad_ready = false;

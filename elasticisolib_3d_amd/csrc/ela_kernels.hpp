@@ -1583,11 +1583,6 @@ struct ConvertArgs {
   int* box[2];             // of the sources and of the receivers, or null
 };
 
-// 64 flags of a call: [1] = *fluid (k_check_solid), the others 0 (one block of 64).
-__global__ void __launch_bounds__(64) k_clear_flags(int* flag, const int* fluid) {
-  flag[threadIdx.x] = threadIdx.x == 1 ? *fluid : 0;
-}
-
 __global__ void __launch_bounds__(256) k_convert_pos(ConvertArgs a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.off[14]) return;
@@ -1802,12 +1797,17 @@ __global__ void __launch_bounds__(256) k_scale_medium(MedArgs<T> a) {
   }
 }
 
-// *fluid = 1 if any interior cell's buoyancies or shear moduli are not safely
-// divided by (see check_solid). NaN counts as such.
+// *fluid = 1 if the buoyancies or shear moduli of any cell that is stepped
+// (interior cells, with ytab those of the windows) are not safely divided by
+// (see check_solid). NaN counts as such.
 template <typename T>
-__global__ void __launch_bounds__(256) k_check_solid(CkArgs<T> a, int* fluid) {
+__global__ void __launch_bounds__(256) k_check_solid(CkArgs<T> a, const int* ytab, int* fluid) {
   bool bad = false;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nI; q += (int64_t)gridDim.x * blockDim.x) {
+    if (ytab) {
+      const uint32_t r = fdiv((uint32_t)q, a.dz), iy = fdiv(r, a.dx), ix = r - iy * (uint32_t)a.nxI;
+      if (!in_window(ytab, (int)ix + FAT, (int)iy + FAT)) continue;
+    }
     const int64_t i = ck_offset(a, q);
     const T least = a.f[L2M][i] * T(0x1p-20);
     bool ok = least > T(0);

@@ -116,3 +116,47 @@ def test_born_adjoint_adds_inside_the_windows_only(precision, device):
         ref = O.lib_born_adjoint(g, P["med"], P["src"], P["spos"], P["rec"], P["rpos"])
         fresh = back(alone.born_adjoint(P["spos"], [to(t) for t in P["src"]], [to(t) for t in P["rec"]], P["rpos"]))
         assert rel(fresh, ref) < TOL[precision]
+
+
+# receivers per window and list: few (injected in the step's blocks) and many (a launch of their own)
+@pytest.mark.parametrize("nrec", [5, 70])
+@pytest.mark.parametrize("fluid", [(), (0, 1, 2)])
+@pytest.mark.parametrize("medium,graph", [("scaled", False), ("scaled", True), ("elastic", True)])
+def test_transposed_steps_of_a_stack_equal_each_window_alone(medium, graph, fluid, nrec):
+    """FP32 gradient, source gradient and Born adjoint of a stack, to the bit
+    what each window gives alone: the cells outside the windows (zeros in a
+    stack of scaled arrays) do not decide how the transposed wavefield is
+    held."""
+    probs = window_problems(nrec, fluid)
+    spos, rpos = stack_points(probs, "spos"), stack_points(probs, "rpos")
+    src, rec = stack_traces(probs, "src"), stack_traces(probs, "rec")
+
+    def run(prop, spos, src, rpos, rec):
+        data = prop.gradient_forward(spos, src, rpos)
+        g8, gs = prop.gradient_backward(spos, src, rpos, rec)
+        return data, g8, gs, prop.born_adjoint(spos, src, rec, rpos)
+
+    prop = make_prop(grid(NX, NY), "f32", graph)
+    set_windows(prop)
+    if medium == "scaled":
+        prop.set_medium(stack(probs, "med", 0.0))
+    else:
+        prop.set_elastic(stack(probs, "elastic", 1.0), probs[0][0].dtw)
+    for _ in range(2):   # a repeated call replays the kept graphs
+        data, g8, gs, img = run(prop, spos, src, rpos, rec)
+        for k, (g, P) in enumerate(probs):
+            alone = make_prop(g, "f32", graph)
+            if medium == "scaled":
+                alone.set_medium(P["med"])
+            else:
+                alone.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+            d1, g1, s1, i1 = run(alone, P["spos"], P["src"], P["rpos"], P["rec"])
+            assert all(np.array_equal(a[nrec * k:nrec * (k + 1)], b) for a, b in zip(data, d1))
+            assert all(np.array_equal(a[2 * k:2 * (k + 1)], b) for a, b in zip(gs, s1))
+            inner = np.s_[:, FAT:-FAT, FAT:-FAT, FAT:-FAT]
+            assert np.array_equal(g8[box(k)][inner], g1[inner])
+            assert np.array_equal(img[box(k)][inner], i1[inner])
+            ref, sref = O.lib_gradient(g, P["med"], P["src"], P["spos"], P["rec"], P["rpos"])
+            assert rel(g1, ref) < TOL["f32"] and rel(s1, sref) < TOL["f32"]
+    out = ~interior()
+    assert not np.any(g8[:, out]) and not np.any(img[:, out])
