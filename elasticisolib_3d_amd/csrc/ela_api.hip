@@ -232,7 +232,11 @@ struct ela_handle {
   DevBuf elastic;           // rho, lambda, mu (ela_set_elastic)
   bool have_elastic = false;  // the steppers form the medium from `elastic` (F_MED3)
   double tdt = 0.0;         // 2 dtw of ela_set_elastic
-  bool solid = false;       // the transposed steps of this call are MODE_BORN_ADJ_Q (check_solid)
+  // form of the transposed steps of this call (check_solid, adj_wave)
+  bool solid = false;       // MODE_BORN_ADJ_Q everywhere
+  bool mixed = false;       // MODE_BORN_ADJ_Q in the solid windows of a stack, MODE_BORN_ADJ_PM in the others
+  std::vector<int> win_fluid;           // per window (one entry without windows): not solid
+  const int* win_fluid_dev = nullptr;   // the same on the device
   DevBuf taper;             // min_pad values
   DevBuf scratch_tm;        // time-major trace buffer
   void* scratch_dev = nullptr;  // device address of ela_scratch on cfg.device (resolved in ela_create)
@@ -276,9 +280,10 @@ struct ela_handle {
   int plan_fmt = 0;
   // windows stacked along y (several shots in one grid)
   std::vector<int64_t> win_y0, win_ny, win_nx;
-  DevBuf ytab;              // per plane {window y0, ny, nx, 0} (int32)
+  DevBuf ytab;              // per plane {window y0, ny, nx, window} (int32)
   DevBuf chunks;            // per y chunk {y0, y1, window y0, ny, nx, 0, 0, 0} (int32)
   int chunks_yc = 0;        // y chunk the table was built for
+  std::vector<int> chunks_fluid;   // window kinds its two further parts were built for (ensure_chunks)
   int nchunks = 0;
   // graph replays of the time loops (ela_set_graph): the coarse step of the
   // nonlinear propagations, the fine-step pairs and checkpoint segments of the
@@ -439,22 +444,29 @@ struct Tiles {
 
 // Chunk table of the stacked windows for the current y chunk (rebuilt when
 // the y chunk changes; a synchronous upload, done before any launch of the
-// propagation that uses it).
+// propagation that uses it). For a stack of solid and fluid windows two more
+// tables follow, of as many rows: the first with the solid windows' rows, the
+// second with the others', the remaining rows being windows of no width, whose
+// blocks return at once.
 int ensure_chunks(ela_handle* h) {
-  if (h->win_y0.empty() || h->chunks_yc == h->ychunk) return ELA_OK;
+  if (h->win_y0.empty() || (h->chunks_yc == h->ychunk && (!h->mixed || h->chunks_fluid == h->win_fluid))) return ELA_OK;
   std::vector<int> tab;
-  for (size_t w = 0; w < h->win_y0.size(); ++w) {
-    const int64_t a = h->win_y0[w] + ela::FAT, b = h->win_y0[w] + h->win_ny[w] - ela::FAT;
-    for (int64_t y = a; y < b; y += h->ychunk) {
-      const int row[8] = {(int)y, (int)std::min<int64_t>(y + h->ychunk, b), (int)h->win_y0[w], (int)h->win_ny[w],
-                          (int)h->win_nx[w], 0, 0, 0};
-      tab.insert(tab.end(), row, row + 8);
+  for (int part = 0; part < (h->mixed ? 3 : 1); ++part) {
+    for (size_t w = 0; w < h->win_y0.size(); ++w) {
+      const int64_t a = h->win_y0[w] + ela::FAT, b = h->win_y0[w] + h->win_ny[w] - ela::FAT;
+      const bool in = part == 0 || h->win_fluid[w] == part - 1;
+      for (int64_t y = a; y < b; y += h->ychunk) {
+        const int row[8] = {(int)y, (int)std::min<int64_t>(y + h->ychunk, b), (int)h->win_y0[w], (int)h->win_ny[w],
+                            in ? (int)h->win_nx[w] : 0, 0, 0, 0};
+        tab.insert(tab.end(), row, row + 8);
+      }
     }
+    if (part == 0) h->nchunks = (int)(tab.size() / 8);
   }
   CHK(h->chunks.alloc(tab.size() * sizeof(int)));
   HIPCHK(hipMemcpy(h->chunks.p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
-  h->nchunks = (int)(tab.size() / 8);
   h->chunks_yc = h->ychunk;
+  h->chunks_fluid = h->mixed ? h->win_fluid : std::vector<int>();
   return ELA_OK;
 }
 
@@ -694,7 +706,7 @@ ela::CkArgs<T> interior_args(const ela_handle* h);
 // that it may underflow). Looked at in every transposed call (one read of the
 // medium, 0.2 ms of the 70 to 90 ms of 40 steps of 232x328x324), not when the
 // medium is set: it depends on the windows too, and a medium may be set by a
-// replayed graph.
+// replayed graph. fluid: a cleared entry per window (one without windows).
 template <typename T>
 int check_solid(ela_handle* h, int* fluid) {
   ela::CkArgs<T> a = interior_args<T>(h);
@@ -706,6 +718,20 @@ int check_solid(ela_handle* h, int* fluid) {
 
 int check_solid(ela_handle* h, int* fluid) {
   return h->esize == 4 ? check_solid<float>(h, fluid) : check_solid<double>(h, fluid);
+}
+
+int64_t window_count(const ela_handle* h) { return std::max<int64_t>(1, (int64_t)h->win_y0.size()); }
+
+// The form of the transposed steps from check_solid's answers (host copy and
+// device array). Every window takes the form it takes alone, so its results
+// are the same to the bit in every stack.
+int set_transposed_form(ela_handle* h, const int* fluid, const int* fluid_dev) {
+  h->win_fluid.assign(fluid, fluid + window_count(h));
+  h->win_fluid_dev = fluid_dev;
+  const int64_t n = std::count(h->win_fluid.begin(), h->win_fluid.end(), 0);
+  h->solid = n == window_count(h);
+  h->mixed = n > 0 && !h->solid;
+  return ensure_chunks(h);
 }
 
 // Copies (host) or reads (device) the caller's int64 positions, converts them
@@ -720,17 +746,19 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
       if (sp->n[g]) CHK(check_dev_ptr(sp->pos[g], "a source position list"));
       if (rp->n[g]) CHK(check_dev_ptr(rp->pos[g], "a receiver position list"));
     }
-  // layout: [int64 staging (host calls)] [int32 converted] [int flag]; with
+  // layout: [int64 staging (host calls)] [int32 converted] [int flags]; with
   // `scratch` (device calls only) the same without the staging, in the caller's scratch
   if (scratch && mem != ELA_MEM_DEVICE) return fail(ELA_ERR_ARG, "scratch point conversion needs device positions");
   const size_t b64 = scratch ? 0 : round_up(total * 8, 256), b32 = round_up(total * 4, 256);
-  if (!scratch) CHK(h->pos.alloc(b64 + b32 + 256));
+  const int64_t nwin = transposed ? window_count(h) : 0;
+  const int64_t nflag = std::max<int64_t>(64, 24 + nwin);   // point_scratch_bytes holds 64, and no transposed call's
+  if (!scratch) CHK(h->pos.alloc(b64 + b32 + nflag * sizeof(int)));
   char* base = scratch ? (char*)scratch : (char*)h->pos.p;
   int64_t* s64 = (int64_t*)base;
   int32_t* s32 = (int32_t*)(base + b64);
   int* flag = (int*)(base + b64 + b32);
-  CHK(fill<int>(h, flag, 64));  // flag[0] bad position, flag[1] fluid; boxes at 8 and 16
-  if (transposed) CHK(check_solid(h, flag + 1));
+  CHK(fill<int>(h, flag, nflag));  // flag[0] bad position; boxes at 8 and 16; fluid windows from 24
+  if (transposed) CHK(check_solid(h, flag + 24));
   if (mem == ELA_MEM_HOST && total) {
     char* pin = h->pinned.room((size_t)total * 8);
     int64_t off = 0;
@@ -769,12 +797,12 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   a.ytab = h->win_y0.empty() ? nullptr : (const int*)h->ytab.p;
   a.bad = flag;
   if (total) launch(h, ela::k_convert_pos, dim3((unsigned)((total + 255) / 256)), dim3(256), a);
-  int host[24];
-  HIPCHK(hipMemcpyAsync(host, flag, sizeof(host), hipMemcpyDeviceToHost, h->stream));
+  std::vector<int> host(24 + nwin);
+  HIPCHK(hipMemcpyAsync(host.data(), flag, host.size() * sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  h->solid = !host[1];
-  ds.fuse = ds.box && fuse_injection(h, ds, host + 8);
-  dr.fuse = dr.box && fuse_injection(h, dr, host + 16);
+  ds.fuse = ds.box && fuse_injection(h, ds, host.data() + 8);
+  dr.fuse = dr.box && fuse_injection(h, dr, host.data() + 16);
+  if (transposed) CHK(set_transposed_form(h, host.data() + 24, flag + 24));
   if (host[0]) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
   return ELA_OK;
 }
@@ -1015,6 +1043,8 @@ Wave<T> wave_ptrs(DevBuf& b, int64_t stride, bool premultiplied = false) {
 // normal stresses keep both: q alone is 3 to 4 % faster still, but the inverse
 // of their 3 x 3 block enlarges q's roundings by (3 lambda + 2 mu) / 2 mu, up to
 // 1.8 times the FP32 error at Vp / Vs = 4; as it is the error is the same.
+// A stack of solid and fluid windows is held in the general form's 36 arrays, of
+// which the steps of its solid windows use q and the normal stresses of n.
 template <typename T>
 Wave<T> adj_wave(ela_handle* h) {
   if (!h->solid) return wave_ptrs<T>(h->wave2, h->stride, true);
@@ -1052,14 +1082,29 @@ ela::PointArgs<T> adj_points(ela_handle* h, const DevPoints& pts, T* const p[9],
   ela::PointArgs<T> a = make_points<T>(h, pts, p, tr, true, n);
   for (int k = 0; k < 9; ++k) a.q[k] = q[k];
   for (int k = 0; k < 8; ++k) a.m[k] = arr<T>(h->med, h->stride, k);
+  if (h->mixed) a.fluid = h->win_fluid_dev;
   return a;
 }
 
+// One transposed step. A mixed stack takes two launches, each over its own
+// windows (ensure_chunks): the solid ones first, then the others with what
+// concerns all of them, the recording and an injection by itself (which adds to
+// n and q alike; the n of a solid window's velocities and shear stresses is
+// read by nobody).
 template <typename T, int FV, int FS>
 int adj_launch(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& rp, const ela::PointArgs<T>& inj,
                const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
   if (h->solid) return step_with_points<T, ela::MODE_BORN_ADJ_Q, FV, FS>(h, a, rp, inj, rec);
-  return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, a, rp, inj, rec);
+  if (!h->mixed) return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, a, rp, inj, rec);
+  ela::StepArgs<T> q = a, pm = a;
+  q.o = a.qn;
+  q.c = a.q;
+  q.q = nullptr;
+  q.qn = a.o + ela::SXX * a.np;
+  q.chunks = a.chunks + 8 * (int64_t)h->nchunks;
+  pm.chunks = q.chunks + 8 * (int64_t)h->nchunks;
+  CHK((launch_step_m<T, ela::MODE_BORN_ADJ_Q, FV, FS>(h, q, 3, rp.fuse ? inj : ela::PointArgs<T>{})));
+  return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, pm, rp, inj, rec);
 }
 
 // The 9 components of a time-major trace buffer share one base pointer
@@ -2230,13 +2275,15 @@ template <typename T>
 int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   const int64_t np = h->stride;
   const int dfmt = drv_format(h);
-  int fluid = 1;
-  int* flag = static_cast<int*>(h->counter.p) + 8;   // behind the step counters
-  CHK(fill<int>(h, flag, 1));
+  const int64_t nwin = window_count(h);
+  std::vector<int> fluid(nwin);
+  CHK(h->pos.alloc(nwin * sizeof(int)));
+  int* flag = static_cast<int*>(h->pos.p);
+  CHK(fill<int>(h, flag, nwin));
   CHK(check_solid(h, flag));
-  HIPCHK(hipMemcpyAsync(&fluid, flag, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipMemcpyAsync(fluid.data(), flag, nwin * sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  h->solid = !fluid;
+  CHK(set_transposed_form(h, fluid.data(), flag));
   CHK(h->wave2.alloc((size_t)adj_arrays(h) * np * sizeof(T)));
   CHK(h->drv.alloc(drv_step_bytes(h, dfmt)));
   CHK(h->g32.alloc((size_t)8 * np * sizeof(T)));
@@ -2631,6 +2678,8 @@ int ela_set_windows(ela_handle* h, int n, const int64_t* y0, const int64_t* ny, 
     DeviceGuard dg(h->cfg.device);
     h->win_y0.clear(); h->win_ny.clear(); h->win_nx.clear();
     h->chunks_yc = 0;
+    h->solid = h->mixed = false;   // asked again by the next transposed call
+    h->win_fluid.clear();
     h->grad_ready = false;
     if (n == 0) return ELA_OK;
     const int64_t NY = h->cfg.ny;
@@ -2647,6 +2696,7 @@ int ela_set_windows(ela_handle* h, int n, const int64_t* y0, const int64_t* ny, 
         tab[4 * y] = (int)y0[w];
         tab[4 * y + 1] = (int)ny[w];
         tab[4 * y + 2] = (int)nx[w];
+        tab[4 * y + 3] = w;
       }
       prev_end = y0[w] + ny[w];
       h->win_y0.push_back(y0[w]); h->win_ny.push_back(ny[w]); h->win_nx.push_back(nx[w]);

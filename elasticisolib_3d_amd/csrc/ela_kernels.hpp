@@ -490,7 +490,8 @@ struct PointArgs {
   // damping (injection only)
   const T* taper;
   int min_pad, nz, nx, ny, nzi, zoff;
-  const int* ytab;         // stacked windows: per plane {window y0, window ny, window nx, 0}, or null
+  const int* ytab;         // stacked windows: per plane {window y0, window ny, window nx, window}, or null
+  const int* fluid;        // per window: general steps (1) or MODE_BORN_ADJ_Q (0), or null: field says it
   const int* its_dev;      // coarse sample index read from device memory (graph replays), or null
   int its_off;             // added to the index read from its_dev
   // fine step k = *step_dev + step_off read from device memory (graph replays
@@ -630,7 +631,9 @@ __device__ __forceinline__ void record_point(const PointArgs<T>& a, int64_t g) {
   T fa, fb;
   if (!point_time<T>(a, its, fa, fb)) return;
   // MODE_BORN_ADJ_Q holds no n of the velocities and shear stresses
-  const T v = a.field[c] ? a.field[c][p] : level_of(a.q[c][p], a.m[c < 3 ? c : MXZ + (c - SXZ)][p]);
+  bool held = a.field[c] != nullptr;
+  if (a.fluid && (c < SXX || c > SZZ)) held = a.fluid[a.ytab[4 * (p / (a.nzi * a.nx)) + 3]];
+  const T v = held ? a.field[c][p] : level_of(a.q[c][p], a.m[c < 3 ? c : MXZ + (c - SXZ)][p]);
   T* tr = a.tr[c] + k * a.tr_stride_pt;
   T& t0 = tr[(int64_t)its * a.tr_stride_t];
   T& t1 = tr[(int64_t)(its + 1) * a.tr_stride_t];
@@ -1666,7 +1669,7 @@ __device__ __forceinline__ int64_t ck_offset(const CkArgs<T>& a, int64_t q) {
 }
 
 // Whether an interior cell of the grid lies in the interior of a window
-// (ytab: per plane {window y0, ny, nx, 0}, zeros between the windows).
+// (ytab: per plane {window y0, ny, nx, window}, zeros between the windows).
 __device__ __forceinline__ bool in_window(const int* ytab, int ix, int iy) {
   const int wy0 = ytab[4 * iy], wny = ytab[4 * iy + 1], wnx = ytab[4 * iy + 2];
   return iy >= wy0 + FAT && iy < wy0 + wny - FAT && ix < wnx - FAT;
@@ -1797,25 +1800,30 @@ __global__ void __launch_bounds__(256) k_scale_medium(MedArgs<T> a) {
   }
 }
 
-// *fluid = 1 if the buoyancies or shear moduli of any cell that is stepped
-// (interior cells, with ytab those of the windows) are not safely divided by
-// (see check_solid). NaN counts as such.
+// fluid[w] = 1 if the buoyancies or shear moduli of any interior cell of window
+// w (without ytab: of the grid, w = 0) are not safely divided by (see
+// check_solid). NaN counts as such. At most one atomic a wave and window.
 template <typename T>
 __global__ void __launch_bounds__(256) k_check_solid(CkArgs<T> a, const int* ytab, int* fluid) {
-  bool bad = false;
+  int told = -1;   // the last window this lane's wave has reported
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nI; q += (int64_t)gridDim.x * blockDim.x) {
+    int w = 0;
     if (ytab) {
       const uint32_t r = fdiv((uint32_t)q, a.dz), iy = fdiv(r, a.dx), ix = r - iy * (uint32_t)a.nxI;
       if (!in_window(ytab, (int)ix + FAT, (int)iy + FAT)) continue;
+      w = ytab[4 * (iy + FAT) + 3];
     }
     const int64_t i = ck_offset(a, q);
     const T least = a.f[L2M][i] * T(0x1p-20);
     bool ok = least > T(0);
     for (int k = MXZ; k <= MYZ; ++k) ok = ok && a.f[k][i] >= least;
     for (int k = BX_; k <= BZ_; ++k) ok = ok && a.f[k][i] > T(0);
-    bad = bad || !ok;
+    if (!ok && w != told) {
+      told = w;
+      const int first = __ffsll((unsigned long long)__ballot(1)) - 1;
+      if ((int)(threadIdx.x & 63) == first || w != __builtin_amdgcn_readfirstlane(w)) atomicOr(fluid + w, 1);
+    }
   }
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(fluid, 1);
 }
 
 // Streaming reference for the roofline: R arrays of n4 16-byte vectors are

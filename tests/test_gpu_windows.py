@@ -120,13 +120,13 @@ def test_born_adjoint_adds_inside_the_windows_only(precision, device):
 
 # receivers per window and list: few (injected in the step's blocks) and many (a launch of their own)
 @pytest.mark.parametrize("nrec", [5, 70])
-@pytest.mark.parametrize("fluid", [(), (0, 1, 2)])
+@pytest.mark.parametrize("fluid", [(), (1,), (0, 2), (0, 1, 2)])
 @pytest.mark.parametrize("medium,graph", [("scaled", False), ("scaled", True), ("elastic", True)])
 def test_transposed_steps_of_a_stack_equal_each_window_alone(medium, graph, fluid, nrec):
     """FP32 gradient, source gradient and Born adjoint of a stack, to the bit
-    what each window gives alone: the cells outside the windows (zeros in a
-    stack of scaled arrays) do not decide how the transposed wavefield is
-    held."""
+    what each window gives alone: neither the cells outside the windows (zeros
+    in a stack of scaled arrays) nor a fluid in another window decides how a
+    window's transposed wavefield is held."""
     probs = window_problems(nrec, fluid)
     spos, rpos = stack_points(probs, "spos"), stack_points(probs, "rpos")
     src, rec = stack_traces(probs, "src"), stack_traces(probs, "rec")
