@@ -10,16 +10,23 @@ of x columns, or the round robin over groups of whole z columns). The best
 choice depends on the grid (tile counts, partial tiles, L2 reuse of halo
 planes), so it is measured: every candidate
 is timed with HIP events on the propagator's own stream
-(ela_time_step_kernels: a velocity and a stress launch of a forward step on
-the handle's current wavefields, which it overwrites), and the fastest is
-applied. Results are cached per device name, precision, medium kind and grid
-shape in a JSON file (ELA_TUNE_CACHE, default ~/.cache/elasticisolib_3d_amd/tuning.json).
+(ela_time_step_kernels: forward steps, both halves in one launch, on the
+handle's current wavefields, which it overwrites). The shape that the handle
+has is a candidate too -- a new handle's is chosen by the grid and on small
+grids none of the others -- and keeps its place unless the fastest other one
+beats it again when the two are timed in turn. Results are cached per device
+name, library build, precision, medium kind and grid shape in a JSON file
+(ELA_TUNE_CACHE, default ~/.cache/elasticisolib_3d_amd/tuning.json).
 """
 from __future__ import annotations
 
+import functools
+import hashlib
 import json
 import os
 from typing import Dict, Iterable, Optional, Sequence, Tuple
+
+from . import _lib
 
 TILE_X = (16, 8, 4)
 Y_CHUNK = (4, 8, 16, 32)
@@ -46,10 +53,20 @@ def _device_name() -> str:
         return "unknown"
 
 
+@functools.lru_cache(maxsize=None)
+def _build() -> str:
+    """Names the kernels a ranking was measured on: a digest of the library."""
+    try:
+        with open(_lib.LIB_PATH, "rb") as f:
+            return hashlib.sha1(f.read()).hexdigest()[:12]
+    except OSError:
+        return "none"
+
+
 def _key(prop, target: str = "forward") -> str:
     ny, nx, nz = prop.shape
     kind = getattr(prop, "medium_kind", "scaled")   # the steppers differ with the medium kind
-    key = f"{_device_name()}|{prop.precision}|{kind}|{nz}x{nx}x{ny}"
+    key = f"{_device_name()}|{_build()}|{prop.precision}|{kind}|{nz}x{nx}x{ny}"
     if target == "gradient":   # the gradient's kernel mix, with its derivative storage
         key += f"|gradient|{prop.gradient_derivatives_used()}"
     return key
@@ -82,11 +99,42 @@ def apply(prop, best: dict) -> None:
         prop.set_tiling_transposed(best.get("tile_x_transposed", 0))
 
 
+def _own_shape(prop) -> Optional[dict]:
+    """The launch shape that `prop` has (None where it cannot say)."""
+    if not (hasattr(prop, "get_tiling") and hasattr(prop, "tile_order")):
+        return None
+    tx, yc = prop.get_tiling()
+    return {"tile_x": tx, "y_chunk": yc, "order": prop.tile_order[0], "x_group": prop.tile_order[1]}
+
+
+def _times(prop, target: str, reps: int) -> dict:
+    if target == "gradient":
+        f, r, t = prop.time_gradient_kernels(reps)
+        return {"ms_step": f + r + t, "ms_forward": f, "ms_recompute": r, "ms_transposed": t}
+    v, s = prop.time_step_kernels(reps)
+    return {"ms_step": v + s, "ms_velocity": v, "ms_stress": s}
+
+
+def _duel(prop, own: dict, best: dict, target: str, reps: int, rounds: int = 3) -> dict:
+    """The better of two shapes, timed in turn (one measurement of each candidate
+    strays by more than the shapes near the front differ)."""
+    least = [None, None]
+    for _ in range(rounds):
+        for k, shape in enumerate((own, best)):
+            apply(prop, shape)
+            t = _times(prop, target, reps)
+            if least[k] is None or t["ms_step"] < least[k]["ms_step"]:
+                least[k] = t
+    k = 0 if least[0]["ms_step"] <= least[1]["ms_step"] else 1
+    return dict((own, best)[k], **least[k])
+
+
 def autotune(prop, reps: int = 10, candidates: Optional[Iterable[Candidate]] = None, use_cache: bool = True,
              verbose: bool = False, target: str = "forward") -> dict:
     """Time every candidate launch shape on `prop` (its medium must be set),
     apply the fastest and return {tile_x, y_chunk, order, x_group, ms_step,
-    table}. The wavefields of the handle are overwritten. `target`
+    table}. Unless `candidates` are given the handle's own shape is among
+    them (_duel). The wavefields of the handle are overwritten. `target`
     "forward" ranks the shapes by a forward step (both halves in one
     launch); "gradient" by the three kernel pairs of an adjoint-state
     gradient step (forward, recomputation with derivative store, transposed
@@ -104,6 +152,14 @@ def autotune(prop, reps: int = 10, candidates: Optional[Iterable[Candidate]] = N
             apply(prop, hit)
             return dict(hit, cached=True)
     cands = list(candidates) if candidates is not None else list(default_candidates(prop.precision))
+    own = _own_shape(prop) if candidates is None else None
+    if own is not None:
+        own["target"] = target
+        shape = (own["tile_x"], own["y_chunk"], own["order"], own["x_group"])
+        if target == "gradient":
+            own["tile_x_transposed"] = prop.get_tiling_transposed()
+        if shape not in cands:
+            cands.append(shape)
     if hasattr(prop, "set_tiling_transposed"):
         prop.set_tiling_transposed(0)   # candidates are timed with one tile for every step
     prop.set_tiling(*cands[0][:2])
@@ -139,6 +195,8 @@ def autotune(prop, reps: int = 10, candidates: Optional[Iterable[Candidate]] = N
                             ms_recompute=f[2], ms_transposed=tr[3], tile_x_transposed=tr[4])
     else:
         best.update(ms_velocity=table[0][1], ms_stress=table[0][2])
+    if own is not None and any(best[k] != v for k, v in own.items()):
+        best = _duel(prop, own, best, target, reps)
     apply(prop, best)
     if use_cache and candidates is None:
         tab = _load()

@@ -64,6 +64,7 @@ class Propagator:
         self.h = h
         self._keep = []
         self.medium_kind = None   # "scaled" (set_medium) or "elastic" (set_elastic)
+        self.tile_order = (3, 4)  # a new handle's (set_tile_order)
 
     def close(self):
         if getattr(self, "h", None):
@@ -339,6 +340,7 @@ class Propagator:
         of x_group columns, 3 hardware order with groups of x_group whole z
         columns per XCD (speed only)."""
         check(self.lib.ela_set_tile_order(self.h, int(order), int(x_group)), "ela_set_tile_order")
+        self.tile_order = (int(order), int(x_group))
 
     def set_born_storage(self, segment: int = 0, budget_bytes: int = 0) -> None:
         """Coarse-wavefield storage of the Born adjoint: 0 automatic (within

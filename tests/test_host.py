@@ -274,6 +274,75 @@ def test_autotuner_gradient_target(tmp_path, monkeypatch):
         A.autotune(q, target="adjoint")
 
 
+class _ShapedProp:
+    """A handle whose grid wants 13 planes a block, a shape no candidate has:
+    every other plane count is 10 % slower. `lucky` is a shape whose first
+    measurement comes out 20 % too short."""
+    precision = "f32"
+    shape = (40, 50, 60)
+
+    def __init__(self, lucky=None):
+        self.tiling, self.tile_order, self.tile_t = (4, 13), (3, 4), 0
+        self.lucky, self.calls = lucky, 0
+
+    def get_tiling(self):
+        return self.tiling
+
+    def set_tiling(self, tx, yc):
+        self.tiling = (tx, yc)
+
+    def set_tile_order(self, o, g):
+        self.tile_order = (o, g)
+
+    def set_tiling_transposed(self, tx):
+        self.tile_t = tx
+
+    def get_tiling_transposed(self):
+        return self.tile_t or self.tiling[0]
+
+    def gradient_derivatives_used(self):
+        return "native"
+
+    def time_step_kernels(self, reps):
+        self.calls += 1
+        t = 1.0 if self.tiling[1] == 13 else 1.1
+        if self.tiling + self.tile_order == self.lucky:
+            self.lucky, t = None, 0.8 * t
+        return t / 2, t / 2
+
+    def time_gradient_kernels(self, reps):
+        return (sum(self.time_step_kernels(reps)),) * 3
+
+
+@pytest.mark.parametrize("target", ["forward", "gradient"])
+@pytest.mark.parametrize("lucky", [None, (8, 16, 3, 2)])
+def test_autotuner_keeps_the_handles_own_shape_where_it_is_fastest(tmp_path, monkeypatch, target, lucky):
+    """Tuning does not slow a handle whose own shape, chosen by the grid, is
+    none of the listed candidates, nor by one measurement that came out short;
+    the kept shape is cached like another."""
+    from elasticisolib_3d_amd import autotune as A
+    monkeypatch.setenv("ELA_TUNE_CACHE", str(tmp_path / "t.json"))
+    p = _ShapedProp(lucky)
+    best = A.autotune(p, target=target)
+    assert p.tiling == (4, 13) and p.tile_order == (3, 4) and p.get_tiling_transposed() == 4
+    assert (best["tile_x"], best["y_chunk"], best["order"], best["x_group"]) == (4, 13, 3, 4) and not best["cached"]
+    assert best["ms_step"] == (1.0 if target == "forward" else 3.0)
+    q = _ShapedProp()
+    q.tiling = (8, 8)
+    assert A.autotune(q, target=target)["cached"] and q.tiling == (4, 13) and q.calls == 0
+
+
+def test_autotuner_cache_is_per_library_build(tmp_path, monkeypatch):
+    """A ranking measured on other kernels is not applied."""
+    from elasticisolib_3d_amd import autotune as A
+    monkeypatch.setenv("ELA_TUNE_CACHE", str(tmp_path / "t.json"))
+    A.autotune(_ShapedProp())
+    assert A.autotune(_ShapedProp())["cached"]
+    monkeypatch.setattr(A, "_build", lambda: "another build")
+    p = _ShapedProp()
+    assert not A.autotune(p)["cached"] and p.calls > 0
+
+
 def test_positions_follow_the_memory_kind_of_the_call():
     """Position lists are handed to the library in the memory kind of the
     call (host here: torch CPU tensors become numpy arrays), so that a
