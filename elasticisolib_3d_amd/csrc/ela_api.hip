@@ -609,17 +609,14 @@ int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::
   return launch_step_s<T, ela::TILE_NARROW, MODE, FV, FS>(h, a, which, inj, rec);
 }
 
-// Forward, nonlinear-adjoint and premultiplied transposed steps form the
-// medium from (rho, lambda, mu) when the handle holds them (ela_set_elastic):
-// 3 medium reads per cell instead of 8. MODE_BORN_ADJ and the injections read
+// The steps form the medium from (rho, lambda, mu) when the handle holds them
+// (ela_set_elastic): 3 medium reads per cell instead of 8. The injections read
 // the 8 scaled arrays, which k_scale_medium derives with the steppers'
 // operations, so both routes give bit-identical results.
 template <typename T, int MODE, int FV, int FS>
 int launch_step_m(ela_handle* h, const ela::StepArgs<T>& a, int which = 3,
                   const ela::PointArgs<T>& inj = ela::PointArgs<T>{}, const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
-  if constexpr (MODE != ela::MODE_BORN_ADJ) {
-    if (h->have_elastic) return launch_step<T, MODE, FV | ela::F_MED3, FS | ela::F_MED3>(h, a, which, inj, rec);
-  }
+  if (h->have_elastic) return launch_step<T, MODE, FV | ela::F_MED3, FS | ela::F_MED3>(h, a, which, inj, rec);
   return launch_step<T, MODE, FV, FS>(h, a, which, inj, rec);
 }
 

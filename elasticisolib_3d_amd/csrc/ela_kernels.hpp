@@ -48,11 +48,13 @@ constexpr int NXCD = 8;      // MI355X: 8 XCDs, blocks dealt round-robin
 enum { VX = 0, VY, VZ, SXX, SYY, SZZ, SXZ, SXY, SYZ };
 enum { BX_ = 0, BY_, BZ_, L2M, LAM, MXZ, MXY, MYZ };
 
-// Stepper modes.
+// Stepper modes. The transposed steps (stepAdjGpuBorn_3D, n = w(w o - D (M c)),
+// which multiplies by the medium at every loaded position,
+// kernelsElaGpu_3D.cu:864-1040) read M c as the step before wrote it, one array
+// per field as in the forward step.
 enum { MODE_FWD = 0,       // n = w(w o + M D c)        stepFwdGpu_3D
        MODE_ADJ = 1,       // n = w(w o - M D c)        stepAdjGpu_3D
-       MODE_BORN_ADJ = 2,  // n = w(w o - D (M c))      stepAdjGpuBorn_3D
-       MODE_BORN_ADJ_PM = 3, // the same with M c read premultiplied (q) and M n written (qn)
+       MODE_BORN_ADJ_PM = 3, // n = w(w o - D q) with q = M c read and M n written (qn) beside n
        MODE_BORN_ADJ_Q = 4   // the same on q = M n alone but for the normal stresses: q' = w(w q - M D c) (adj_wave)
 };
 
@@ -164,11 +166,6 @@ __device__ __forceinline__ T damp_w(const StepArgs<T>& a, int iz, int ix, int iy
   int d = min(min(iz - FAT, ix - FAT), min(a.nz - iz - 1 - FAT, wnx - ix - 1 - FAT));
   d = min(d, min(iy - wy0 - FAT, wy0 + wny - iy - 1 - FAT));
   return d < a.min_pad ? a.taper[d] : T(1);
-}
-
-template <typename T>
-__device__ __forceinline__ T ld(const T* __restrict__ p, int64_t i, bool ok) {
-  return ok ? p[i] : T(0);
 }
 
 // y-derivative from an 8-deep queue q[j] = f[iy - s + j], s = 3 for D+ and 4
@@ -320,52 +317,12 @@ __device__ __forceinline__ float load_dq16(const int16_t* q, const float* sc, ui
   return (float)*at(q, i) * *at(sc, i / DQ_BLOCK);
 }
 
-// Values that the derivative operators see. In MODE_BORN_ADJ they are the
-// medium-multiplied fields (stepAdjGpuBorn_3D multiplies at every loaded
-// position, kernelsElaGpu_3D.cu:864-1040); MODE_BORN_ADJ_PM reads the same
-// products from the premultiplied level that the previous step wrote, so its
-// halo and queue loads are one array per field as in the forward stepper.
-//
-// The loads are not predicated: a tile's columns, halo rows and halo column
-// past the grid are clamped to its last row and column (tile_coord), where no
-// interior cell's stencil reads them. That keeps them inside the arrays and
-// makes idle lanes read lines their neighbours read anyway (unclamped, behind
-// every array's guard of GUARD_ROWS rows plus GUARD_EXTRA elements, forward
-// 152x152x148 took 5 % longer).
-template <typename T, int MODE>
-struct StressVal {
-  const StepArgs<T>& a;
-  int64_t np;
-  __device__ __forceinline__ T c(int f, uint32_t i) const {
-    return *at(fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np), i);
-  }
-  __device__ __forceinline__ T m(int k, uint32_t i) const { return *at(fam(a.m, k, np), i); }
-  // f: the normal stress, g and h the two others
-  __device__ __forceinline__ T normal(int f, int g, int h, uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ) return c(f, i) * m(L2M, i) + (c(g, i) + c(h, i)) * m(LAM, i);
-    return c(f, i);
-  }
-  __device__ __forceinline__ T shear(int f, int k, uint32_t i) const {
-    return MODE == MODE_BORN_ADJ ? c(f, i) * m(k, i) : c(f, i);
-  }
-  __device__ __forceinline__ T sxx(uint32_t i) const { return normal(SXX, SYY, SZZ, i); }
-  __device__ __forceinline__ T syy(uint32_t i) const { return normal(SYY, SXX, SZZ, i); }
-  __device__ __forceinline__ T szz(uint32_t i) const { return normal(SZZ, SXX, SYY, i); }
-  __device__ __forceinline__ T sxz(uint32_t i) const { return shear(SXZ, MXZ, i); }
-  __device__ __forceinline__ T sxy(uint32_t i) const { return shear(SXY, MXY, i); }
-  __device__ __forceinline__ T syz(uint32_t i) const { return shear(SYZ, MYZ, i); }
-};
-
-template <typename T, int MODE>
-struct VelVal {
-  const StepArgs<T>& a;
-  int64_t np;
-  __device__ __forceinline__ T v(int f, uint32_t i) const {
-    if (MODE == MODE_BORN_ADJ_PM) return *at(fam(a.q, f, np), i);
-    const T c = *at(fam(a.c, f, np), i);
-    return MODE == MODE_BORN_ADJ ? c * *at(fam(a.m, f, np), i) : c;  // BX_/BY_/BZ_ == VX/VY/VZ
-  }
-};
+// The stencil's loads are not predicated: a tile's columns, halo rows and halo
+// column past the grid are clamped to its last row and column (tile_coord),
+// where no interior cell's stencil reads them. That keeps them inside the
+// arrays and makes idle lanes read lines their neighbours read anyway
+// (unclamped, behind every array's guard of GUARD_ROWS rows plus GUARD_EXTRA
+// elements, forward 152x152x148 took 5 % longer).
 
 // Per-thread tile geometry, halo roles and 32-bit column offsets.
 //
@@ -377,10 +334,9 @@ struct TileCoord {
   int tz, ty, iz, izo, ix, y0, y1, z0, x0;   // iz internal, izo reference z
   int wy0, wny, wnx;       // the tile's window: first plane, planes, x extent (whole grid without windows)
   bool empty;              // no interior cell in the tile (its window is narrower than the tile's x)
-  bool okc, active;        // own column inside the grid / inside the interior
+  bool active;             // own column inside the interior
   bool xin;                // the tile row (wave-uniform) is an interior x row
-  bool xh, okxl, okxh;     // x-halo loader (ty < 4) and its low/high validity
-  bool zh, okzh;           // z-halo loader (lanes 0-7) and validity
+  bool xh, zh;             // x-halo loader (ty < 4), z-halo loader (tz < 8)
   int colh;                // LDS column of the z-halo value
   uint32_t col, cxl, cxh, czh;  // own column, x-halo rows, z-halo column, each clamped to the grid (window)
   uint32_t colu;                // own column, not clamped (F_Q16 stores of whole lines)
@@ -435,17 +391,13 @@ __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int n
   }
   nx = t.wnx;
   t.empty = t.x0 >= nx - FAT;
-  t.okc = t.izo < nz && t.ix < nx;
   t.xin = t.ix < nx - FAT;
   t.active = (t.izo < nz - FAT) && t.xin;
   t.xh = t.ty < FAT;
   const int ixlo = t.x0 - FAT + t.ty, ixhi = t.x0 + BX + t.ty;
-  t.okxl = t.xh && t.izo < nz;
-  t.okxh = t.okxl && ixhi < nx;
   t.zh = t.tz < 2 * FAT;
   const int izh = t.tz < FAT ? t.z0 - FAT + t.tz : t.z0 + BZ + (t.tz - FAT);
   t.colh = t.tz < FAT ? t.tz : BZ + t.tz;
-  t.okzh = t.zh && (izh - zoff) < nz && t.ix < nx;
   // Lanes past the last z cell and rows past the last x row read the last
   // one: no interior stencil uses their values, and without the clamp they
   // fetched lines nobody needs (a 144-cell z interior is 2.25 tiles: 200
@@ -773,18 +725,16 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
   static_assert(!QS || (!SS && !ACC && (F & F_GRAD) == 0 && MODE == MODE_FWD), "F_Q16 stores: MODE_FWD recomputation");
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
-  static_assert(!MED3 || MODE != MODE_BORN_ADJ, "MODE_BORN_ADJ reads the scaled medium");
   auto& l_xx = L.xx; auto& l_zz = L.zz; auto& l_xy = L.xy; auto& l_xz = L.xz; auto& l_yz = L.yz;
   auto& l_rho = L.rho;
   const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   int64_t np = a.np;
-  auto S_ = [&]() { return StressVal<T, MODE>{a, np}; };
-  // FP32 rows that are plain array values go straight from HBM to LDS
-  // (MODE_BORN_ADJ multiplies them by the medium first, in registers)
-  constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
+  // FP32 rows go straight from HBM to LDS, FP64 rows through registers
+  constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4;
   auto src = [&](int f) -> const T* { return fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np); };
+  auto val = [&](int f, uint32_t i) { return *at(src(f), i); };
   const int r = t.ty + FAT, q = t.tz + FAT;
   // first x row of the wave (a wide tile's wave is one row), wave-uniform
   const int wy = __builtin_amdgcn_readfirstlane(t.ty), wr = wy + FAT;
@@ -797,26 +747,26 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
       rows_to_lds<S>(src(SZZ), pl + t.col, l_zz[nb], wr, FAT);
       rows_to_lds<S>(src(SXZ), pl + t.col, l_xz[nb], wr, FAT);
     } else {
-      v.xx = S_().sxx(pl + t.col);
-      v.zz = S_().szz(pl + t.col);
-      v.xz = S_().sxz(pl + t.col);
+      v.xx = val(SXX, pl + t.col);
+      v.zz = val(SZZ, pl + t.col);
+      v.xz = val(SXZ, pl + t.col);
     }
-    v.nxy = S_().sxy(pl + 4 * ys + t.col);
-    v.nyy = S_().syy(pl + 3 * ys + t.col);
-    v.nyz = S_().syz(pl + 4 * ys + t.col);
+    v.nxy = val(SXY, pl + 4 * ys + t.col);
+    v.nyy = val(SYY, pl + 3 * ys + t.col);
+    v.nyz = val(SYZ, pl + 4 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
         rows_to_lds<S>(src(SXX), pl + t.cxl, l_xx[nb], wy, FAT); rows_to_lds<S>(src(SXX), pl + t.cxh, l_xx[nb], wr + BX, FAT);
         rows_to_lds<S>(src(SXY), pl + t.cxl, l_xy[nb], wy, FAT); rows_to_lds<S>(src(SXY), pl + t.cxh, l_xy[nb], wr + BX, FAT);
         rows_to_lds<S>(src(SXZ), pl + t.cxl, l_xz[nb], wy, FAT); rows_to_lds<S>(src(SXZ), pl + t.cxh, l_xz[nb], wr + BX, FAT);
       } else {
-        v.hxx0 = S_().sxx(pl + t.cxl); v.hxx1 = S_().sxx(pl + t.cxh);
-        v.hxy0 = S_().sxy(pl + t.cxl); v.hxy1 = S_().sxy(pl + t.cxh);
-        v.hxz0 = S_().sxz(pl + t.cxl); v.hxz1 = S_().sxz(pl + t.cxh);
+        v.hxx0 = val(SXX, pl + t.cxl); v.hxx1 = val(SXX, pl + t.cxh);
+        v.hxy0 = val(SXY, pl + t.cxl); v.hxy1 = val(SXY, pl + t.cxh);
+        v.hxz0 = val(SXZ, pl + t.cxl); v.hxz1 = val(SXZ, pl + t.cxh);
       }
     }
     if (t.zh) {
-      v.hzz = S_().szz(pl + t.czh); v.hxz = S_().sxz(pl + t.czh); v.hyz = S_().syz(pl + t.czh);
+      v.hzz = val(SZZ, pl + t.czh); v.hxz = val(SXZ, pl + t.czh); v.hyz = val(SYZ, pl + t.czh);
     }
     if (MED3) {
       // the column's own cell and its x - 1 / z - 1 neighbours
@@ -855,9 +805,9 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
   T qxy[8], qyy[8], qyz[8];
 #pragma unroll
   for (int j = 0; j < 7; ++j) {
-    qxy[j] = S_().sxy((uint32_t)(t.y0 - 3 + j) * ys + t.col);
-    qyy[j] = S_().syy((uint32_t)(t.y0 - 4 + j) * ys + t.col);
-    qyz[j] = S_().syz((uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qxy[j] = val(SXY, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qyy[j] = val(SYY, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qyz[j] = val(SYZ, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
   }
   bool inj_hit;  // block-uniform
   {
@@ -903,7 +853,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
         o3[f] = ld_nt(fam(a.o, f, np), i);
-        if (!MED3 && MODE != MODE_BORN_ADJ) m3[f] = ld_nt(fam(a.m, f, np), i);
+        if (!MED3) m3[f] = ld_nt(fam(a.m, f, np), i);
         if constexpr (HOIST) {
           if (SS) ss3[f] = load_ss(f);
           if (ACC) load_acc(f);
@@ -1000,25 +950,23 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
   static_assert(!Q16 || sizeof(T) == 4, "F_Q16 is an FP32 format");
   static_assert(!QS || (!SS && !ACC && (F & F_GRAD) == 0 && MODE == MODE_FWD), "F_Q16 stores: MODE_FWD recomputation");
   constexpr bool HOIST = sizeof(T) == 4;  // per-cell operands loaded ahead of the stores
-  static_assert(!MED3 || MODE != MODE_BORN_ADJ, "MODE_BORN_ADJ reads the scaled medium");
   auto& l_vx = L.vx; auto& l_vy = L.vy; auto& l_vz = L.vz; auto& l_mu = L.mu;
   const TileCoord t = tile_coord<S>(bid, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap, a.xgroup, a.chunks);
   if (t.empty) return;  // block-uniform, before any barrier
   const uint32_t ys = (uint32_t)a.ys;
   int64_t np = a.np;
-  auto V_ = [&]() { return VelVal<T, MODE>{a, np}; };
-  // FP32 rows that are plain array values go straight from HBM to LDS (see velocity_block)
-  constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4 && MODE != MODE_BORN_ADJ;
+  constexpr bool DMA = ELA_LDS_DMA && sizeof(T) == 4;
   auto src = [&](int f) -> const T* { return fam(MODE == MODE_BORN_ADJ_PM ? a.q : a.c, f, np); };
+  auto val = [&](int f, uint32_t i) { return *at(src(f), i); };
   const int r = t.ty + FAT, q = t.tz + FAT;
   const int wy = __builtin_amdgcn_readfirstlane(t.ty), wr = wy + FAT;  // wave-uniform row
 
   // plane p's values: LDS rows of buffer nb directly (DMA), the rest into v
   auto fetch = [&](StressStage<T>& v, int p, int nb) {
     const uint32_t pl = (uint32_t)p * ys;
-    v.nx = V_().v(VX, pl + 3 * ys + t.col);
-    v.ny = V_().v(VY, pl + 4 * ys + t.col);
-    v.nz = V_().v(VZ, pl + 3 * ys + t.col);
+    v.nx = val(VX, pl + 3 * ys + t.col);
+    v.ny = val(VY, pl + 4 * ys + t.col);
+    v.nz = val(VZ, pl + 3 * ys + t.col);
     if (wy < FAT) {  // the x-halo loaders (t.xh) are whole waves
       if constexpr (DMA) {
         rows_to_lds<S>(src(VX), pl + t.cxl, l_vx[nb], wy, FAT); rows_to_lds<S>(src(VX), pl + t.cxh, l_vx[nb], wr + BX, FAT);
@@ -1026,12 +974,12 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         rows_to_lds<S>(src(VZ), pl + t.cxl, l_vz[nb], wy, FAT); rows_to_lds<S>(src(VZ), pl + t.cxh, l_vz[nb], wr + BX, FAT);
       } else {
 #pragma unroll
-        for (int f = 0; f < 3; ++f) { v.hlo[f] = V_().v(f, pl + t.cxl); v.hhi[f] = V_().v(f, pl + t.cxh); }
+        for (int f = 0; f < 3; ++f) { v.hlo[f] = val(f, pl + t.cxl); v.hhi[f] = val(f, pl + t.cxh); }
       }
     }
     if (t.zh) {
 #pragma unroll
-      for (int f = 0; f < 3; ++f) v.hz[f] = V_().v(f, pl + t.czh);
+      for (int f = 0; f < 3; ++f) v.hz[f] = val(f, pl + t.czh);
     }
   };
   // F_MED3: shear modulus of plane p around the column
@@ -1070,9 +1018,9 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
   T qx[8], qy[8], qz[8];
 #pragma unroll
   for (int j = 0; j < 7; ++j) {
-    qx[j] = V_().v(VX, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
-    qy[j] = V_().v(VY, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
-    qz[j] = V_().v(VZ, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qx[j] = val(VX, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
+    qy[j] = val(VY, (uint32_t)(t.y0 - 3 + j) * ys + t.col);
+    qz[j] = val(VZ, (uint32_t)(t.y0 - 4 + j) * ys + t.col);
   }
   // F_MED3: the previous plane's terms carried in registers -- Sx(mu) of the
   // column, mu of the column and of its z - 1 neighbour -- which are the
@@ -1185,7 +1133,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         mxz = (T(0.5) * (sx_c + sx_zm)) * a.tdt;
         mxy = (T(0.5) * (sx_c + sx_prev)) * a.tdt;
         myz = (T(0.5) * (sy_c + sy_zm)) * a.tdt;
-      } else if (MODE != MODE_BORN_ADJ) {
+      } else {
         l2m = ld_nt(fam(a.m, L2M, np), i); lam = ld_nt(fam(a.m, LAM, np), i);
         mxz = ld_nt(fam(a.m, MXZ, np), i); mxy = ld_nt(fam(a.m, MXY, np), i); myz = ld_nt(fam(a.m, MYZ, np), i);
       }
@@ -1208,7 +1156,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         }
       }
       T u[6];
-      if (MODE == MODE_BORN_ADJ || MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q) {
+      if (MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q) {
         u[0] = w * o6[0] - exx;
         u[1] = w * o6[1] - eyy;
         u[2] = w * o6[2] - ezz;
@@ -1218,7 +1166,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
         u[1] = w * o6[1] + sg * (l2m * eyy) + sg * (lam * (exx + ezz));
         u[2] = w * o6[2] + sg * (l2m * ezz) + sg * (lam * (exx + eyy));
       }
-      if (MODE == MODE_BORN_ADJ || MODE == MODE_BORN_ADJ_PM) {
+      if (MODE == MODE_BORN_ADJ_PM) {
         u[3] = w * o6[3] - gxz;
         u[4] = w * o6[4] - gxy;
         u[5] = w * o6[5] - gyz;
