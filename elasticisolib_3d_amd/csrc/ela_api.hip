@@ -201,17 +201,22 @@ int check_dev_ptr(const void* p, const char* what) {
   return ELA_OK;
 }
 
-// Whether p is memory of GPU `dev` itself. Output sums are added by a kernel
-// in place there; memory that the GPU may reach otherwise or not at all (another
-// GPU's, pinned host, managed) is copied in and out by the runtime.
-bool own_memory(const void* p, int dev) {
+// Whether [p, p + bytes) is one allocation's memory of GPU `dev` itself. Output
+// sums are added by a kernel in place there; memory that the GPU may reach
+// otherwise or not at all (another GPU's, pinned host, managed, past the end of
+// the array handed over) is copied in and out by the runtime, which checks it.
+bool own_memory(const void* p, size_t bytes, int dev) {
   hipPointerAttribute_t attr;
   std::memset(&attr, 0, sizeof(attr));
-  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  return attr.type == hipMemoryTypeDevice && attr.device == dev;
+  const size_t at = static_cast<const char*>(p) - static_cast<const char*>(base);
+  return attr.type == hipMemoryTypeDevice && attr.device == dev && at <= size && bytes <= size - at;
 }
 
 }  // namespace
@@ -794,12 +799,14 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   a.ytab = h->win_y0.empty() ? nullptr : (const int*)h->ytab.p;
   a.bad = flag;
   if (total) launch(h, ela::k_convert_pos, dim3((unsigned)((total + 255) / 256)), dim3(256), a);
-  std::vector<int> host(24 + nwin);
-  HIPCHK(hipMemcpyAsync(host.data(), flag, host.size() * sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  int few[64];
+  std::vector<int> many(24 + nwin > 64 ? 24 + nwin : 0);
+  int* host = many.empty() ? few : many.data();
+  HIPCHK(hipMemcpyAsync(host, flag, (24 + nwin) * sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  ds.fuse = ds.box && fuse_injection(h, ds, host.data() + 8);
-  dr.fuse = dr.box && fuse_injection(h, dr, host.data() + 16);
-  if (transposed) CHK(set_transposed_form(h, host.data() + 24, flag + 24));
+  ds.fuse = ds.box && fuse_injection(h, ds, host + 8);
+  dr.fuse = dr.box && fuse_injection(h, dr, host + 16);
+  if (transposed) CHK(set_transposed_form(h, host + 24, flag + 24));
   if (host[0]) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
   return ELA_OK;
 }
@@ -1617,10 +1624,10 @@ int born_run(ela_handle* h, const ela_points* sp_in, const ela_traces* st_in, co
 
   // forward: the perturbations in the library layout (read at interior cells
   // only); adjoint: the image to add to, the caller's or its device copy
-  const bool in_place = adjoint && mem == ELA_MEM_DEVICE && own_memory(dmod_out, h->cfg.device);
+  const size_t img_bytes = (size_t)8 * h->n_model * sizeof(T);
+  const bool in_place = adjoint && mem == ELA_MEM_DEVICE && own_memory(dmod_out, img_bytes, h->cfg.device);
   if (!in_place) CHK(h->dmod.alloc(8 * np * sizeof(T)));
   T* dm = (T*)h->dmod.p;
-  const size_t img_bytes = (size_t)8 * h->n_model * sizeof(T);
   if (!adjoint) {
     CHK(copy_in_3d(h, dm, dmod_in, 8, mem));
   } else if (in_place) {
@@ -2128,7 +2135,7 @@ int grad_backward(ela_handle* h, const ela_points* sp_in, const ela_traces* st_i
   CHK(fill<T>(h, g32, 8 * np));
   // a call on this GPU's memory adds its sums to the caller's arrays at the
   // end; other arrays are the start of the sums
-  const bool in_place = mem == ELA_MEM_DEVICE && own_memory(grad8, h->cfg.device);
+  const bool in_place = mem == ELA_MEM_DEVICE && own_memory(grad8, (size_t)8 * h->n_model * sizeof(double), h->cfg.device);
   bool summed = !in_place;   // g64 holds something
   if (!in_place) {
     CHK(fill<double>(h, g64, 8 * np));
