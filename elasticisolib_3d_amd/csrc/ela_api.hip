@@ -702,10 +702,11 @@ size_t point_scratch_bytes(int64_t total) { return (size_t)round_up(total * 4, 2
 template <typename T>
 ela::CkArgs<T> interior_args(const ela_handle* h);
 
-// Whether the transposed steps may divide by M (adj_wave): every buoyancy and
-// shear modulus that is stepped is positive, the shear moduli at least 2^-20 of
-// lamb2MuDtw (in a fluid M n says nothing of a shear stress n, and far below
-// that it may underflow). Looked at in every transposed call (one read of the
+// Whether the transposed steps may divide by M (adj_wave): the shear moduli
+// that are stepped are at least 2^-20 of lamb2MuDtw (in a fluid M n says nothing
+// of a shear stress n), they and the buoyancies at least 2^-64. Below that M n
+// underflows in FP32 where n does not (n of 2^-62 has all its bits at 2^-64),
+// and under 2^-128 1 / M overflows: a body made rigid by its density. Looked at in every transposed call (one read of the
 // medium, 0.2 ms of the 70 to 90 ms of 40 steps of 232x328x324), not when the
 // medium is set: it depends on the windows too, and a medium may be set by a
 // replayed graph. fluid: a cleared entry per window (one without windows).

@@ -1762,10 +1762,11 @@ __global__ void __launch_bounds__(256) k_check_solid(CkArgs<T> a, const int* yta
       w = ytab[4 * (iy + FAT) + 3];
     }
     const int64_t i = ck_offset(a, q);
-    const T least = a.f[L2M][i] * T(0x1p-20);
-    bool ok = least > T(0);
+    constexpr T tiny = T(0x1p-64);
+    const T least = max(a.f[L2M][i] * T(0x1p-20), tiny);
+    bool ok = a.f[L2M][i] > T(0);
     for (int k = MXZ; k <= MYZ; ++k) ok = ok && a.f[k][i] >= least;
-    for (int k = BX_; k <= BZ_; ++k) ok = ok && a.f[k][i] > T(0);
+    for (int k = BX_; k <= BZ_; ++k) ok = ok && a.f[k][i] >= tiny;
     if (!ok && w != told) {
       told = w;
       const int first = __ffsll((unsigned long long)__ballot(1)) - 1;

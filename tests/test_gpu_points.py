@@ -171,6 +171,31 @@ def test_transposed_wavefield_kinds(precision, ratio):
         assert e[0] < 2 * TOL[precision] and e[1] < 2 * TOL[precision] and e[2] < 2 * TOL[precision]
 
 
+# densities of a rigid body: 1 / M overflows in FP32, M n underflows, and both still fit
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("rho", [1e36, 1e32, 1e12])
+def test_transposed_steps_in_a_rigid_body(precision, rho):
+    """A block whose buoyancies are next to nothing: n is not recovered from
+    M n there. Born adjoint and gradient against the oracle, every array by
+    itself (the buoyancies' hold the block's cells)."""
+    g = grid(4, 4)
+    P = random_problem(g, seed=27, nsrc=2, nrec=9)
+    r = P["rho"].copy()
+    r[6:12, 6:11, 30:50] = rho
+    med = O.lib_scale_medium(r, P["lam"], P["mu"], g.dtw)
+    img = O.lib_born_adjoint(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+    g8_ref, gs_ref = O.lib_gradient(g, med, P["src"], P["spos"], P["rec"], P["rpos"])
+    prop = make_prop(g, precision)
+    prop.set_gradient_checkpoints(4, 0, "native")
+    prop.set_elastic(np.stack([r, P["lam"], P["mu"]]), g.dtw)
+    out = prop.born_adjoint(P["spos"], P["src"], P["rec"], P["rpos"])
+    prop.gradient_forward(P["spos"], P["src"], P["rpos"])
+    g8, gs = prop.gradient_backward(P["spos"], P["src"], P["rpos"], P["rec"])
+    e = [rel(a, b) for a, b in zip([*out, *g8], [*img, *g8_ref])] + [rel(gs, gs_ref)]
+    print(f"{precision} rho {rho:g}: worst array {max(e):.2e}", flush=True)
+    assert np.all(np.isfinite(out)) and np.all(np.isfinite(g8)) and max(e) < 2 * TOL[precision]
+
+
 @pytest.mark.parametrize("precision", ["f64", "f32"])
 def test_velocity_tile_direction(precision):
     """Velocity tiles run backwards where the layers of y chunks are small
