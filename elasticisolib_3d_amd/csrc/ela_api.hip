@@ -239,9 +239,8 @@ struct ela_handle {
   double tdt = 0.0;         // 2 dtw of ela_set_elastic
   // form of the transposed steps of this call (check_solid, adj_wave)
   bool solid = false;       // MODE_BORN_ADJ_Q everywhere
-  bool mixed = false;       // MODE_BORN_ADJ_Q in the solid windows of a stack, MODE_BORN_ADJ_PM in the others
-  std::vector<int> win_fluid;           // per window (one entry without windows): not solid
-  const int* win_fluid_dev = nullptr;   // the same on the device
+  bool mixed = false;       // MODE_BORN_ADJ_MIXED: a stack of solid and other windows
+  const int* win_fluid = nullptr;   // device: per window, not solid (valid during the call)
   DevBuf taper;             // min_pad values
   DevBuf scratch_tm;        // time-major trace buffer
   void* scratch_dev = nullptr;  // device address of ela_scratch on cfg.device (resolved in ela_create)
@@ -286,9 +285,8 @@ struct ela_handle {
   // windows stacked along y (several shots in one grid)
   std::vector<int64_t> win_y0, win_ny, win_nx;
   DevBuf ytab;              // per plane {window y0, ny, nx, window} (int32)
-  DevBuf chunks;            // per y chunk {y0, y1, window y0, ny, nx, 0, 0, 0} (int32)
+  DevBuf chunks;            // per y chunk {y0, y1, window y0, ny, nx, window, 0, 0} (int32)
   int chunks_yc = 0;        // y chunk the table was built for
-  std::vector<int> chunks_fluid;   // window kinds its two further parts were built for (ensure_chunks)
   int nchunks = 0;
   // graph replays of the time loops (ela_set_graph): the coarse step of the
   // nonlinear propagations, the fine-step pairs and checkpoint segments of the
@@ -449,29 +447,22 @@ struct Tiles {
 
 // Chunk table of the stacked windows for the current y chunk (rebuilt when
 // the y chunk changes; a synchronous upload, done before any launch of the
-// propagation that uses it). For a stack of solid and fluid windows two more
-// tables follow, of as many rows: the first with the solid windows' rows, the
-// second with the others', the remaining rows being windows of no width, whose
-// blocks return at once.
+// propagation that uses it).
 int ensure_chunks(ela_handle* h) {
-  if (h->win_y0.empty() || (h->chunks_yc == h->ychunk && (!h->mixed || h->chunks_fluid == h->win_fluid))) return ELA_OK;
+  if (h->win_y0.empty() || h->chunks_yc == h->ychunk) return ELA_OK;
   std::vector<int> tab;
-  for (int part = 0; part < (h->mixed ? 3 : 1); ++part) {
-    for (size_t w = 0; w < h->win_y0.size(); ++w) {
-      const int64_t a = h->win_y0[w] + ela::FAT, b = h->win_y0[w] + h->win_ny[w] - ela::FAT;
-      const bool in = part == 0 || h->win_fluid[w] == part - 1;
-      for (int64_t y = a; y < b; y += h->ychunk) {
-        const int row[8] = {(int)y, (int)std::min<int64_t>(y + h->ychunk, b), (int)h->win_y0[w], (int)h->win_ny[w],
-                            in ? (int)h->win_nx[w] : 0, 0, 0, 0};
-        tab.insert(tab.end(), row, row + 8);
-      }
+  for (size_t w = 0; w < h->win_y0.size(); ++w) {
+    const int64_t a = h->win_y0[w] + ela::FAT, b = h->win_y0[w] + h->win_ny[w] - ela::FAT;
+    for (int64_t y = a; y < b; y += h->ychunk) {
+      const int row[8] = {(int)y, (int)std::min<int64_t>(y + h->ychunk, b), (int)h->win_y0[w], (int)h->win_ny[w],
+                          (int)h->win_nx[w], (int)w, 0, 0};
+      tab.insert(tab.end(), row, row + 8);
     }
-    if (part == 0) h->nchunks = (int)(tab.size() / 8);
   }
   CHK(h->chunks.alloc(tab.size() * sizeof(int)));
   HIPCHK(hipMemcpy(h->chunks.p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
+  h->nchunks = (int)(tab.size() / 8);
   h->chunks_yc = h->ychunk;
-  h->chunks_fluid = h->mixed ? h->win_fluid : std::vector<int>();
   return ELA_OK;
 }
 
@@ -598,13 +589,17 @@ template <typename T, int MODE, int FV, int FS>
 int launch_step(ela_handle* h, const ela::StepArgs<T>& a, int which, const ela::PointArgs<T>& inj,
                 const ela::PointArgs<T>& rec) {
   // the premultiplied transposed steps (Born adjoint, gradient) may take a tile of their own
-  const bool transposed = MODE == ela::MODE_BORN_ADJ_PM || MODE == ela::MODE_BORN_ADJ_Q;
+  const bool transposed = ela::premultiplied(MODE);
   const int bx = transposed && h->by_x_t ? h->by_x_t : h->by_x;
   // 16 rows (1024 threads, at most 128 registers) only where the step fits:
   // FP64 and the steps with per-cell extra operands spill there (Born adjoint
   // of 232x328x324 69-97 ms with 16 rows, 60 with 4) and run 4 rows instead
-  constexpr bool wide = sizeof(T) == 4 && ((FV | FS) & (ela::F_SS | ela::F_ACC | ela::F_GRAD)) == 0;
-  if (bx == 8) return launch_step_s<T, 8, MODE, FV, FS>(h, a, which, inj, rec);
+  // mixed stacks, which are rare, run 256-thread tiles alone (each kernel holds two forms)
+  constexpr bool mixed = MODE == ela::MODE_BORN_ADJ_MIXED;
+  constexpr bool wide = sizeof(T) == 4 && !mixed && ((FV | FS) & (ela::F_SS | ela::F_ACC | ela::F_GRAD)) == 0;
+  if constexpr (!mixed) {
+    if (bx == 8) return launch_step_s<T, 8, MODE, FV, FS>(h, a, which, inj, rec);
+  }
   if constexpr (wide) {
     if (bx == 16) return launch_step_s<T, 16, MODE, FV, FS>(h, a, which, inj, rec);
   }
@@ -728,13 +723,11 @@ int64_t window_count(const ela_handle* h) { return std::max<int64_t>(1, (int64_t
 // The form of the transposed steps from check_solid's answers (host copy and
 // device array). Every window takes the form it takes alone, so its results
 // are the same to the bit in every stack.
-int set_transposed_form(ela_handle* h, const int* fluid, const int* fluid_dev) {
-  h->win_fluid.assign(fluid, fluid + window_count(h));
-  h->win_fluid_dev = fluid_dev;
-  const int64_t n = std::count(h->win_fluid.begin(), h->win_fluid.end(), 0);
+void set_transposed_form(ela_handle* h, const int* fluid, const int* fluid_dev) {
+  const int64_t n = std::count(fluid, fluid + window_count(h), 0);
   h->solid = n == window_count(h);
   h->mixed = n > 0 && !h->solid;
-  return ensure_chunks(h);
+  h->win_fluid = fluid_dev;
 }
 
 // Copies (host) or reads (device) the caller's int64 positions, converts them
@@ -807,7 +800,7 @@ int convert_points(ela_handle* h, const ela_points* sp, const ela_points* rp, in
   HIPCHK(hipStreamSynchronize(h->stream));
   ds.fuse = ds.box && fuse_injection(h, ds, host + 8);
   dr.fuse = dr.box && fuse_injection(h, dr, host + 16);
-  if (transposed) CHK(set_transposed_form(h, host + 24, flag + 24));
+  if (transposed) set_transposed_form(h, host + 24, flag + 24);
   if (host[0]) return fail(ELA_ERR_ARG, "a source or receiver position lies outside the FD interior");
   return ELA_OK;
 }
@@ -882,7 +875,7 @@ int step_with_points(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& 
   if (ip.fuse || inj.off[9] == 0) return ELA_OK;
   const unsigned nb = (unsigned)((inj.off[9] + 255) / 256);
   launch(h, ela::k_inject<T, ((FV | FS) & ela::F_ACC) != 0, ((FV | FS) & ela::F_GRAD) != 0,
-                          MODE == ela::MODE_BORN_ADJ_PM || MODE == ela::MODE_BORN_ADJ_Q>, dim3(nb), dim3(256), inj);
+                          ela::premultiplied(MODE)>, dim3(nb), dim3(256), inj);
   return ELA_OK;
 }
 
@@ -1049,7 +1042,9 @@ Wave<T> wave_ptrs(DevBuf& b, int64_t stride, bool premultiplied = false) {
 // of their 3 x 3 block enlarges q's roundings by (3 lambda + 2 mu) / 2 mu, up to
 // 1.8 times the FP32 error at Vp / Vs = 4; as it is the error is the same.
 // A stack of solid and fluid windows is held in the general form's 36 arrays, of
-// which the steps of its solid windows use q and the normal stresses of n.
+// which the steps of its solid windows use q and the normal stresses of n
+// (MODE_BORN_ADJ_MIXED; an injection adds to n and q alike, and the n of a solid
+// window's velocities and shear stresses is read by nobody).
 template <typename T>
 Wave<T> adj_wave(ela_handle* h) {
   if (!h->solid) return wave_ptrs<T>(h->wave2, h->stride, true);
@@ -1076,6 +1071,7 @@ ela::StepArgs<T> adj_args(ela_handle* h, Wave<T>& w) {
   } else {
     a.q = w.q1[0];
     a.qn = w.q0[0];
+    if (h->mixed) a.fluid = h->win_fluid;
   }
   return a;
 }
@@ -1087,29 +1083,16 @@ ela::PointArgs<T> adj_points(ela_handle* h, const DevPoints& pts, T* const p[9],
   ela::PointArgs<T> a = make_points<T>(h, pts, p, tr, true, n);
   for (int k = 0; k < 9; ++k) a.q[k] = q[k];
   for (int k = 0; k < 8; ++k) a.m[k] = arr<T>(h->med, h->stride, k);
-  if (h->mixed) a.fluid = h->win_fluid_dev;
+  if (h->mixed) a.fluid = h->win_fluid;
   return a;
 }
 
-// One transposed step. A mixed stack takes two launches, each over its own
-// windows (ensure_chunks): the solid ones first, then the others with what
-// concerns all of them, the recording and an injection by itself (which adds to
-// n and q alike; the n of a solid window's velocities and shear stresses is
-// read by nobody).
 template <typename T, int FV, int FS>
 int adj_launch(ela_handle* h, const ela::StepArgs<T>& a, const DevPoints& rp, const ela::PointArgs<T>& inj,
                const ela::PointArgs<T>& rec = ela::PointArgs<T>{}) {
   if (h->solid) return step_with_points<T, ela::MODE_BORN_ADJ_Q, FV, FS>(h, a, rp, inj, rec);
-  if (!h->mixed) return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, a, rp, inj, rec);
-  ela::StepArgs<T> q = a, pm = a;
-  q.o = a.qn;
-  q.c = a.q;
-  q.q = nullptr;
-  q.qn = a.o + ela::SXX * a.np;
-  q.chunks = a.chunks + 8 * (int64_t)h->nchunks;
-  pm.chunks = q.chunks + 8 * (int64_t)h->nchunks;
-  CHK((launch_step_m<T, ela::MODE_BORN_ADJ_Q, FV, FS>(h, q, 3, rp.fuse ? inj : ela::PointArgs<T>{})));
-  return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, pm, rp, inj, rec);
+  if (h->mixed) return step_with_points<T, ela::MODE_BORN_ADJ_MIXED, FV, FS>(h, a, rp, inj, rec);
+  return step_with_points<T, ela::MODE_BORN_ADJ_PM, FV, FS>(h, a, rp, inj, rec);
 }
 
 // The 9 components of a time-major trace buffer share one base pointer
@@ -2288,7 +2271,7 @@ int time_gradient_kernels(ela_handle* h, int reps, double* ms3) {
   CHK(check_solid(h, flag));
   HIPCHK(hipMemcpyAsync(fluid.data(), flag, nwin * sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  CHK(set_transposed_form(h, fluid.data(), flag));
+  set_transposed_form(h, fluid.data(), flag);
   CHK(h->wave2.alloc((size_t)adj_arrays(h) * np * sizeof(T)));
   CHK(h->drv.alloc(drv_step_bytes(h, dfmt)));
   CHK(h->g32.alloc((size_t)8 * np * sizeof(T)));
@@ -2684,7 +2667,6 @@ int ela_set_windows(ela_handle* h, int n, const int64_t* y0, const int64_t* ny, 
     h->win_y0.clear(); h->win_ny.clear(); h->win_nx.clear();
     h->chunks_yc = 0;
     h->solid = h->mixed = false;   // asked again by the next transposed call
-    h->win_fluid.clear();
     h->grad_ready = false;
     if (n == 0) return ELA_OK;
     const int64_t NY = h->cfg.ny;

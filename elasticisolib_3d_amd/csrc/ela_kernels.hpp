@@ -55,8 +55,10 @@ enum { BX_ = 0, BY_, BZ_, L2M, LAM, MXZ, MXY, MYZ };
 enum { MODE_FWD = 0,       // n = w(w o + M D c)        stepFwdGpu_3D
        MODE_ADJ = 1,       // n = w(w o - M D c)        stepAdjGpu_3D
        MODE_BORN_ADJ_PM = 3, // n = w(w o - D q) with q = M c read and M n written (qn) beside n
-       MODE_BORN_ADJ_Q = 4   // the same on q = M n alone but for the normal stresses: q' = w(w q - M D c) (adj_wave)
+       MODE_BORN_ADJ_Q = 4,  // the same on q = M n alone but for the normal stresses: q' = w(w q - M D c) (adj_wave)
+       MODE_BORN_ADJ_MIXED = 5 // a stack of windows: _Q in the solid ones, _PM in the others (k_step)
 };
+constexpr bool premultiplied(int mode) { return mode >= MODE_BORN_ADJ_PM; }   // injections go into M n too
 
 // Optional work fused into a stepper launch (bit flags).
 //
@@ -130,7 +132,8 @@ struct StepArgs {
   int remap;            // tile order (see tile_coord)
   int rev;              // velocity blocks run backwards through the tiles (see k_step)
   int xgroup;           // x columns per group of the y-major order
-  const int* chunks;    // stacked windows: per y chunk {y0, y1, window y0, window ny, window nx}, or null
+  const int* chunks;    // stacked windows: per y chunk {y0, y1, window y0, window ny, window nx, window}, or null
+  const int* fluid;     // MODE_BORN_ADJ_MIXED: per window, 1 general (_PM) or 0 solid (_Q)
 };
 
 template <typename P>
@@ -333,6 +336,7 @@ __device__ __forceinline__ float load_dq16(const int16_t* q, const float* sc, ui
 struct TileCoord {
   int tz, ty, iz, izo, ix, y0, y1, z0, x0;   // iz internal, izo reference z
   int wy0, wny, wnx;       // the tile's window: first plane, planes, x extent (whole grid without windows)
+  int win;                 // its number
   bool empty;              // no interior cell in the tile (its window is narrower than the tile's x)
   bool active;             // own column inside the interior
   bool xin;                // the tile row (wave-uniform) is an interior x row
@@ -383,11 +387,11 @@ __device__ __forceinline__ TileCoord tile_coord(int bid, int nbz, int nbx, int n
   t.ix = t.x0 + t.ty;
   if (chunks) {
     const int* c = chunks + 8 * by;
-    t.y0 = c[0]; t.y1 = c[1]; t.wy0 = c[2]; t.wny = c[3]; t.wnx = c[4];
+    t.y0 = c[0]; t.y1 = c[1]; t.wy0 = c[2]; t.wny = c[3]; t.wnx = c[4]; t.win = c[5];
   } else {
     t.y0 = FAT + by * ychunk;
     t.y1 = min(t.y0 + ychunk, ny - FAT);
-    t.wy0 = 0; t.wny = ny; t.wnx = nx;
+    t.wy0 = 0; t.wny = ny; t.wnx = nx; t.win = 0;
   }
   nx = t.wnx;
   t.empty = t.x0 >= nx - FAT;
@@ -718,7 +722,6 @@ __device__ __forceinline__ void normal_moduli(T tdt, double tdt64, T lam, T mu, 
 template <typename T, int S, int MODE, int F>
 __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
                                                VelLds<T, S, (F & F_MED3) != 0>& L) {
-  constexpr bool PREMULT = MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q;  // injections go into M n too
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
@@ -919,7 +922,7 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
     __syncthreads();
     b ^= 1;
   }
-  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, PREMULT>(0, VX, SXX);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, premultiplied(MODE)>(0, VX, SXX);
 }
 
 // ---------------------------------------------------------------------------
@@ -943,7 +946,6 @@ struct StressStage {
 template <typename T, int S, int MODE, int F>
 __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointArgs<T>& inj, int bid,
                                              StressLds<T, S, (F & F_MED3) != 0>& L) {
-  constexpr bool PREMULT = MODE == MODE_BORN_ADJ_PM || MODE == MODE_BORN_ADJ_Q;  // injections go into M n too
   constexpr int BX = tile_x(S);
   constexpr bool SS = (F & F_SS) != 0, ACC = (F & F_ACC) != 0, MED3 = (F & F_MED3) != 0;
   constexpr bool Q16 = (F & F_Q16) != 0, QS = Q16 && (F & F_STORE) != 0;
@@ -1244,7 +1246,7 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
     __syncthreads();
     b ^= 1;
   }
-  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, PREMULT>(1, SXX, SYZ + 1);
+  if (inj_hit) inject_tile<T, S, ACC, (F & F_GRAD) != 0, premultiplied(MODE)>(1, SXX, SYZ + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1284,9 +1286,29 @@ __global__ void __launch_bounds__(tile_threads(S), (step_waves<T, FV, FS>())) k_
   __shared__ Lds L;
   static_assert(sizeof(StepArgs<T>) % alignof(PointArgs<T>) == 0, "inject_tile finds inj behind a");
   const int nb = a.nbz * a.nbx * a.nby, bid = (int)blockIdx.x + a.first;  // block-uniform
-  if (bid < nb) velocity_block<T, S, MODE, FV>(a, inj, a.rev ? nb - 1 - bid : bid, L.v);
-  else if (bid < 2 * nb) stress_block<T, S, MODE, FS>(a, inj, bid - nb, L.s);
-  else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
+  if (bid < 2 * nb) {
+    const bool vel = bid < nb;
+    const int tile = vel ? (a.rev ? nb - 1 - bid : bid) : bid - nb;
+    if constexpr (MODE == MODE_BORN_ADJ_MIXED) {
+      const int w = tile_coord<S>(tile, a.nbz, a.nbx, a.nby, a.ychunk, a.nz, a.nzi, a.zoff, a.nx, a.ny, a.remap,
+                                  a.xgroup, a.chunks).win;
+      if (a.fluid[w]) {
+        if (vel) velocity_block<T, S, MODE_BORN_ADJ_PM, FV>(a, inj, tile, L.v);
+        else stress_block<T, S, MODE_BORN_ADJ_PM, FS>(a, inj, tile, L.s);
+      } else {
+        StepArgs<T> s = a;   // q in the places of n, the normal stresses of n as adj_args hands them over
+        s.o = a.qn;
+        s.c = a.q;
+        s.qn = fam(a.o, SXX, a.np);
+        if (vel) velocity_block<T, S, MODE_BORN_ADJ_Q, FV>(s, inj, tile, L.v);
+        else stress_block<T, S, MODE_BORN_ADJ_Q, FS>(s, inj, tile, L.s);
+      }
+    } else if (vel) {
+      velocity_block<T, S, MODE, FV>(a, inj, tile, L.v);
+    } else {
+      stress_block<T, S, MODE, FS>(a, inj, tile, L.s);
+    }
+  } else record_point(rec, (int64_t)(bid - 2 * nb) * tile_threads(S) + threadIdx.y * WAVE + threadIdx.x);
 }
 
 // The injection by itself: lists too long or too spread for a step's blocks.

@@ -160,3 +160,42 @@ def test_transposed_steps_of_a_stack_equal_each_window_alone(medium, graph, flui
             assert rel(g1, ref) < TOL["f32"] and rel(s1, sref) < TOL["f32"]
     out = ~interior()
     assert not np.any(g8[:, out]) and not np.any(img[:, out])
+
+
+# z interiors of 32-cell and of 64-cell tiles, both derivative formats, both precisions
+@pytest.mark.parametrize("precision,nz,derivatives", [("f64", 27, "native"), ("f32", 27, "s16"), ("f32", 58, "native"),
+                                                      ("f32", 58, "s16")])
+@pytest.mark.parametrize("medium", ["scaled", "elastic"])
+def test_mixed_stack_in_every_kernel(monkeypatch, medium, precision, nz, derivatives):
+    """A stack with a fluid in one window, in the kernels the test above does
+    not reach and for tile settings of 4, 8 and 16 rows: each window's own
+    gradient, source gradient and image to the bit."""
+    import sys
+    monkeypatch.setattr(sys.modules[__name__], "NZ", nz)
+    probs = window_problems(5, (1,))
+    spos, rpos = stack_points(probs, "spos"), stack_points(probs, "rpos")
+    src, rec = stack_traces(probs, "src"), stack_traces(probs, "rec")
+
+    def run(prop, spos, src, rpos, rec):
+        prop.set_gradient_derivatives(derivatives)
+        prop.gradient_forward(spos, src, rpos)
+        return prop.gradient_backward(spos, src, rpos, rec) + (prop.born_adjoint(spos, src, rec, rpos),)
+
+    own = []
+    for g, P in probs:
+        alone = make_prop(g, precision)
+        alone.set_medium(P["med"]) if medium == "scaled" else \
+            alone.set_elastic(np.stack([P["rho"], P["lam"], P["mu"]]), g.dtw)
+        own.append(run(alone, P["spos"], P["src"], P["rpos"], P["rec"]))
+    prop = make_prop(grid(NX, NY), precision)
+    set_windows(prop)
+    prop.set_medium(stack(probs, "med", 0.0)) if medium == "scaled" else \
+        prop.set_elastic(stack(probs, "elastic", 1.0), probs[0][0].dtw)
+    for tile in (None, (4, 3), (8, 5), (16, 8)):
+        if tile:
+            prop.set_tiling(*tile)
+        g8, gs, img = run(prop, spos, src, rpos, rec)
+        for k, (g1, s1, i1) in enumerate(own):
+            inner = np.s_[:, FAT:-FAT, FAT:-FAT, FAT:-FAT]
+            assert all(np.array_equal(a[2 * k:2 * (k + 1)], b) for a, b in zip(gs, s1))
+            assert np.array_equal(g8[box(k)][inner], g1[inner]) and np.array_equal(img[box(k)][inner], i1[inner])
