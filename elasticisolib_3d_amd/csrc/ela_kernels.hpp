@@ -5,9 +5,10 @@
 //   staggered derivatives, cosine sponge. The reference runs, per fine step,
 //   one stepper launch (kernelsElaGpu_3D.cu:110-460), 7 injection launches, a
 //   damping launch over both time levels (:1182-1226) and 7 recording launches.
-//   Here one fine step is one stencil launch (velocity and stress blocks, which
-//   read only level n and so are independent) plus one injection and one
-//   recording launch, with the sponge folded into the stencil:
+//   Here one fine step is one launch (velocity and stress blocks, which read
+//   only level n and so are independent, and blocks that record level n; short
+//   lists of sources are injected by the stencil's blocks, longer ones by a
+//   launch behind it), with the sponge folded into the stencil:
 //       n = w * (w * o + M D(c) [+ secondary source])
 //   where every stored level has been damped exactly once. This equals the
 //   reference's "step, inject, damp p0 and p1, swap" sequence, whose p0 after
@@ -19,9 +20,9 @@
 //   - fields needing x or z derivatives are staged per plane in LDS with a
 //     4-cell halo; y derivatives come from an 8-deep register queue per
 //     thread, so each plane of each field is read from HBM once per tile;
-//   - blocks are dealt round-robin to the 8 XCDs by the hardware; an optional
-//     remap gives each XCD a contiguous range of tiles instead (measured
-//     slower on the 328 x 472 x 468 grid, so off by default).
+//   - blocks are dealt round-robin to the 8 XCDs by the hardware, which sweeps
+//     the grid; the default order hands out groups of whole z columns that way,
+//     so that z and x neighbours share an L2 (orders: tile_coord).
 // No MFMA: the stencil is not a dense contraction; the kernels are HBM-bound.
 #pragma once
 
@@ -284,8 +285,9 @@ __device__ __forceinline__ void rows_to_lds(const float* base, uint32_t i, P& pl
 // Largest magnitude over each 32-lane half of the wave (one DQ_BLOCK), in
 // every lane: DPP lane moves inside each 16-lane row (swap neighbours, swap
 // pairs, mirror within 8, mirror within 16) and one swizzle that exchanges
-// the two rows of a half (lane ^ 16). All 64 lanes must be active. The
-// magnitudes are compared as unsigned integers (the bit patterns of
+// the two rows of a half (lane ^ 16). Each half must be active or inactive as a
+// whole (a narrow tile's second x row may lie past the interior) and no move may
+// cross the halves. The magnitudes are compared as unsigned integers (the bit patterns of
 // non-negative floats order as their values), which needs no NaN quieting.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_umax(uint32_t u) {
@@ -302,8 +304,9 @@ __device__ __forceinline__ float half_wave_absmax(float x) {
   return __uint_as_float(u);
 }
 
-// F_Q16 store of one derivative combination at element i: every lane of the
-// wave calls it; lanes outside the interior pass x = 0. The last z tile of a
+// F_Q16 store of one derivative combination at element i: every lane of an
+// interior x row (half a wave of a narrow tile) calls it; lanes past the row's
+// interior cells pass x = 0. The last z tile of a
 // row may reach past the row into the next row's leading non-interior line
 // ([0, zoff + FAT) = [0, 32)), which no stepper reads and no other tile
 // writes. The hardware reciprocal (1 ulp) serves for 1 / m: |x| 32767 rcp(m)
@@ -339,7 +342,7 @@ struct TileCoord {
   int win;                 // its number
   bool empty;              // no interior cell in the tile (its window is narrower than the tile's x)
   bool active;             // own column inside the interior
-  bool xin;                // the tile row (wave-uniform) is an interior x row
+  bool xin;                // the tile row (a wave, half a wave of a narrow tile) is an interior x row
   bool xh, zh;             // x-halo loader (ty < 4), z-halo loader (tz < 8)
   int colh;                // LDS column of the z-halo value
   uint32_t col, cxl, cxh, czh;  // own column, x-halo rows, z-halo column, each clamped to the grid (window)
@@ -827,8 +830,8 @@ __device__ __forceinline__ void velocity_block(const StepArgs<T>& a, const Point
     np = opaque(a.np);
     VelStage<T> nx_;
     if (more) fetch(nx_, iy + 1, b ^ 1);  // buffer b ^ 1 is free: every wave passed the last barrier
-    // F_STORE with F_Q16: the whole wave of an interior row takes the branch
-    // (the block maxima are wave reductions) and only the interior lanes store
+    // F_STORE with F_Q16: all lanes of an interior row take the branch (the
+    // block maxima are reductions over half waves) and the interior ones store
     if (QS ? t.xin : t.active) {
       const uint32_t i = (uint32_t)iy * ys + (QS ? t.colu : t.col);
       const T* cx = a.cx; const T* cy = a.cy; const T* cz = a.cz;
@@ -1266,6 +1269,12 @@ __device__ __forceinline__ void stress_block(const StepArgs<T>& a, const PointAr
 // 152x152x148, which the cache does not limit. It costs the planes that a block
 // shares with the y chunk after it, which then were read two layers of chunks
 // ago instead of just now: launch_step_s reverses where four layers fit.
+//
+// MODE_BORN_ADJ_MIXED holds two forms of a block and takes that of the window
+// its chunk belongs to (transposed steps of two windows 328x290x260, one with a
+// fluid, half of them imaging: 1.76-1.79 ms a step against 1.84-1.88 in the
+// general form alone; a launch for each form cost stacks of 60^3 windows 15 to
+// 26 % of a backward pass).
 // ---------------------------------------------------------------------------
 // Waves per SIMD asked of the compiler: the FP32 steps without per-cell extra
 // operands need 115-129 VGPRs and run at 4 (at most 128); the others hold more

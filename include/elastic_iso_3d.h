@@ -383,7 +383,8 @@ int ela_set_graph(ela_handle* h, int on);
  * handle: 4 rows and 2 to 13 planes, by the grid's size). 4 rows become 8 rows
  * of a 32-wide z tile where that is faster (FP64, and z extents that leave
  * fewer cells idle), 16 rows become 4 in the steps whose registers do not
- * allow 16. Any setting gives the same result; it only changes speed. */
+ * allow 16, and 8 and 16 rows in the transposed steps of stacks of solid and
+ * fluid windows. Any setting gives the same result; it only changes speed. */
 int ela_set_tiling(ela_handle* h, int tile_x, int y_chunk);
 int ela_get_tiling(const ela_handle* h, int* tile_x, int* y_chunk);
 /* Block-to-tile order of the stencil launches (speed only): 0 the hardware's
