@@ -91,7 +91,8 @@ typedef struct ela_points {
   int64_t n[7];
 } ela_points;
 
-/* One trace array per component; element type follows the handle precision. */
+/* One trace array per component; element type follows the handle precision.
+ * A component with points and a null array is an argument error. */
 typedef struct ela_traces {
   void* tr[9];
 } ela_traces;

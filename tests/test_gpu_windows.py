@@ -162,6 +162,33 @@ def test_transposed_steps_of_a_stack_equal_each_window_alone(medium, graph, flui
     assert not np.any(g8[:, out]) and not np.any(img[:, out])
 
 
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_born_forward_of_a_stack_equals_each_window_alone(precision):
+    """Linearised data of a stack, after a call over the whole grid left other
+    perturbations in the handle's buffer: each window's own to the bit, and
+    the oracle's; perturbations outside the windows are not read."""
+    probs = window_problems(5)
+    spos, rpos = stack_points(probs, "spos"), stack_points(probs, "rpos")
+    src = stack_traces(probs, "src")
+    full = grid(NX, NY)
+    P = random_problem(full, seed=1)
+    prop = make_prop(full, precision)
+    prop.set_medium(P["med"])
+    prop.born_forward(spos, src, P["dm"], rpos)
+    set_windows(prop)
+    prop.set_medium(stack(probs, "med", 0.0))
+    dm = np.full((8, NY, NX, NZ), np.nan)
+    for k, (_, P) in enumerate(probs):
+        dm[box(k)] = P["dm"]
+    data = prop.born_forward(spos, src, dm, rpos)
+    for k, (g, P) in enumerate(probs):
+        alone = make_prop(g, precision)
+        alone.set_medium(P["med"])
+        own = alone.born_forward(P["spos"], P["src"], P["dm"], P["rpos"])
+        assert all(np.array_equal(a[5 * k:5 * (k + 1)], b) for a, b in zip(data, own))
+        assert rel(own, O.lib_born_forward(g, P["med"], P["src"], P["spos"], P["dm"], P["rpos"])) < TOL[precision]
+
+
 # z interiors of 32-cell and of 64-cell tiles, both derivative formats, both precisions
 @pytest.mark.parametrize("precision,nz,derivatives", [("f64", 27, "native"), ("f32", 27, "s16"), ("f32", 58, "native"),
                                                       ("f32", 58, "s16")])
